@@ -508,19 +508,13 @@ typedef struct {
   uint32_t triangle_tile;            /* triangles per tile in the cull/sort kernels (64..2048) */
   uint32_t scatter_waves;            /* wavefronts per tile in the sort's scatter pass: 1 or 4 */
   uint32_t use_graph;                /* replay the batched chain from a HIP graph */
-  uint32_t store_mode;               /* assembly stores: bit 0 = direct per-lane stores instead of
-                                        LDS-staged rows, bit 1 = non-temporal (streaming) stores,
-                                        bit 2 = stage 32 rows at a time instead of 64, bit 3 =
-                                        software-pipelined gathers, bit 4 = four wavefronts per block,
-                                        bit 5 = one output stream per block (colour vertices and indices,
-                                        or depth vertices; twice the blocks), bit 6 = the assembly's
-                                        blocks in launch order whatever xcd_swizzle says for the other
-                                        passes (0-4, 6, 8, 10, 12, 14, 16, 18, 20, 22, 34, 38, 50, 54,
-                                        and 80, 82, 114 for 16, 18, 50 with bit 6) */
+  uint32_t store_mode;               /* assembly: bit 1 = non-temporal (streaming) stores, bit 6 = its blocks
+                                        in launch order whatever xcd_swizzle says for the other passes; the
+                                        other bits (of 0-4, 6, 8, 10, 12, 14, 16, 18, 20, 22, 34, 38, 50, 54, 80,
+                                        82, 114, the accepted values) change nothing */
   uint32_t assemble_split;           /* assembly blocks per tile: a power of two, tile/split >= 64 */
   uint32_t xcd_swizzle;              /* 1: each XCD takes a contiguous range of a launch's blocks */
-  uint32_t vertex_split;             /* 1: clip positions and colours in two arrays instead of one
-                                        interleaved 32-byte record per vertex */
+  uint32_t vertex_split;             /* 0 or 1; changes nothing (the cull pass always reads its own array) */
   uint32_t cull_block;               /* threads per tile block in the cull pass: 256, 512 or 1024 */
   uint32_t model_stage;              /* 1: the batched form runs the model-level stage (frustum test, render
                                         pairs and their order, per-pair slices) on the device when the

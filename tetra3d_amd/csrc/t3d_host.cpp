@@ -213,6 +213,31 @@ uint64_t carve_size(uint64_t count) {
   return align_up(std::max<uint64_t>(count, 1) * sizeof(T), 256);
 }
 
+// Per-vertex and per-triangle records of a frame: 49 bytes a vertex (65 when the frame has a skinned model) and
+// 22 a triangle.
+uint64_t record_scratch(uint64_t V, uint64_t T, bool skinned) {
+  return carve_size<float4>(2 * V) + carve_size<float4>(V) + carve_size<uint8_t>(V) + carve_size<float4>(skinned ? V : 1) +
+         carve_size<float>(T) + carve_size<uint16_t>(T) + carve_size<uint4>(T);
+}
+void take_records(Carve& sc, FrameArgs& a, uint64_t V, uint64_t T, bool skinned) {
+  a.touch_records = V > kTouchVertices ? 1u : 0u;
+  a.vab = sc.take<float4>(2 * V);
+  a.vq = sc.take<float4>(V);
+  a.vz = sc.take<uint8_t>(V);
+  a.vpos = sc.take<float4>(skinned ? V : 1);
+  a.key = sc.take<float>(T);
+  a.tri_loc = sc.take<uint16_t>(T);
+  a.tri_vo = sc.take<uint4>(T);
+}
+// What t3d_render_noalloc counts against T3D_NOALLOC_SCRATCH_BYTES for them: 52 bytes a vertex and 36 a triangle,
+// whatever the records take, so which frames fit is a rule on their sizes that a change of layout does not move.
+// The static array is a quarter larger than the limit: a frame whose models are all skinned takes up to 65 bytes
+// where 52 are counted.
+uint64_t placed_charge(uint64_t V, uint64_t T) {
+  return carve_size<float4>(2 * V) + carve_size<float4>(V) + carve_size<uint32_t>(T) + 2 * carve_size<uint4>(T) +
+         carve_size<float4>(128) + carve_size<float>(V);
+}
+
 // ---------------------------------------------------------------------------
 // camera (camera.go:638-679, 933-983, 1085-1088)
 // ---------------------------------------------------------------------------
@@ -740,6 +765,7 @@ t3d_status t3d_mesh_upload(t3d_ctx* c, const t3d_mesh_desc* d, uint64_t* out_han
       }
     if (r.triangle_count == 0) lo = hi = 0;
     m->parts.push_back(r);
+    m->max_part = std::max(m->max_part, r.triangle_count);
     m->part_vmin.push_back(lo);
     m->part_vcount.push_back(r.triangle_count ? hi - lo + 1 : 0);
   }
@@ -1111,11 +1137,7 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
   }
   {
     ProfScope ps(c, st, "k_assemble", tr.uv, prof);
-    HIP_TRY(c, launch_assemble(a, tb0, tb1 - tb0, c->tuning.store_mode, c->tuning.assemble_split, st));
-  }
-  if (f->any_normals) {
-    ProfScope ps(c, st, "k_normals", 0, prof);
-    HIP_TRY(c, launch_normals(a, tb0, tb1 - tb0, st));
+    HIP_TRY(c, launch_assemble(a, tb0, tb1 - tb0, c->tuning.store_mode, c->tuning.assemble_split, f->max_triangles, st));
   }
   return T3D_OK;
 }
@@ -1325,7 +1347,8 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   uint64_t nm = 0, nmat = 0, ncand = 0, nlights = 0, pal_floats = 0, skw_floats = 0;
   uint64_t pose_bones = 0, pose_roots = 0, npose = 0;
   uint64_t wV = 0, wT = 0, wvch = 0, wtiles = 0, wsb = 0, wps = 0, whist = 0, wpl = 0;
-  bool any_normals = false;
+  bool any_normals = false, any_skinned = false;
+  uint32_t max_tri = 0;
   uint64_t last_id = 0;
   Mesh* last = nullptr;
   auto find_mesh = [&](uint64_t id) -> Mesh* {
@@ -1358,6 +1381,7 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
       Mesh* m = find_mesh(md.mesh);   // validate_desc found it
       mesh_worst_case(*m, vchunk, tile);
       const uint32_t np = (uint32_t)m->parts.size();
+      max_tri = std::max(max_tri, m->max_part);
       nm++;
       ncand += np;
       if (md.materials) nmat += np;
@@ -1369,6 +1393,7 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
       }
       wpl += (uint64_t)np * lc;
       if (md.skinned) {
+        any_skinned = true;
         pal_floats += 16ull * md.bone_count;
         if (md.bone_poses) {
           pose_bones += md.bone_count;
@@ -1427,11 +1452,10 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
                           4 * carve_size<uint32_t>(ncand) + carve_size<float>(ncand) + carve_size<int32_t>(ncand) +
                           carve_size<uint4>(2 * ncand) + 2 * carve_size<uint4>(ncand) + 2 * carve_size<uint32_t>(ndesc) +
                           carve_size<uint32_t>(8ull * maxP) +
-                          carve_size<float4>(2 * wV) + carve_size<float4>(wV) + carve_size<uint32_t>(wT) +
-                          2 * carve_size<uint4>(wT) + carve_size<uint32_t>(whist) + carve_size<uint32_t>(wsb) +
-                          2 * carve_size<uint32_t>(wtiles) + carve_size<uint32_t>(wvch) + carve_size<float4>(128) +
+                          record_scratch(wV, wT, any_skinned) + carve_size<uint32_t>(whist) + carve_size<uint32_t>(wsb) +
+                          2 * carve_size<uint32_t>(wtiles) + carve_size<uint32_t>(wvch) +
                           carve_size<PartLight>(wpl) + carve_size<M4>(pose_bones) +
-                          carve_size<float4>(any_normals ? wV : 1) + carve_size<float>(wV);
+                          carve_size<float4>(any_normals ? wV : 1);
   t3d_status st = ensure(c, f->tables, f->tables_cap, tbytes);
   if (st) return st;
   if (tbytes > f->pinned_cap) {
@@ -1647,26 +1671,16 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   ms.vchunk = vchunk;
   ms.tile = tile;
   ms.max_pairs = maxP;
-  {
-    float4* v = sc.take<float4>(2 * wV);
-    a.vstride = tu.vertex_split ? 1u : 2u;
-    a.vclip = v;
-    a.vcol = tu.vertex_split ? v + wV : v + 1;
-  }
-  a.vpos = sc.take<float4>(wV);
-  a.key = sc.take<float>(wT);
-  a.tri_rec = sc.take<uint4>(wT);
-  a.tri_vo = sc.take<uint4>(wT);
+  take_records(sc, a, wV, wT, any_skinned);
+  f->max_triangles = max_tri;
   a.hist = sc.take<uint32_t>(whist);
   a.bsum = sc.take<uint32_t>(wsb);
   a.tile_count = sc.take<uint32_t>(wtiles);
   a.tile_part = sc.take<uint32_t>(wtiles);
   a.vchunk_part = sc.take<uint32_t>(wvch);
-  a.sink = sc.take<float4>(128);
   a.plights = sc.take<PartLight>(wpl);
   a.pose_world = sc.take<M4>(pose_bones);
   a.vnrm = sc.take<float4>(any_normals ? wV : 1);
-  a.vud = sc.take<float>(wV);
   Carve oc{reinterpret_cast<uint8_t*>(f->outputs.ptr)};
   a.out_color = reinterpret_cast<float4*>(oc.take<t3d_vertex>(3 * wT));
   a.out_depth = reinterpret_cast<float4*>(oc.take<t3d_vertex>(3 * wT));
@@ -2213,12 +2227,13 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
                           carve_size<PaletteJob>(npose) + carve_size<uint2>(ngroups);
   // scratch: vertex records, skinned positions, keys, survivor records, stats, histograms, block sums
   const uint32_t ntiles_total = f->tile_prefix.back();
-  const uint64_t sbytes = carve_size<float4>(2 * sumV) + carve_size<float4>(sumV) + carve_size<uint32_t>(sumT) +
-                          2 * carve_size<uint4>(sumT) + carve_size<uint32_t>(4ull * P_n) + carve_size<uint32_t>(sumHist) +
-                          carve_size<uint32_t>(sblocks) + 2 * carve_size<uint32_t>(ntiles_total) +
-                          carve_size<uint32_t>(f->vchunk_prefix.back()) + carve_size<float4>(128) +
-                          carve_size<PartLight>(n_plights) + carve_size<M4>(pose_bones) +
-                          carve_size<float4>(any_normals ? sumV : 1) + carve_size<float>(sumV);
+  bool any_skinned = false;
+  for (uint32_t i = 0; i < P_n && !any_skinned; i++) any_skinned = (f->parts[i].flags & PF_SKINNED) != 0;
+  const uint64_t rest = carve_size<uint32_t>(4ull * P_n) + carve_size<uint32_t>(sumHist) +
+                        carve_size<uint32_t>(sblocks) + 2 * carve_size<uint32_t>(ntiles_total) +
+                        carve_size<uint32_t>(f->vchunk_prefix.back()) + carve_size<PartLight>(n_plights) +
+                        carve_size<M4>(pose_bones) + carve_size<float4>(any_normals ? sumV : 1);
+  const uint64_t sbytes = rest + record_scratch(sumV, sumT, any_skinned);
   uint8_t *tables_dev, *tables_host, *scratch_dev;
   t3d_vertex *out_color, *out_depth, *out_normal = nullptr;
   uint32_t* out_idx;
@@ -2227,9 +2242,13 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
       return fail(c, T3D_ERR_UNSUPPORTED, "render_noalloc: Camera.RenderNormals needs a normal vertex array, which "
                                           "this entry point does not take");
     // no allocation: tables and scratch carved from the placement's scratch, outputs the caller's
-    if (tbytes + sbytes > place->scratch_bytes)
+    const uint64_t charge = tbytes + rest + placed_charge(sumV, sumT);
+    if (charge > place->scratch_bytes)
       return fail(c, T3D_ERR_BUDGET, "render_noalloc: the frame needs %llu bytes of scratch, the static scratch holds %llu",
-                  (unsigned long long)(tbytes + sbytes), (unsigned long long)place->scratch_bytes);
+                  (unsigned long long)charge, (unsigned long long)place->scratch_bytes);
+    if (tbytes + sbytes > place->scratch_room)
+      return fail(c, T3D_ERR_BUDGET, "render_noalloc: the frame's records need %llu bytes, the static array has %llu",
+                  (unsigned long long)(tbytes + sbytes), (unsigned long long)place->scratch_room);
     if (3 * sumT > place->capacity)
       return fail(c, T3D_ERR_INVALID_ARGUMENT, "render_noalloc: outputs hold %llu vertices, the frame needs %llu",
                   (unsigned long long)place->capacity, (unsigned long long)(3 * sumT));
@@ -2369,27 +2388,18 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   a.tile_prefix = d_tpre;
   a.sblock_prefix = d_spre;
   a.pscan_prefix = d_ppre;
-  {
-    float4* v = sc.take<float4>(2 * sumV);
-    a.vstride = tu.vertex_split ? 1u : 2u;
-    a.vclip = v;
-    a.vcol = tu.vertex_split ? v + sumV : v + 1;
-  }
-  a.vpos = sc.take<float4>(sumV);
-  a.key = sc.take<float>(sumT);
-  a.tri_rec = sc.take<uint4>(sumT);
-  a.tri_vo = sc.take<uint4>(sumT);
+  take_records(sc, a, sumV, sumT, any_skinned);
+  f->max_triangles = 0;
+  for (const PartGPU& P : f->parts) f->max_triangles = std::max(f->max_triangles, P.tcount);
   a.stats = sc.take<uint32_t>(4ull * P_n);
   a.hist = sc.take<uint32_t>(sumHist);
   a.bsum = sc.take<uint32_t>(sblocks);
   a.tile_count = sc.take<uint32_t>(ntiles_total);
   a.tile_part = sc.take<uint32_t>(ntiles_total);
   a.vchunk_part = sc.take<uint32_t>(f->vchunk_prefix.back());
-  a.sink = sc.take<float4>(128);
   a.plights = sc.take<PartLight>(n_plights);
   a.pose_world = sc.take<M4>(pose_bones);
   a.vnrm = sc.take<float4>(any_normals ? sumV : 1);
-  a.vud = sc.take<float>(sumV);
   a.out_normal = reinterpret_cast<float4*>(out_normal);
   a.pal_jobs = d_pjobs;
   a.groups = d_groups;
@@ -2451,10 +2461,11 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
     }
   } else if (allow_graph && c->tuning.use_graph && !(profile && c->profiling)) {
     // graph of the whole chain; reused while the launch shape is unchanged
-    std::vector<uint8_t> key(sizeof(FrameArgs) + 9 * sizeof(uint32_t));
-    uint32_t shape[9] = {f->total_vchunks,       f->total_tiles,           f->total_sblocks,
+    std::vector<uint8_t> key(sizeof(FrameArgs) + 10 * sizeof(uint32_t));
+    uint32_t shape[10] = {f->total_vchunks,       f->total_tiles,           f->total_sblocks,
                          f->vertex_threads,      c->tuning.store_mode,     c->tuning.scatter_waves,
-                         c->tuning.assemble_split, c->tuning.cull_block,   f->total_pscan};
+                         c->tuning.assemble_split, c->tuning.cull_block,   f->total_pscan,
+                         f->max_triangles};
     std::memcpy(key.data(), &a, sizeof(FrameArgs));
     std::memcpy(key.data() + sizeof(FrameArgs), shape, sizeof shape);
     if (!f->graph_exec || key != f->graph_key) {
@@ -3070,10 +3081,8 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
       {&t3d_tuning::vertices_per_thread, {1, 2, 4}},
       {&t3d_tuning::scatter_waves, {1, 4}},
       {&t3d_tuning::assemble_split, {1, 2, 4, 8, 16, 32}},
-      {&t3d_tuning::store_mode, {0, 2, 4, 6, 8, 10, 12, 14, 16, 18, 20, 22, 34, 38, 50, 54, 80, 82, 114}},   // staged rows (64 or
-                                      // 32), streaming or not, pipelined or not, 1 or 4 waves, one stream per block
+      {&t3d_tuning::store_mode, {16, 18, 80, 82}},   // streaming stores or not, block order
       {&t3d_tuning::xcd_swizzle, {0, 1}},
-      {&t3d_tuning::vertex_split, {0, 1}},
       {&t3d_tuning::cull_block, {256, 512, 1024}},
       {&t3d_tuning::model_stage, {0, 1}},
   };
@@ -3107,10 +3116,9 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
       }
       if (st) break;
     }
-    // four-wave assembly blocks want larger slot ranges per block than one-wave blocks: store mode and
-    // assembly split together
-    for (uint32_t mode : {16u, 18u, 20u, 22u, 50u, 54u, 80u, 82u})
-      for (uint32_t split : {1u, 2u, 4u, 8u}) {
+    // how finely the assembly is split and in which order its blocks run go together
+    for (uint32_t mode : {18u, 82u})
+      for (uint32_t split : {2u, 4u, 8u, 16u}) {
         if (st) break;
         t3d_tuning t = best;
         t.store_mode = mode;

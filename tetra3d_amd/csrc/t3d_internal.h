@@ -7,11 +7,11 @@
 //     unit-stride coalesced load.
 //   frame tables (uploaded per render): PartGPU[P], LightGPU[L], PartLight[sum],
 //     block->part prefix arrays.
-//   frame scratch: per vertex a clip f32x4 and a colour f32x4, interleaved
-//     (one 32-byte record per vertex) or as two arrays (the cull pass then
-//     reads only clip positions), vpos[sumV] f32x4 (skinned positions),
-//     key[sumT] f32,
-//     tri_rec/tri_vo[sumT] u32x4 (survivor records by triangle / by slot),
+//   frame scratch: per vertex vab f32x4 x 2 (the first two thirds of its
+//     ebiten colour vertex), vq f32x4 (screen position, depth, Custom0) and
+//     vz u8 (Z inside the range); vpos[sumV] f32x4 (skinned positions, frames
+//     with a skinned model only); key[sumT] f32 and tri_loc[sumT] u16 (each
+//     tile's survivors), tri_vo[sumT] u32x4 (survivor records by slot),
 //     stats[P] u32x4, hist, bsum.
 //   outputs: color[3*sumT] t3d_vertex, depth[3*sumT] t3d_vertex, idx[3*sumT] u32;
 //     render pair p owns vertices [out_base, out_base + 3*T_p) and fills the
@@ -28,7 +28,8 @@ constexpr uint32_t kBins = 512;        // sortingTriangles.go:166-168
 constexpr uint32_t kMaxLights = 64;    // lights of one pair the vertex pass stages in LDS (more are read from HBM)
 constexpr uint32_t kMaxLdsBones = 64;  // bone palettes staged in LDS up to this size
 constexpr uint32_t kScanBlock = 2048;  // elements per scan block (256 threads x 8)
-constexpr uint32_t kMaxTile = 2048;    // triangles per tile (keys of a tile are staged in LDS)
+constexpr uint32_t kMaxTile = 2048;    // triangles per tile (keys of a tile are staged in LDS; below 2^16: tri_loc)
+constexpr uint64_t kTouchVertices = 2400000;  // frames with more vertex records read them ahead of the assembly
 constexpr uint32_t kScanPartMax = 65536;  // histogram matrices up to this size are scanned by one block
 
 // PartGPU.flags
@@ -295,33 +296,32 @@ struct FrameArgs {
   uint32_t nparts;
   uint32_t vchunk;              // vertices per vertex-kernel block
   uint32_t tile;                // triangles per tile
-  uint32_t xcd_swizzle;         // 1: give each XCD a contiguous range of blocks (see block_index)
+  uint32_t xcd_swizzle;         // 1: give each XCD a contiguous range of blocks (see block_index_n)
+  uint32_t touch_records;       // 1: more vertex records than the memory-side cache keeps (see k_scatter4)
+  uint32_t pad0;
   const LightGPU* lights;
   PartLight* plights;
   const uint32_t* vchunk_prefix;  // [P+1]
   const uint32_t* tile_prefix;    // [P+1]
   const uint32_t* sblock_prefix;  // [P+1]
   const uint32_t* pscan_prefix;   // [P+1] one k_scan_part block per multi-tile part with a small matrix
-  float4* vclip;                // clip position of vertex record o at vclip[o * vstride]
-  float4* vcol;                 // its colour at vcol[o * vstride]
-  uint32_t vstride;             // 2: interleaved records; 1: two arrays
-  uint32_t pad1;
-  float4* vpos;
+  float4* vab;                  // [sumV][2] DstX, DstY, SrcX, SrcY and the colour of each vertex record
+  float4* vq;                   // [sumV] X/W and Y/W as the cull tests them, the depth list's value, Custom0
+  uint8_t* vz;                  // [sumV] 1: Z inside the camera's range
+  float4* vpos;                 // [sumV] skinned positions (frames with a skinned model)
   float* key;
-  uint4* tri_rec;               // [sumT] survivors, triangle order: {vertex-record offsets x3, triangle}
-  uint4* tri_vo;                // [sumT] the same records in output-slot order
-  uint32_t* stats;              // [P][4]: min bits, max bits, survivors, 0
+  uint16_t* tri_loc;            // [sumT] survivors, triangle order: the triangle's place in its tile
+  uint4* tri_vo;                // [sumT] survivors, output-slot order: {vertex-record offsets x3, triangle}
+  uint32_t* stats;              // [P][4]: min bits, max bits, survivors, 1 when some vertex's Z is out of range
   uint32_t* tile_count;         // [tiles] survivors of each tile (compacted at the tile's front)
   uint32_t* tile_part;          // [tiles] render pair of each tile (written by k_uniforms)
   uint32_t* vchunk_part;        // [vertex chunks] render pair of each vertex-kernel block (k_uniforms)
-  float4* sink;                 // [128] store target of lanes past the end of a chunk (never read)
   uint32_t* hist;
   uint32_t* bsum;
   float4* out_color;            // t3d_vertex as 3 float4
   float4* out_depth;
   uint32_t* out_idx;
   float4* vnrm;                 // [sumV] normal-list colour per vertex record (render_normals cameras only)
-  float* vud;                   // [sumV] unbillboarded depth Z per vertex record (PF_UNBB parts only)
   float4* out_normal;           // normal vertices, laid out as out_color (null when no camera renders normals)
   const FrameConst* fc;         // [jobs] device copies, so graph kernel arguments stay fixed across frames
   const PaletteJob* pal_jobs;   // [npal_jobs] armatures posed on the device
@@ -399,10 +399,10 @@ hipError_t launch_scan(const FrameArgs& a, uint32_t sblk0, uint32_t nsblk, uint3
                        hipStream_t s);
 hipError_t launch_scan_part(const FrameArgs& a, uint32_t blk0, uint32_t nblk, hipStream_t s);
 hipError_t launch_scatter(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t waves, hipStream_t s);
+// max_triangles: the largest render pair's (a bound is enough)
 hipError_t launch_assemble(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t mode, uint32_t split,
-                           hipStream_t s);
+                           uint32_t max_triangles, hipStream_t s);
 hipError_t launch_pack(const PackArgs& a, uint32_t nblocks, hipStream_t s);
-hipError_t launch_normals(const FrameArgs& a, uint32_t blk0, uint32_t nblk, hipStream_t s);
 hipError_t launch_groups(const FrameArgs& a, uint32_t part0, uint32_t part1, hipStream_t s);
 // The model-level stage of a device-built frame (t3d_models.hip): k_models, then k_plist.
 hipError_t launch_model_stage(const FrameArgs& a, hipStream_t s);

@@ -17,14 +17,16 @@
 //   k_scan*     exclusive scan of each part's [bin][tile] histogram matrix
 //   k_scatter   stable counting sort: output slot of every survivor
 //               (sortingTriangleBucket Sort + ForEach, sortingTriangles.go:38-125)
-//   k_assemble  per drawn triangle in slot order: ebiten colour/depth vertices
-//               and indices, staged in LDS and written as contiguous float4 rows
-//               with streaming stores (camera.go:1646-1820)
-//   k_normals   Camera.RenderNormals: the normal vertex list (camera.go:1710-1722)
+//   k_assemble  per drawn triangle in slot order: ebiten colour/depth vertices,
+//               indices and, with Camera.RenderNormals, the normal vertices,
+//               copied from the vertex records with streaming stores
+//               (camera.go:1646-1820)
 //
 // All arithmetic is float32 in the reference's order; the build uses
 // -ffp-contract=off and correctly rounded division and square root.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "t3d_internal.h"
 #include "t3d_stage.h"
@@ -57,7 +59,16 @@ __device__ __forceinline__ uint32_t block_index_n(uint32_t swizzle, uint32_t n) 
   const uint32_t per = n / kXcds, rem = n % kXcds, x = i % kXcds;
   return x * per + min(x, rem) + i / kXcds;
 }
-__device__ __forceinline__ uint32_t block_index(uint32_t swizzle) { return block_index_n(swizzle, gridDim.x); }
+// The assembly's map: runs of kAsmRun consecutive blocks go to one XCD and the
+// next run to the next, so the eight XCDs also share a pair whose drawn
+// triangles fill only the first part of its blocks.  Blocks past the last
+// whole group keep their number, so this too is a bijection of [0, n).
+constexpr uint32_t kAsmRun = 16;
+__device__ __forceinline__ uint32_t block_index_runs(uint32_t swizzle, uint32_t n) {
+  const uint32_t i = blockIdx.x, per = kXcds * kAsmRun, g = i / per, r = i % per;
+  if (!swizzle || (g + 1) * per > n) return i;
+  return g * per + (r % kXcds) * kAsmRun + r / kXcds;
+}
 
 // The logical block of this workgroup.  A frame built on the device is
 // launched for every candidate pair being drawn; its actual block count is
@@ -65,13 +76,14 @@ __device__ __forceinline__ uint32_t block_index(uint32_t swizzle) { return block
 // kNoBlock (block-uniform: the whole workgroup returns).  The swizzle then
 // deals the actual blocks, not the launch's, over the XCDs.
 constexpr uint32_t kNoBlock = 0xFFFFFFFFu;
+template <bool kRuns = false>
 __device__ __forceinline__ uint32_t frame_block(const FrameArgs& a, uint32_t which, uint32_t mult) {
   uint32_t n = gridDim.x;
   if (a.counts) {
     n = a.counts[which] * mult;
     if (blockIdx.x >= n) return kNoBlock;
   }
-  return block_index_n(a.xcd_swizzle, n);
+  return kRuns ? block_index_runs(a.xcd_swizzle, n) : block_index_n(a.xcd_swizzle, n);
 }
 // The same for the launches that never swizzle (scan blocks, pairs).
 __device__ __forceinline__ bool past_count(const FrameArgs& a, uint32_t which) {
@@ -221,6 +233,53 @@ __device__ __forceinline__ void light_vertex(const LightGPU& l, const PartLight&
 // k_vertex
 // ---------------------------------------------------------------------------
 
+// What the later passes read of a vertex, computed once here instead of once
+// per triangle corner (about six corners share a vertex): the first two
+// float4 of its ebiten colour vertex (a: DstX, DstY, SrcX, SrcY, b: colour),
+// and q: the screen position the cull tests, the depth list's value and
+// Custom0.  zin: its Z is inside the camera's range.
+struct VertexRecord {
+  float4 a, b, q;
+  bool zin;
+};
+
+// Screen position, texture position and depth of a vertex from its clip
+// position (model.go:869-887, camera.go:1655-1711, 1765-1784).  Where the
+// cull's and the assembly's clamps of W leave it alone (W > 0, perspective)
+// their quotients are one: y / -w is -(y / w) in every rounding.
+__device__ __forceinline__ void place_vertex(const FrameConst& fc, V4 clip, float zd, float2 uv, float src_w,
+                                             float src_h, VertexRecord& r) {
+  const bool persp = fc.perspective != 0;
+  const float wc = clip.w < 0 ? 0.000001f : clip.w;
+  const float nx = fdiv(clip.x, wc), ny = fdiv(clip.y, wc);
+  float w = clip.w;                                               // camera.go:1655-1667
+  if (!persp) w = 1.0f;
+  if (w < 0) w = 0.001f;
+  float qx = nx, qy = -ny;
+  if (!(persp && clip.w > 0)) {
+    qx = fdiv(clip.x, w);
+    qy = fdiv(clip.y, -w);
+  }
+  float uvU, uvV, c0 = 0.0f;
+  if (fc.pc_tex) {                                                // camera.go:1688-1711
+    uvU = fdiv(uv.x, w) * src_w;
+    uvV = fdiv(1.0f - uv.y, w) * src_h;
+    c0 = fdiv(1.0f, w);
+  } else {
+    uvU = uv.x * src_w;
+    uvV = (1.0f - uv.y) * src_h;
+  }
+  float depth = 0.0f;
+  if (fc.render_depth) {                                          // camera.go:1765-1784
+    depth = fdiv(zd + fc.dmp, fc.spread);
+    if (depth < 0) depth = 0;
+    else if (depth > 1) depth = 1;
+  }
+  r.a = make_float4(qx * fc.cam_w + fc.half_w, qy * fc.cam_h + fc.half_h, uvU, uvV);
+  r.q = make_float4(nx, ny, depth, c0);
+  r.zin = clip.z + 1.0f >= fc.near_ && clip.z < fc.far_;          // model.go:883-886
+}
+
 __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_VCHUNKS, 1);
   if (lb == kNoBlock) return;
@@ -257,6 +316,7 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
   const FrameConst fc = a.fc[P.cam];
   const uint32_t first = (b - a.vchunk_prefix[p]) * a.vchunk;
   const uint32_t last = min(first + a.vchunk, P.vcount);
+  bool out_of_range = false;
   for (uint32_t i = first + threadIdx.x; i < last; i += blockDim.x) {
     const uint32_t v = P.vmin + i;
     // VertexPositionWithShapeKeys / VertexNormalWithShapeKeys (mesh.go:796-822)
@@ -280,6 +340,7 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
     }
     V3 vp, vn;
     V4 clip;
+    float zu = 0.0f;                                                // Z of DepthModeUnbillboarded
     if (skinned) {
       // Model.skinVertex (model.go:559-596)
       const ushort4 bi = reinterpret_cast<const ushort4*>(P.bones)[v];
@@ -321,7 +382,7 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
       vp = pos;
       vn = nrm;
       clip = mult_vec_w(P.mvp, pos);                                // model.go:795-798
-      if (flags & PF_UNBB) a.vud[P.vbase + i] = mult_vec_w(s_umvp, pos).z;   // model.go:800-803, not snapped
+      if (flags & PF_UNBB) zu = mult_vec_w(s_umvp, pos).z;          // model.go:800-803, not snapped
     }
     if (fc.snap > 0) {                                              // model.go:807-812
       clip.x = fdiv(roundf(clip.x * fc.snap), fc.snap);
@@ -383,10 +444,18 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
       const V3 tn = mult_vec(P.nrot, vp);
       a.vnrm[o] = make_float4(tn.x * 0.5f + 0.5f, tn.y * 0.5f + 0.5f, tn.z * 0.5f + 0.5f, 0.0f);
     }
-    a.vclip[(size_t)o * a.vstride] = make_float4(clip.x, clip.y, clip.z, clip.w);
-    a.vcol[(size_t)o * a.vstride] = make_float4(cr, cg, cb, ca);
+    const float2 uv = (flags & PF_HAS_UV) ? reinterpret_cast<const float2*>(P.uv)[v] : make_float2(0.0f, 0.0f);
+    VertexRecord r;
+    place_vertex(fc, clip, (flags & PF_UNBB) ? zu : clip.z, uv, P.src_w, P.src_h, r);
+    a.vab[2 * (size_t)o + 0] = r.a;
+    a.vab[2 * (size_t)o + 1] = make_float4(cr, cg, cb, ca);
+    a.vq[o] = r.q;
+    a.vz[o] = r.zin ? 1 : 0;
+    out_of_range |= !r.zin;
     if (skinned) a.vpos[o] = make_float4(vp.x, vp.y, vp.z, 0.0f);
   }
+  // a pair with no vertex out of the Z range needs no look at vz in the cull
+  if (__ballot(out_of_range) && threadIdx.x % 64 == 0) a.stats[4 * p + 3] = 1u;   // every writer stores the same word
 }
 
 // ---------------------------------------------------------------------------
@@ -491,11 +560,14 @@ __global__ __launch_bounds__(kPoseThreads) void k_palettes(FrameArgs a) {
 // pair, beginModel's working position (light.go:175-189), the per-model
 // point-light skip (camera.go:1592, 1625-1629) and the per-object LightVolume
 // cell (light.go:610-628).  The same float32 functions the host would run, so
-// the values are the ones the reference computes on the CPU.  One wavefront
-// per render pair: lane k handles the pair's lights k, k + 64, ..., lane 0 also the pair's own uniforms and the reset of its depth range
+// the values are the ones the reference computes on the CPU.  One block per
+// render pair: lane k handles the pair's lights k, k + 64, ..., lane 0 also the pair's own uniforms and the reset of its depth range
 // and survivor count, so the latency is one light's, not the sum over lights;
-// all lanes first write the pair's entries of the block->pair maps.
-__global__ __launch_bounds__(64) void k_uniforms(FrameArgs a, uint32_t part0, uint32_t nparts) {
+// all wavefronts first write the pair's entries of the block->pair maps (a
+// 1024 x 1024 grid has over 5,000, which one wavefront took 11 us to store);
+// the first then works alone.
+constexpr uint32_t kUniformThreads = 256;
+__global__ __launch_bounds__(kUniformThreads) void k_uniforms(FrameArgs a, uint32_t part0, uint32_t nparts) {
   if (past_count(a, FC_PAIRS)) return;
   PartGPU& P = const_cast<PartGPU*>(a.parts)[part0 + blockIdx.x];
   if (a.counts) {   // a device-built frame: the pair's record is built here from the model, mesh and material
@@ -505,15 +577,16 @@ __global__ __launch_bounds__(64) void k_uniforms(FrameArgs a, uint32_t part0, ui
     static_assert(sizeof(PartGPU) % 16 == 0, "whole float4 rows");
     const float4* src = reinterpret_cast<const float4*>(&s_part);
     float4* dst = reinterpret_cast<float4*>(&P);
-    for (uint32_t i = threadIdx.x; i < sizeof(PartGPU) / 16; i += 64) dst[i] = src[i];
+    for (uint32_t i = threadIdx.x; i < sizeof(PartGPU) / 16; i += kUniformThreads) dst[i] = src[i];
     __syncthreads();
   }
   const uint32_t k = threadIdx.x;
   {  // block -> pair maps of the later kernels: one load where a search over the prefixes took nine
     const uint32_t p = part0 + blockIdx.x;
-    for (uint32_t i = a.tile_prefix[p] + k; i < a.tile_prefix[p + 1]; i += 64) a.tile_part[i] = p;
-    for (uint32_t i = a.vchunk_prefix[p] + k; i < a.vchunk_prefix[p + 1]; i += 64) a.vchunk_part[i] = p;
+    for (uint32_t i = a.tile_prefix[p] + k; i < a.tile_prefix[p + 1]; i += kUniformThreads) a.tile_part[i] = p;
+    for (uint32_t i = a.vchunk_prefix[p] + k; i < a.vchunk_prefix[p + 1]; i += kUniformThreads) a.vchunk_part[i] = p;
   }
+  if (k >= 64) return;
   const uint32_t flags = P.flags;
   const uint32_t nl = (flags & PF_LIGHTING) ? P.light_count : 0u;
   if (k > 0 && k >= nl) return;
@@ -590,6 +663,51 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 // k_cull
 // ---------------------------------------------------------------------------
 
+// The vertex records of triangle t's corners.
+__device__ __forceinline__ void corner_records(const PartGPU& P, uint32_t t, uint32_t (&ov)[3]) {
+  const uint32_t d = P.vbase - P.vmin;
+  if (P.idx16) {                                  // uniform: the pair's mesh index width
+    const uint16_t* ix = P.idx16 + 3 * (size_t)t;
+    for (int k = 0; k < 3; k++) ov[k] = d + ix[k];
+  } else {
+    const uint32_t* ix = P.idx + 3 * (size_t)t;
+    for (int k = 0; k < 3; k++) ov[k] = d + ix[k];
+  }
+}
+
+// Whether a triangle is drawn, from its corners' screen positions and whether
+// any is inside the Z range (model.go:855-925).
+__device__ __forceinline__ bool visible(const float4 (&c)[3], bool zin, bool backface) {
+  if (!zin) return false;
+  if ((c[0].x < -0.5f && c[1].x < -0.5f && c[2].x < -0.5f) || (c[0].x > 0.5f && c[1].x > 0.5f && c[2].x > 0.5f) ||
+      (c[0].y < -0.5f && c[1].y < -0.5f && c[2].y < -0.5f) || (c[0].y > 0.5f && c[1].y > 0.5f && c[2].y > 0.5f))
+    return false;                                                       // model.go:890-898
+  if (backface) {                                                       // model.go:902-925
+    const float n0x = c[0].x - c[1].x;
+    const float n0y = c[0].y - c[1].y;
+    const float n1x = c[1].x - c[2].x;
+    const float n1y = c[1].y - c[2].y;
+    const float nor = (n0x * n1y) - (n1x * n0y);
+    if (nor < 0) return false;
+  }
+  return true;
+}
+
+// Squared distance of a triangle's centre from the camera: a skinned
+// triangle's three positions, or a static one's stored Triangle.Center
+// (mesh.go:1980-1982) in q[0].
+__device__ __forceinline__ float depth_key(bool skinned, V3 cam, V3 icp, const V3 (&q)[3]) {
+  V3 from = icp, c = q[0];
+  if (skinned) {                                                        // model.go:860-864, 941-960
+    from = cam;
+    V3 s = v3(0, 0, 0);
+    for (int k = 0; k < 3; k++) s = add(s, q[k]);
+    c = v3(fdiv(s.x, 3.0f), fdiv(s.y, 3.0f), fdiv(s.z, 3.0f));
+  }
+  const float dx = from.x - c.x, dy = from.y - c.y, dz = from.z - c.z;
+  return dx * dx + dy * dy + dz * dz;
+}
+
 // kThreads: 256, 512 or 1024 threads per tile block (tunable).
 template <uint32_t kThreads>
 __global__ __launch_bounds__(kThreads) void k_cull(FrameArgs a, uint32_t blk0) {
@@ -610,7 +728,8 @@ __global__ __launch_bounds__(kThreads) void k_cull(FrameArgs a, uint32_t blk0) {
   const V3 icp = v3(P.icp[0], P.icp[1], P.icp[2]);
 
   // Survivors are compacted in triangle order to the front of the tile's
-  // range of key[] and tri_rec[]; tile_count[b] says how many there are.
+  // range of key[] and tri_loc[]; tile_count[b] says how many there are.
+  const bool look_z = !all && a.stats[4 * p + 3] != 0;   // some vertex of the pair is out of the Z range
   float mn = kMaxF32, mx = 0.0f;
   const uint32_t wv = threadIdx.x / warpSize, ln = threadIdx.x % warpSize;
   const uint64_t lt_mask = (ln == 0) ? 0ull : (~0ull >> (64 - ln));
@@ -620,31 +739,17 @@ __global__ __launch_bounds__(kThreads) void k_cull(FrameArgs a, uint32_t blk0) {
     const uint32_t t = base + threadIdx.x;
     bool keep = false;
     float depth = -1.0f;
-    uint32_t ov[3] = {0, 0, 0};
     if (t < t1) {
-      uint32_t i0, i1, i2;
-      if (P.idx16) {                              // uniform: the pair's mesh index width
-        i0 = P.idx16[3 * (size_t)t + 0];
-        i1 = P.idx16[3 * (size_t)t + 1];
-        i2 = P.idx16[3 * (size_t)t + 2];
-      } else {
-        i0 = P.idx[3 * (size_t)t + 0];
-        i1 = P.idx[3 * (size_t)t + 1];
-        i2 = P.idx[3 * (size_t)t + 2];
-      }
-      const uint32_t vi[3] = {i0, i1, i2};
-      float nx[3], ny[3];
-      bool outOfBounds = true;
-      V3 stc = v3(0, 0, 0);
-      // every gather of the triangle first, so their latencies overlap: clip
-      // positions, and what its depth key needs (a static triangle's stored
-      // Triangle.Center, or the three skinned positions)
+      uint32_t ov[3];
+      corner_records(P, t, ov);
+      // every gather of the triangle first, so their latencies overlap:
+      // screen positions, and what its depth key needs (a static triangle's
+      // stored Triangle.Center, or the three skinned positions)
       float4 cc[3];
       V3 q[3];
-      for (int k = 0; k < 3; k++) {
-        ov[k] = P.vbase + (vi[k] - P.vmin);
-        cc[k] = a.vclip[(size_t)ov[k] * a.vstride];
-      }
+      bool zin = true;
+      for (int k = 0; k < 3; k++) cc[k] = a.vq[ov[k]];
+      if (look_z) zin = (a.vz[ov[0]] | a.vz[ov[1]] | a.vz[ov[2]]) != 0;
       if (skinned) {
         for (int k = 0; k < 3; k++) {
           const float4 s = a.vpos[ov[k]];
@@ -654,45 +759,9 @@ __global__ __launch_bounds__(kThreads) void k_cull(FrameArgs a, uint32_t blk0) {
         const float* cp = P.ctr + 3 * (size_t)t;
         q[0] = v3(cp[0], cp[1], cp[2]);
       }
-      for (int k = 0; k < 3; k++) {                                   // model.go:855-886
-        const float4 c = cc[k];
-        if (skinned) {
-          stc.x += q[k].x;
-          stc.y += q[k].y;
-          stc.z += q[k].z;
-        }
-        float w = c.w;
-        if (w < 0) w = 0.000001f;
-        nx[k] = fdiv(c.x, w);
-        ny[k] = fdiv(c.y, w);
-        if (c.z + 1.0f >= fc.near_ && c.z < fc.far_) outOfBounds = false;
-      }
-      keep = all || !outOfBounds;
-      if (keep && !all && ((nx[0] < -0.5f && nx[1] < -0.5f && nx[2] < -0.5f) ||      // model.go:890-898
-                   (nx[0] > 0.5f && nx[1] > 0.5f && nx[2] > 0.5f) ||
-                   (ny[0] < -0.5f && ny[1] < -0.5f && ny[2] < -0.5f) ||
-                   (ny[0] > 0.5f && ny[1] > 0.5f && ny[2] > 0.5f)))
-        keep = false;
-      if (keep && !all && backface) {                                  // model.go:902-925
-        const float n0x = nx[0] - nx[1];
-        const float n0y = ny[0] - ny[1];
-        const float n1x = nx[1] - nx[2];
-        const float n1y = ny[1] - ny[2];
-        const float nor = (n0x * n1y) - (n1x * n0y);
-        if (nor < 0) keep = false;
-      }
+      keep = all || visible(cc, zin, backface);
       if (keep) {                                                       // model.go:941-960
-        if (skinned) {
-          const float dx = camPos.x - fdiv(stc.x, 3.0f);
-          const float dy = camPos.y - fdiv(stc.y, 3.0f);
-          const float dz = camPos.z - fdiv(stc.z, 3.0f);
-          depth = dx * dx + dy * dy + dz * dz;
-        } else {
-          const float dx = icp.x - q[0].x;    // Triangle.Center, stored at upload (mesh.go:1980-1982)
-          const float dy = icp.y - q[0].y;
-          const float dz = icp.z - q[0].z;
-          depth = dx * dx + dy * dy + dz * dz;
-        }
+        depth = depth_key(skinned, camPos, icp, q);
         if (!all && (isnan(depth) || isinf(depth))) {
           keep = false;
           depth = -1.0f;
@@ -710,7 +779,7 @@ __global__ __launch_bounds__(kThreads) void k_cull(FrameArgs a, uint32_t blk0) {
     if (keep) {
       const uint32_t pos = P.tbase + t0 + run + wbase + (uint32_t)__popcll(m & lt_mask);
       a.key[pos] = depth;
-      a.tri_rec[pos] = make_uint4(ov[0], ov[1], ov[2], t);
+      a.tri_loc[pos] = (uint16_t)(t - t0);
       mn = fminf(mn, depth);
       mx = fmaxf(mx, depth);
     }
@@ -961,7 +1030,15 @@ __global__ __launch_bounds__(1024) void k_scan_part(FrameArgs a, uint32_t blk0) 
 // histogram, or from a local scan when the part is a single tile.  This is
 // sortingTriangleBucket.Sort + ForEach (sortingTriangles.go:38-125): bins
 // visited 511->0 (BackToFront) or 0->511, insertion order kept within a bin.
-// The survivor's record {vertex-record offsets, triangle} moves to its slot.
+// The survivor's record {vertex-record offsets, triangle} goes to its slot; its
+// corners are read from the mesh's indices here, where the tile's triangles
+// still come in mesh order, so the cull writes 6 bytes per survivor, not 20.
+__device__ __forceinline__ uint4 slot_record(const PartGPU& P, uint32_t t) {
+  uint32_t ov[3];
+  corner_records(P, t, ov);
+  return make_uint4(ov[0], ov[1], ov[2], t);
+}
+
 __global__ __launch_bounds__(64) void k_scatter(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_TILES, 1);
   if (lb == kNoBlock) return;
@@ -974,7 +1051,8 @@ __global__ __launch_bounds__(64) void k_scatter(FrameArgs a, uint32_t blk0) {
   const uint32_t lane = threadIdx.x;
   const uint32_t tbase = P.tbase;
   const uint32_t mode = (P.flags >> PF_SORT_SHIFT) & 3u;
-  const uint4* __restrict__ rec_in = a.tri_rec + tbase + tl * a.tile;
+  const uint32_t t0 = tl * a.tile;
+  const uint16_t* __restrict__ loc = a.tri_loc + tbase + t0;
   uint4* __restrict__ rec_out = a.tri_vo + tbase;
 
   __shared__ uint32_t run[kBins];
@@ -1012,14 +1090,14 @@ __global__ __launch_bounds__(64) void k_scatter(FrameArgs a, uint32_t blk0) {
   }
 
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint4 rec_next = lane < n ? rec_in[lane] : make_uint4(0, 0, 0, 0);   // records one chunk ahead
+  uint4 rec_next = lane < n ? slot_record(P, t0 + loc[lane]) : make_uint4(0, 0, 0, 0);   // records one chunk ahead
   for (uint32_t base_i = 0; base_i < n; base_i += 64) {
     const uint32_t i = base_i + lane;
     const bool valid = i < n;
     const float d = valid ? s_key[i] : -1.0f;
     const uint64_t vmask = __ballot(valid);
     const uint4 rec = rec_next;
-    if (i + 64 < n) rec_next = rec_in[i + 64];
+    if (i + 64 < n) rec_next = slot_record(P, t0 + loc[i + 64]);
     const uint32_t bin = valid ? visit_bin(d, mn, rd, mode) : 0xFFFFFFFFu;
     const uint64_t peers = bin_peers(bin, vmask);
     const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
@@ -1053,7 +1131,7 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
   const uint32_t tid = threadIdx.x, lane = tid % 64u, wv = tid / 64u;
   const uint32_t tbase = P.tbase;
   const uint32_t mode = (P.flags >> PF_SORT_SHIFT) & 3u;
-  const uint4* __restrict__ rec_in = a.tri_rec + tbase;
+  const uint16_t* __restrict__ loc = a.tri_loc + tbase + t0;
   uint4* __restrict__ rec_out = a.tri_vo + tbase;
 
   __shared__ uint32_t s_off[kScatterWaves][kBins];
@@ -1069,6 +1147,24 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
     col_run[0] = col[(size_t)tid * P.ntiles];
     col_run[1] = col[(size_t)(tid + 256) * P.ntiles];
   }
+  // In a large frame, this tile's share of its pair's vertex records, a word
+  // of every 128-byte line, read so that the assembly finds them in the
+  // 256 MB memory-side cache: its reads wait long behind its own stores where
+  // they have to go to HBM.  With 3.9 M vertex records (187 MB) the assembly
+  // takes 212 us with it and 320 us without, this pass 66 us instead of 37;
+  // with 2.8 M 161 and 188 against 49 and 34; with 1.9 M records (94 MB) and
+  // less they are still cached and reading them only costs (113 and 110
+  // against 35 and 25).
+  float touch = 0.0f;
+  if (a.touch_records) {
+    constexpr uint32_t kLine = 128 / sizeof(float);
+    const uint32_t v0 = (uint32_t)((uint64_t)P.vcount * tl / P.ntiles);
+    const uint32_t nv = (uint32_t)((uint64_t)P.vcount * (tl + 1) / P.ntiles) - v0;
+    const float* ab = reinterpret_cast<const float*>(a.vab + 2 * ((size_t)P.vbase + v0));
+    const float* vq = reinterpret_cast<const float*>(a.vq + (size_t)P.vbase + v0);
+    for (uint32_t i = tid * kLine; i < 8 * nv; i += 256 * kLine) touch += ab[i];
+    for (uint32_t i = tid * kLine; i < 4 * nv; i += 256 * kLine) touch += vq[i];
+  }
   const uint32_t nchunks = (n + 63) / 64;
   const uint32_t c0 = (wv * nchunks) / kScatterWaves, c1 = ((wv + 1) * nchunks) / kScatterWaves;
   // every key and record of this wave's chunks (at most kChunks of 64) is
@@ -1076,6 +1172,7 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
   constexpr uint32_t kChunks = kMaxTile / 64 / kScatterWaves;
   float d[kChunks];
   uint4 rec[kChunks];
+  uint32_t tri[kChunks];
   uint32_t bin[kChunks];
   bool in[kChunks];
 #pragma unroll
@@ -1083,8 +1180,10 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
     const uint32_t i = (c0 + j) * 64 + lane;
     in[j] = c0 + j < c1 && i < n;
     d[j] = in[j] ? a.key[tbase + t0 + i] : 0.0f;
-    rec[j] = in[j] ? rec_in[t0 + i] : make_uint4(0, 0, 0, 0);
+    tri[j] = t0 + (in[j] ? loc[i] : 0u);
   }
+#pragma unroll
+  for (uint32_t j = 0; j < kChunks; j++) rec[j] = slot_record(P, tri[j]);   // any lane's triangle is in the mesh
   __syncthreads();
 #pragma unroll
   for (uint32_t j = 0; j < kChunks; j++) {
@@ -1144,6 +1243,7 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
     __builtin_amdgcn_wave_barrier();
     if (valid) rec_out[slot] = rec[j];
   }
+  asm volatile("" ::"v"(touch));                  // the loads are wanted for the caches alone
 }
 
 typedef float f4v __attribute__((ext_vector_type(4)));
@@ -1163,321 +1263,94 @@ __device__ __forceinline__ void store1(uint32_t* p, uint32_t v) {
   else *p = v;
 }
 
-// Output-order assembly: per drawn triangle in slot order,
-// the ebiten colour/depth vertices and indices (camera.go:1646-1820).  The
-// sort pass left each slot's three vertex-record offsets in tri_vo, so the
-// only gathers are the 32-byte vertex records and UVs.  kStage: stage each
-// wavefront's 64 triangles in LDS and write contiguous float4 rows (else each
-// lane stores its own 144-byte runs); kNT: non-temporal (streaming) stores.
-// `split` blocks share one tile's slot range (a power of two dividing the
-// tile), so the grid follows the survivors more finely than the sort's tiles.
-// kOne: each slot range goes to two blocks, adjacent in launch order (so on
-// one XCD, sharing the gathered records in its L2): the first writes the
-// colour vertices and the indices, the second the depth vertices, so every
-// block writes one contiguous output stream.
-template <int kStage, bool kNT, uint32_t kWaves, bool kOne>
-__global__ __launch_bounds__(64 * kWaves) void k_assemble(FrameArgs a, uint32_t blk0, uint32_t split) {
-  constexpr uint32_t kHalves = kOne ? 2 : 1;
-  const uint32_t lf = frame_block(a, FC_TILES, split * kHalves);
-  if (lf == kNoBlock) return;
-  const bool w_color = !kOne || (lf % kHalves) == 0;   // block-uniform
-  const bool w_depth = !kOne || (lf % kHalves) == 1;
-  const uint32_t li = lf / kHalves;
-  const uint32_t b = blk0 + li / split;
-  const uint32_t p = a.tile_part[b];
-  const PartGPU P = a.parts[p];        // by value: read once, before any store
-  const uint32_t S = a.stats[4 * p + 2];
-  const uint32_t sub = a.tile / split;
-  const uint32_t k0 = (b - a.tile_prefix[p]) * a.tile + (li % split) * sub;
-  if (k0 >= S) return;                 // block-uniform: every wave of the block leaves together
-  const uint32_t k1 = min(k0 + sub, S);
-  const FrameConst fc = a.fc[P.cam];
-  const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  // Everything uniform is read once into registers here: the output stores
-  // below may alias these tables as far as the compiler knows, and would
-  // otherwise force a reload (a full memory round trip) per vertex.
-  const uint32_t vbase = P.vbase, vmin = P.vmin, tbase = P.tbase;
-  const bool has_uv = (P.flags & PF_HAS_UV) != 0;
-  const bool unbb = (P.flags & PF_UNBB) != 0;
-  const float* __restrict__ vud = a.vud;
-  const float src_w = P.src_w, src_h = P.src_h;
-  const float* __restrict__ uvp = P.uv;
-  const uint64_t out_base = P.out_base;
-  const uint32_t idx_base = P.idx_base;
-  const bool persp = fc.perspective != 0, pc_tex = fc.pc_tex != 0, rdepth = fc.render_depth != 0;
-  const float cam_w = fc.cam_w, half_w = fc.half_w, cam_h = fc.cam_h, half_h = fc.half_h;
-  const float dmp = fc.dmp, spread = fc.spread;
-  const float4* __restrict__ vclip = a.vclip;
-  const float4* __restrict__ vcol = a.vcol;
-  const uint32_t vstride = a.vstride;
-  const uint4* __restrict__ tvo = a.tri_vo + tbase;
-  float4* __restrict__ out_c = a.out_color + out_base * 3;   // 3 float4 per vertex
-  float4* __restrict__ out_d = a.out_depth + out_base * 3;
-  uint32_t* __restrict__ out_i = a.out_idx + out_base;
-  const float da = rdepth ? 1.0f : 0.0f;
-
-  // kStage 1: all 64 triangles of a wave staged at once; 2: 32 at a time,
-  // halving the LDS per wavefront so twice as many wavefronts fit on a CU.
-  // With kWaves > 1 the block's waves take consecutive 64-triangle chunks of
-  // its slot range, each staging in its own LDS rows.
-  constexpr uint32_t kRows = kStage == 2 ? 32 : 64;
-  __shared__ float4 stage_all[kStage ? kWaves * kRows * 9 : 1];
-  float4* stage = stage_all + (kStage ? wave * kRows * 9 : 0);
-  constexpr uint32_t kStep = 64 * kWaves;
-  uint4 vo_next = make_uint4(0, 0, 0, 0);   // slot records one chunk ahead
-  if (k0 + wave * 64 + lane < k1) vo_next = tvo[k0 + wave * 64 + lane];
-  for (uint32_t base = k0; base < k1; base += kStep) {   // block-uniform trip count
-    const uint32_t wk0 = base + wave * 64;
-    const uint32_t k = wk0 + lane;
-    const bool active = k < k1;
-    const uint32_t wcount = wk0 < k1 ? min(64u, k1 - wk0) : 0u;
-    const uint4 vo = vo_next;
-    if (k + kStep < k1) vo_next = tvo[k + kStep];
-    float4 cq[9];
-    float dd[3];
-    if (active) {
-      const uint32_t ov[3] = {vo.x, vo.y, vo.z};
-      // all nine gathers of the triangle first, so their latencies overlap
-      float4 c[3], col[3];
-      float2 uv[3];
-      for (int vi = 0; vi < 3; vi++) {
-        c[vi] = vclip[(size_t)ov[vi] * vstride];
-        col[vi] = w_color ? vcol[(size_t)ov[vi] * vstride] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        uv[vi] = has_uv ? reinterpret_cast<const float2*>(uvp)[ov[vi] - vbase + vmin] : make_float2(0.0f, 0.0f);
-      }
-      for (int vi = 0; vi < 3; vi++) {
-        float w = c[vi].w;                                        // camera.go:1655-1667
-        if (!persp) w = 1.0f;
-        if (w < 0) w = 0.001f;
-        const float dx = fdiv(c[vi].x, w) * cam_w + half_w;
-        const float dy = fdiv(c[vi].y, -w) * cam_h + half_h;
-        const float U = uv[vi].x, V = uv[vi].y;
-        float uvU, uvV, c0 = 0.0f;
-        if (pc_tex) {                                             // camera.go:1688-1711
-          uvU = fdiv(U, w) * src_w;
-          uvV = fdiv(1.0f - V, w) * src_h;
-          c0 = fdiv(1.0f, w);
-        } else {
-          uvU = U * src_w;
-          uvV = (1.0f - V) * src_h;
-        }
-        float depth = 0.0f;
-        if (rdepth && w_depth) {                                  // camera.go:1765-1784
-          const float zd = unbb ? vud[ov[vi]] : c[vi].z;          // DepthModeUnbillboarded: the unaltered Z
-          depth = fdiv(zd + dmp, spread);
-          if (depth < 0) depth = 0;
-          else if (depth > 1) depth = 1;
-        }
-        cq[3 * vi + 0] = make_float4(dx, dy, uvU, uvV);
-        cq[3 * vi + 1] = col[vi];
-        cq[3 * vi + 2] = make_float4(c0, 0.0f, 0.0f, 0.0f);
-        dd[vi] = depth;
-      }
-    }
-    if (kStage) {
-      for (uint32_t h = 0; h < 64 / kRows; h++) {
-        const uint32_t r0 = h * kRows;                              // first row of this round
-        const uint32_t rows = wcount > r0 ? min(kRows, wcount - r0) : 0u;
-        const bool mine = active && lane >= r0 && lane < r0 + kRows;
-        const uint32_t row = lane - r0;
-        if (w_color) {
-          if (mine)
-            for (int q = 0; q < 9; q++) stage[row * 9 + q] = cq[q];
-          __syncthreads();
-          // a fixed number of (predicated) stores per lane, so the compiler
-          // can count them and wait only for the loads it needs
-#pragma unroll
-          for (uint32_t q = 0; q < (kRows * 9 + 63) / 64; q++) {
-            const uint32_t f = q * 64 + lane;
-            if (f < rows * 9) store4<kNT>(&out_c[(size_t)(wk0 + r0) * 9 + f], stage[f]);
-          }
-          __syncthreads();
-        }
-        if (w_depth) {
-          if (mine)
-            for (int vi = 0; vi < 3; vi++) {
-              if (!w_color) {                                     // rows not staged for the colour list
-                stage[row * 9 + 3 * vi + 0] = cq[3 * vi + 0];
-                stage[row * 9 + 3 * vi + 2] = cq[3 * vi + 2];
-              }
-              stage[row * 9 + 3 * vi + 1] = make_float4(dd[vi], dd[vi], dd[vi], da);
-            }
-          __syncthreads();
-#pragma unroll
-          for (uint32_t q = 0; q < (kRows * 9 + 63) / 64; q++) {
-            const uint32_t f = q * 64 + lane;
-            if (f < rows * 9) store4<kNT>(&out_d[(size_t)(wk0 + r0) * 9 + f], stage[f]);
-          }
-          __syncthreads();
-        }
-      }
-    } else if (active) {
-      float4* oc = out_c + (size_t)k * 9;
-      float4* od = out_d + (size_t)k * 9;
-      if (w_color)
-        for (int q = 0; q < 9; q++) store4<kNT>(&oc[q], cq[q]);
-      if (w_depth)
-        for (int vi = 0; vi < 3; vi++) {
-          store4<kNT>(&od[3 * vi + 0], cq[3 * vi + 0]);
-          store4<kNT>(&od[3 * vi + 1], make_float4(dd[vi], dd[vi], dd[vi], da));
-          store4<kNT>(&od[3 * vi + 2], cq[3 * vi + 2]);
-        }
-    }
-    // indices: flush-local iota, as the reference's indexList (camera.go:1816)
-    if (w_color) {
-#pragma unroll
-      for (uint32_t q = 0; q < 3; q++) {
-        const uint32_t f = q * 64 + lane;
-        if (f < wcount * 3) store1<kNT>(&out_i[(size_t)wk0 * 3 + f], idx_base + wk0 * 3 + f);
-      }
-    }
-  }
-}
-
-// The same assembly, software-pipelined: the nine gathers of chunk i+1 are
-// issued before chunk i's stores, so their latency hides behind the stores.
-// Every memory instruction runs on all 64 lanes (lanes past the end read a
-// clamped slot and write to a sink), which keeps the number of stores per
-// chunk fixed: the wait for the next chunk's gathers can then let the
-// current chunk's stores stay in flight instead of draining them.
-template <uint32_t kRows, bool kNT>
-__global__ __launch_bounds__(64) void k_assemble_pipe(FrameArgs a, uint32_t blk0, uint32_t split) {
-  const uint32_t li = frame_block(a, FC_TILES, split);
+// Output-order assembly: the ebiten colour, depth (and normal) vertices and
+// the indices of a pair's drawn triangles in slot order (camera.go:1646-1820,
+// 1710-1722).  A list of S triangles is 9 * S float4 (three per vertex:
+// position and texture position, colour, custom values), and every lane owns
+// one float4 of each list: it finds its corner's record in the slot records
+// and copies its piece, so a wavefront's stores are whole 1 KB runs with no
+// staging and no barrier, and the three lanes of a corner read one record.
+// A wavefront takes 576 float4 (64 triangles' worth) at a time, all nine
+// gathers of a lane in flight together.  Chunks start at multiples of 64
+// float4 of the whole list, not of the pair's, so every store covers whole
+// 128-byte lines except at a pair's ends: a pair's first vertex lies anywhere.
+// `per` blocks of `sub` triangles share one tile's slot range, so the grid
+// follows the survivors more finely than the sort's tiles.
+//
+// What bounds it: the stores.  1.02 GB of lists (3.4 M triangles of 465 pairs)
+// take 212 us, 4.8 TB/s; a kernel that only stores the same lists takes 190
+// (242 with its runs 48 bytes off the lines).  Three float4 computed per
+// corner and staged in LDS, nine rows a triangle, took 265 us.
+constexpr uint32_t kAsmThreads = 256;
+template <bool kNT, bool kNormals>
+__global__ __launch_bounds__(kAsmThreads) void k_assemble(FrameArgs a, uint32_t blk0, uint32_t sub, uint32_t per) {
+  const uint32_t li = frame_block<true>(a, FC_TILES, per);
   if (li == kNoBlock) return;
-  const uint32_t b = blk0 + li / split;
+  const uint32_t b = blk0 + li / per;
   const uint32_t p = a.tile_part[b];
-  const PartGPU P = a.parts[p];
   const uint32_t S = a.stats[4 * p + 2];
-  const uint32_t sub = a.tile / split;
-  const uint32_t k0 = (b - a.tile_prefix[p]) * a.tile + (li % split) * sub;
-  if (k0 >= S) return;
-  const uint32_t k1 = min(k0 + sub, S), last = k1 - 1;
-  const FrameConst fc = a.fc[P.cam];
-  const uint32_t lane = threadIdx.x;
-  const uint32_t vbase = P.vbase, vmin = P.vmin, tbase = P.tbase;
-  const bool has_uv = (P.flags & PF_HAS_UV) != 0;
-  const bool unbb = (P.flags & PF_UNBB) != 0;
-  const float* __restrict__ vud = a.vud;
-  const float src_w = P.src_w, src_h = P.src_h;
-  const float2* __restrict__ uvp = reinterpret_cast<const float2*>(P.uv);
+  if (S == 0) return;
+  const PartGPU& P = a.parts[p];
+  // read before the first store, which may alias these tables as far as the compiler knows
   const uint64_t out_base = P.out_base;
-  const uint32_t idx_base = P.idx_base;
-  const bool persp = fc.perspective != 0, pc_tex = fc.pc_tex != 0, rdepth = fc.render_depth != 0;
-  const float cam_w = fc.cam_w, half_w = fc.half_w, cam_h = fc.cam_h, half_h = fc.half_h;
-  const float dmp = fc.dmp, spread = fc.spread;
-  const float4* __restrict__ vclip = a.vclip;
-  const float4* __restrict__ vcol = a.vcol;
-  const uint32_t vstride = a.vstride;
-  const uint4* __restrict__ tvo = a.tri_vo + tbase;
-  float4* __restrict__ out_c = a.out_color + out_base * 3;
-  float4* __restrict__ out_d = a.out_depth + out_base * 3;
+  const uint32_t idx_base = P.idx_base, tbase = P.tbase, ntiles = P.ntiles;
+  const FrameConst& fc = a.fc[P.cam];
+  const float da = fc.render_depth ? 1.0f : 0.0f;
+  const bool normals = kNormals && fc.render_normals != 0;
+  const uint32_t j = (b - a.tile_prefix[p]) * per + li % per;       // this block's place among the pair's
+  const uint32_t span = sub * 9;                                    // float4 per block; the last takes the rest
+  const int64_t end = 9 * (int64_t)S;
+  const int64_t first = (int64_t)j * span - (int64_t)(3 * out_base % 64);
+  const int64_t last = j + 1 == ntiles * per ? end : min(first + (int64_t)span, end);
+  const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const uint32_t* __restrict__ tvo = reinterpret_cast<const uint32_t*>(a.tri_vo + tbase);
+  const float4* __restrict__ vab = a.vab;
+  const float4* __restrict__ vq = a.vq;
+  const float4* __restrict__ vnrm = a.vnrm;
+  float4* __restrict__ out_c = a.out_color + 3 * out_base;
+  float4* __restrict__ out_d = a.out_depth + 3 * out_base;
+  float4* __restrict__ out_n = kNormals ? a.out_normal + 3 * out_base : nullptr;
   uint32_t* __restrict__ out_i = a.out_idx + out_base;
-  float4* __restrict__ sink = a.sink + lane;                 // per-lane sink, never read
-  uint32_t* __restrict__ sink_i = reinterpret_cast<uint32_t*>(a.sink + 64) + lane;
-  const float da = rdepth ? 1.0f : 0.0f;
-  __shared__ float4 stage[kRows * 9];
-
-  struct Gathered {
-    float4 c[3], col[3];
-    float2 uv[3];
-    float zd[3];                 // Z the depth list takes: clip Z, or the unbillboarded Z
-  };
-  auto gather = [&](Gathered& g, const uint4 vo) {
-    const uint32_t ov[3] = {vo.x, vo.y, vo.z};
-    for (int vi = 0; vi < 3; vi++) {
-      g.c[vi] = vclip[(size_t)ov[vi] * vstride];
-      g.col[vi] = vcol[(size_t)ov[vi] * vstride];
-      g.uv[vi] = has_uv ? uvp[ov[vi] - vbase + vmin] : make_float2(0.0f, 0.0f);
-      g.zd[vi] = unbb ? vud[ov[vi]] : g.c[vi].z;
-    }
-  };
-  auto compute = [&](const Gathered& g, float4 (&cq)[9], float (&dd)[3]) {
-    for (int vi = 0; vi < 3; vi++) {
-      float w = g.c[vi].w;                                        // camera.go:1655-1667
-      if (!persp) w = 1.0f;
-      if (w < 0) w = 0.001f;
-      const float dx = fdiv(g.c[vi].x, w) * cam_w + half_w;
-      const float dy = fdiv(g.c[vi].y, -w) * cam_h + half_h;
-      const float U = g.uv[vi].x, V = g.uv[vi].y;
-      float uvU, uvV, c0 = 0.0f;
-      if (pc_tex) {                                               // camera.go:1688-1711
-        uvU = fdiv(U, w) * src_w;
-        uvV = fdiv(1.0f - V, w) * src_h;
-        c0 = fdiv(1.0f, w);
-      } else {
-        uvU = U * src_w;
-        uvV = (1.0f - V) * src_h;
-      }
-      float depth = 0.0f;
-      if (rdepth) {                                               // camera.go:1765-1784
-        depth = fdiv(g.zd[vi] + dmp, spread);
-        if (depth < 0) depth = 0;
-        else if (depth > 1) depth = 1;
-      }
-      cq[3 * vi + 0] = make_float4(dx, dy, uvU, uvV);
-      cq[3 * vi + 1] = g.col[vi];
-      cq[3 * vi + 2] = make_float4(c0, 0.0f, 0.0f, 0.0f);
-      dd[vi] = depth;
-    }
-  };
-  auto store_chunk = [&](const float4 (&cq)[9], const float (&dd)[3], uint32_t wk0) {
-    const uint32_t wcount = min(64u, k1 - wk0);
+  constexpr uint32_t kPer = 9, kChunk = 64 * kPer;                  // float4 per lane and per wavefront
+  for (int64_t c0 = first + wave * kChunk; c0 < last; c0 += (kAsmThreads / 64) * kChunk) {   // wave-uniform
+    const int64_t c1 = min(c0 + (int64_t)kChunk, last);
+    const uint32_t tri0 = c0 > 0 ? (uint32_t)(c0 / 9) : 0u;
+    const int32_t rel = (int32_t)(c0 - 9 * (int64_t)tri0);          // the chunk's start from triangle tri0's
+    const int32_t lim = (int32_t)(c1 - 9 * (int64_t)tri0);
+    float4 v[kPer], n[kPer];
+    float d[kPer];
+    uint32_t ov[kPer];
 #pragma unroll
-    for (uint32_t h = 0; h < 64 / kRows; h++) {
-      const uint32_t r0 = h * kRows;
-      const uint32_t rows = wcount > r0 ? min(kRows, wcount - r0) : 0u;
-      const bool mine = lane >= r0 && lane < r0 + kRows;
-      if (mine)
-        for (int q = 0; q < 9; q++) stage[(lane - r0) * 9 + q] = cq[q];
-      __syncthreads();
-#pragma unroll
-      for (uint32_t q = 0; q < (kRows * 9 + 63) / 64; q++) {
-        const uint32_t f = q * 64 + lane;
-        store4<kNT>(f < rows * 9 ? &out_c[(size_t)(wk0 + r0) * 9 + f] : sink, stage[min(f, kRows * 9 - 1)]);
-      }
-      __syncthreads();
-      if (mine)
-        for (int vi = 0; vi < 3; vi++) stage[(lane - r0) * 9 + 3 * vi + 1] = make_float4(dd[vi], dd[vi], dd[vi], da);
-      __syncthreads();
-#pragma unroll
-      for (uint32_t q = 0; q < (kRows * 9 + 63) / 64; q++) {
-        const uint32_t f = q * 64 + lane;
-        store4<kNT>(f < rows * 9 ? &out_d[(size_t)(wk0 + r0) * 9 + f] : sink, stage[min(f, kRows * 9 - 1)]);
-      }
-      __syncthreads();
+    for (uint32_t q = 0; q < kPer; q++) {
+      const uint32_t g = (uint32_t)min(max(rel + (int32_t)(q * 64 + lane), 0), lim - 1);   // an active float4
+      const uint32_t corner = g / 3, tri = corner / 3;
+      ov[q] = tvo[4 * (size_t)(tri0 + tri) + corner - 3 * tri];
     }
 #pragma unroll
-    for (uint32_t q = 0; q < 3; q++) {                            // indices (camera.go:1816)
-      const uint32_t f = q * 64 + lane;
-      store1<kNT>(f < wcount * 3 ? &out_i[(size_t)wk0 * 3 + f] : sink_i, idx_base + wk0 * 3 + f);
+    for (uint32_t q = 0; q < kPer; q++) {
+      const uint32_t g = (uint32_t)min(max(rel + (int32_t)(q * 64 + lane), 0), lim - 1);
+      const uint32_t piece = g % 3;
+      v[q] = *(piece == 2 ? vq + ov[q] : vab + 2 * (size_t)ov[q] + piece);
+      d[q] = 0.0f;
+      if (piece == 1) {
+        d[q] = vq[ov[q]].z;
+        if (normals) n[q] = vnrm[ov[q]];
+      }
     }
-  };
-
-  // two register sets, used in turn: no copies between chunks
-  Gathered ga, gb;
-  gather(ga, tvo[min(k0 + lane, last)]);
-  uint4 vo_next = tvo[min(k0 + 64 + lane, last)];
-  float4 cq[9];
-  float dd[3];
-  for (uint32_t wk0 = k0;;) {
-    compute(ga, cq, dd);
-    bool more = wk0 + 64 < k1;                                    // uniform
-    if (more) {
-      gather(gb, vo_next);
-      vo_next = tvo[min(wk0 + 128 + lane, last)];
+#pragma unroll
+    for (uint32_t q = 0; q < kPer; q++) {
+      const int32_t g = rel + (int32_t)(q * 64 + lane);
+      if (g < 0 || g >= lim) continue;
+      const uint32_t piece = (uint32_t)g % 3;
+      const int64_t f = c0 + q * 64 + lane;
+      const float4 custom = make_float4(v[q].w, 0.0f, 0.0f, 0.0f);
+      store4<kNT>(&out_c[f], piece == 2 ? custom : v[q]);
+      store4<kNT>(&out_d[f], piece == 2 ? custom : piece == 1 ? make_float4(d[q], d[q], d[q], da) : v[q]);
+      if (normals) store4<kNT>(&out_n[f], piece == 0 ? v[q] : piece == 1 ? n[q] : make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     }
-    store_chunk(cq, dd, wk0);
-    wk0 += 64;
-    if (!more) break;
-    compute(gb, cq, dd);
-    more = wk0 + 64 < k1;
-    if (more) {
-      gather(ga, vo_next);
-      vo_next = tvo[min(wk0 + 128 + lane, last)];
-    }
-    store_chunk(cq, dd, wk0);
-    wk0 += 64;
-    if (!more) break;
+    // indices: flush-local iota, as the reference's indexList (camera.go:1816), of the vertices that start here
+    const uint32_t i0 = c0 > 0 ? (uint32_t)((c0 + 2) / 3) : 0u, i1 = (uint32_t)((c1 + 2) / 3);
+    for (uint32_t i = i0 + lane; i < i1; i += 64) store1<kNT>(&out_i[i], idx_base + i);
   }
 }
 
@@ -1551,37 +1424,6 @@ __global__ __launch_bounds__(256) void k_groups(FrameArgs a, uint32_t part0, uin
   }
 }
 
-// Camera.RenderNormals: the normal vertex list (camera.go:1710-1722), after
-// the assembly.  Per drawn triangle in slot order, each corner takes the
-// colour vertex's DstX, DstY, SrcX, SrcY (its first float4, just written)
-// and as colour the vertex's rotated position times 0.5 plus 0.5
-// (k_vertex's vnrm); alpha and the custom fields stay 0.  One 256-thread
-// block per sort tile, one thread per (triangle, corner).
-__global__ __launch_bounds__(256) void k_normals(FrameArgs a, uint32_t blk0) {
-  const uint32_t lb = frame_block(a, FC_TILES, 1);
-  if (lb == kNoBlock) return;
-  const uint32_t b = blk0 + lb;
-  const uint32_t p = a.tile_part[b];
-  const PartGPU P = a.parts[p];
-  if (!a.fc[P.cam].render_normals) return;
-  const uint32_t S = a.stats[4 * p + 2];
-  const uint32_t k0 = (b - a.tile_prefix[p]) * a.tile;
-  if (k0 >= S) return;
-  const uint32_t k1 = min(k0 + a.tile, S);
-  const uint4* __restrict__ tvo = a.tri_vo + P.tbase;
-  const float4* __restrict__ oc = a.out_color + P.out_base * 3;
-  float4* __restrict__ on = a.out_normal + P.out_base * 3;
-  const float4* __restrict__ vn = a.vnrm;
-  for (uint32_t c = 3 * k0 + threadIdx.x; c < 3 * k1; c += blockDim.x) {   // corner c of the pair's list
-    const uint4 vo = tvo[c / 3];
-    const uint32_t vi = c % 3;
-    const uint32_t o = vi == 0 ? vo.x : (vi == 1 ? vo.y : vo.z);
-    on[3 * (size_t)c + 0] = oc[3 * (size_t)c + 0];
-    on[3 * (size_t)c + 1] = vn[o];
-    on[3 * (size_t)c + 2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  }
-}
-
 // Plain float4 copy of a known size: the reference point for HBM byte counters.
 __global__ __launch_bounds__(256) void k_copy(const float4* __restrict__ src, float4* __restrict__ dst, uint64_t n) {
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
@@ -1608,7 +1450,7 @@ hipError_t launch_palettes(const FrameArgs& a, hipStream_t s) {
 }
 hipError_t launch_uniforms(const FrameArgs& a, uint32_t part0, uint32_t nparts, hipStream_t s) {
   if (!nparts) return hipSuccess;
-  hipLaunchKernelGGL(k_uniforms, dim3(nparts), dim3(64), 0, s, a, part0, nparts);
+  hipLaunchKernelGGL(k_uniforms, dim3(nparts), dim3(kUniformThreads), 0, s, a, part0, nparts);
   return hipGetLastError();
 }
 hipError_t launch_vertex(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, hipStream_t s) {
@@ -1651,37 +1493,21 @@ hipError_t launch_scatter(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint
   return hipGetLastError();
 }
 hipError_t launch_assemble(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t mode, uint32_t split,
-                           hipStream_t s) {
+                           uint32_t max_triangles, hipStream_t s) {
   if (!nblk) return hipSuccess;
   if (split == 0 || (split & (split - 1)) || a.tile % split) return hipErrorInvalidValue;
-  if (mode & 64u) {   // bit 6: the assembly's blocks in launch order, whatever the other passes use
-    FrameArgs b = a;
-    b.xcd_swizzle = 0;
-    return launch_assemble(b, blk0, nblk, mode & ~64u, split, s);
-  }
-  const dim3 g(nblk * split), g2(2 * nblk * split);
-  switch (mode) {
-    case 8: hipLaunchKernelGGL((k_assemble_pipe<64, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 10: hipLaunchKernelGGL((k_assemble_pipe<64, true>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 12: hipLaunchKernelGGL((k_assemble_pipe<32, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 14: hipLaunchKernelGGL((k_assemble_pipe<32, true>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 0: hipLaunchKernelGGL((k_assemble<1, false, 1, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 1: hipLaunchKernelGGL((k_assemble<0, false, 1, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 2: hipLaunchKernelGGL((k_assemble<1, true, 1, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 3: hipLaunchKernelGGL((k_assemble<0, true, 1, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 4: hipLaunchKernelGGL((k_assemble<2, false, 1, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    case 6: hipLaunchKernelGGL((k_assemble<2, true, 1, false>), g, dim3(64), 0, s, a, blk0, split); break;
-    // bit 4: four wavefronts per block, each staging its own rows
-    case 16: hipLaunchKernelGGL((k_assemble<1, false, 4, false>), g, dim3(256), 0, s, a, blk0, split); break;
-    case 18: hipLaunchKernelGGL((k_assemble<1, true, 4, false>), g, dim3(256), 0, s, a, blk0, split); break;
-    case 20: hipLaunchKernelGGL((k_assemble<2, false, 4, false>), g, dim3(256), 0, s, a, blk0, split); break;
-    case 22: hipLaunchKernelGGL((k_assemble<2, true, 4, false>), g, dim3(256), 0, s, a, blk0, split); break;
-    // bit 5: one output stream per block (colour vertices and indices, or depth vertices), twice the blocks
-    case 34: hipLaunchKernelGGL((k_assemble<1, true, 1, true>), g2, dim3(64), 0, s, a, blk0, split); break;
-    case 38: hipLaunchKernelGGL((k_assemble<2, true, 1, true>), g2, dim3(64), 0, s, a, blk0, split); break;
-    case 50: hipLaunchKernelGGL((k_assemble<1, true, 4, true>), g2, dim3(256), 0, s, a, blk0, split); break;
-    case 54: hipLaunchKernelGGL((k_assemble<2, true, 4, true>), g2, dim3(256), 0, s, a, blk0, split); break;
-    default: return hipErrorInvalidValue;
+  // pairs of one tile with few triangles need fewer blocks than the tile has room for: 4,096 cubes of 12
+  // triangles took 26 us with eight blocks each, 10 us with one
+  const uint32_t sub = a.tile / split;
+  const uint32_t per = max_triangles < a.tile ? std::max(1u, (max_triangles + sub - 1) / sub) : split;
+  FrameArgs b = a;
+  if (mode & 64u) b.xcd_swizzle = 0;   // bit 6: the assembly's blocks in launch order, whatever the other passes use
+  const dim3 g(nblk * per);
+  switch ((mode & 2u) | (a.out_normal ? 1u : 0u)) {
+    case 0: hipLaunchKernelGGL((k_assemble<false, false>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
+    case 1: hipLaunchKernelGGL((k_assemble<false, true>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
+    case 2: hipLaunchKernelGGL((k_assemble<true, false>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
+    default: hipLaunchKernelGGL((k_assemble<true, true>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
   }
   return hipGetLastError();
 }
@@ -1693,11 +1519,6 @@ hipError_t launch_fill(void* dst, uint64_t bytes, uint32_t word, hipStream_t s) 
 hipError_t launch_pack(const PackArgs& a, uint32_t nblocks, hipStream_t s) {
   if (!nblocks) return hipSuccess;
   hipLaunchKernelGGL(k_pack, dim3(nblocks), dim3(256), 0, s, a);
-  return hipGetLastError();
-}
-hipError_t launch_normals(const FrameArgs& a, uint32_t blk0, uint32_t nblk, hipStream_t s) {
-  if (!nblk) return hipSuccess;
-  hipLaunchKernelGGL(k_normals, dim3(nblk), dim3(256), 0, s, a, blk0);
   return hipGetLastError();
 }
 hipError_t launch_groups(const FrameArgs& a, uint32_t part0, uint32_t part1, hipStream_t s) {

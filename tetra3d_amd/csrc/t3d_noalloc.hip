@@ -4,8 +4,7 @@
 // The frame's tables (per-pair uniforms, lights, block prefixes, palettes)
 // and its scratch (vertex records, depth keys, survivor records, histograms,
 // per-pair stats) come from one file-scope device array of
-// T3D_NOALLOC_SCRATCH_BYTES per GPU, which each GPU holds until the process
-// ends.  The host side reaches it only through the address
+// kNoallocRoom bytes per GPU, which each GPU holds until the process ends.  The host side reaches it only through the address
 // hipGetSymbolAddress returns for the current device: the array's name in
 // host code is a host-side stand-in, not a device address.
 //
@@ -21,7 +20,7 @@
 
 namespace t3d {
 
-static __device__ __align__(256) uint8_t scratch[T3D_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) uint8_t scratch[kNoallocRoom];
 
 namespace {
 
@@ -70,6 +69,7 @@ extern "C" t3d_status t3d_render_noalloc(t3d_ctx* c, t3d_frame* f, const t3d_ren
   Placement pl;
   pl.scratch = reinterpret_cast<uint8_t*>(c->noalloc_scratch);
   pl.scratch_bytes = T3D_NOALLOC_SCRATCH_BYTES;
+  pl.scratch_room = kNoallocRoom;
   pl.color = color_vertices;
   pl.depth = depth_vertices;
   pl.idx = indices;

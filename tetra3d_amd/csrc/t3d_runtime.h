@@ -37,6 +37,7 @@ struct Mesh {
   const uint16_t* idx16 = nullptr; // ... or uint16 when the mesh has at most 65,536 vertices
   const float* ctr = nullptr;      // Triangle.Center per triangle, xyz (mesh.go:1980-1982, kept as AddTriangles does)
   uint32_t V = 0, T = 0, K = 0;
+  uint32_t max_part = 0;           // triangles of its largest part
   std::vector<t3d_part_range> parts;
   std::vector<uint32_t> part_vmin, part_vcount;
   float dmin[3], dmax[3];
@@ -139,6 +140,7 @@ struct t3d_frame {
   const t3d::MaterialGPU* stage_mats = nullptr;
   uint64_t table_bytes = 0;
   uint64_t total_triangles = 0;
+  uint32_t max_triangles = 0;      // of one render pair (with the device stage: of any MeshPart)
   uint32_t nparts = 0;
   uint32_t total_vchunks = 0, total_tiles = 0, total_sblocks = 0;
   std::vector<uint32_t> vchunk_prefix, tile_prefix, sblock_prefix, pscan_prefix;
@@ -192,6 +194,8 @@ t3d_status fail(t3d_ctx* c, t3d_status st, const char* fmt, ...);
 // Device address of `device`'s copy of the no-allocation scratch array (t3d_noalloc.hip); the device must be
 // current.  Looked up once per device.
 hipError_t noalloc_scratch_address(int device, void** out);
+// Its size: a quarter over the limit that frames are counted against.
+constexpr uint64_t kNoallocRoom = T3D_NOALLOC_SCRATCH_BYTES + T3D_NOALLOC_SCRATCH_BYTES / 4;
 t3d_status dev_alloc(t3d_ctx* c, DevBuf& b, uint64_t bytes);
 // Grow `b` to at least `bytes` (contents discarded); the caller holds ctx->mu.
 t3d_status ensure(t3d_ctx* c, DevBuf& b, uint64_t& cap, uint64_t bytes);
@@ -211,7 +215,8 @@ t3d_status validate_desc(t3d_ctx* c, const t3d_render_desc* desc);
 // tables and scratch are carved from `scratch`, its outputs are the caller's.
 struct Placement {
   uint8_t* scratch = nullptr;
-  uint64_t scratch_bytes = 0;
+  uint64_t scratch_bytes = 0;    // what a frame may count (T3D_NOALLOC_SCRATCH_BYTES)
+  uint64_t scratch_room = 0;     // bytes at `scratch`
   t3d_vertex* color = nullptr;
   t3d_vertex* depth = nullptr;
   uint32_t* idx = nullptr;
