@@ -25,7 +25,6 @@
 namespace t3d {
 
 constexpr uint32_t kBins = 512;        // sortingTriangles.go:166-168
-constexpr uint32_t kMaxLights = 64;    // lights of one pair the vertex pass stages in LDS (more are read from HBM)
 constexpr uint32_t kMaxLdsBones = 64;  // bone palettes staged in LDS up to this size
 constexpr uint32_t kScanBlock = 2048;  // elements per scan block (256 threads x 8)
 constexpr uint32_t kMaxTile = 2048;    // triangles per tile (keys of a tile are staged in LDS; below 2^16: tri_loc)

@@ -6,8 +6,9 @@
 // (scalar loads) and no block straddles two parts.
 //
 //   k_vertex    per vertex: shape keys, skinning or MVP transform, snapping,
-//               lighting (lights staged in LDS), vertex colour, fog
-//               (model.go:751-822, camera.go:1610-1644, 1740-1810)
+//               lighting (light constants in scalar registers), vertex
+//               colour, fog, screen and texture position
+//               (model.go:751-822, camera.go:1610-1644, 1655-1711, 1740-1810)
 //   k_cull      per triangle: w clamp, z-range / screen / backface rejects,
 //               depth key, per-part survivor count and min/max depth
 //               (model.go:828-969)
@@ -88,6 +89,22 @@ __device__ __forceinline__ uint32_t frame_block(const FrameArgs& a, uint32_t whi
 // The same for the launches that never swizzle (scan blocks, pairs).
 __device__ __forceinline__ bool past_count(const FrameArgs& a, uint32_t which) {
   return a.counts && blockIdx.x >= a.counts[which];
+}
+
+// A record at an address that is the same for the whole wavefront, read
+// through the scalar cache into scalar registers (the compiler does so by
+// itself only where it can tell that no store of the kernel may reach it).
+template <class T>
+__device__ __forceinline__ T load_uniform(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  using Word = const __attribute__((address_space(4))) uint32_t;
+  Word* w = (Word*)(uintptr_t)p;
+  uint32_t v[sizeof(T) / 4];
+#pragma unroll
+  for (uint32_t i = 0; i < sizeof(T) / 4; i++) v[i] = w[i];
+  T r;
+  __builtin_memcpy(&r, v, sizeof(T));
+  return r;
 }
 
 __device__ __forceinline__ float clampf(float v, float lo, float hi) {   // math32.go:38-45
@@ -280,7 +297,12 @@ __device__ __forceinline__ void place_vertex(const FrameConst& fc, V4 clip, floa
   r.zin = clip.z + 1.0f >= fc.near_ && clip.z < fc.far_;          // model.go:883-886
 }
 
-__global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
+// Its vertices move about 105 bytes each (3.9 M of them: 410 MB in 94 us, 4.4
+// TB/s, where a copy reaches 4.7).  Light constants staged in LDS instead of
+// scalar registers held the occupancy at six wavefronts a SIMD and cost an
+// LDS read per light and field: 112 us; scalar, but with 65 registers (seven
+// wavefronts), 104 us.
+__global__ __launch_bounds__(256, 8) void k_vertex(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_VCHUNKS, 1);
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
@@ -288,8 +310,6 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
   const PartGPU P = a.parts[p];        // by value: read once, before any store
   const uint32_t flags = P.flags;
 
-  __shared__ LightGPU s_light[kMaxLights];
-  __shared__ PartLight s_pl[kMaxLights];
   // bone palette rows in LDS, five float4 per bone (four rows and one of
   // padding): lanes blending different bones then start on different LDS
   // banks instead of two bank groups (a 64-byte stride covers 16 of 32 banks)
@@ -297,12 +317,6 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
   __shared__ float4 s_bone_rows[kMaxLdsBones * kBoneRows];
 
   const uint32_t nl = (flags & PF_LIGHTING) ? P.light_count : 0u;
-  const bool lds_lights = nl <= kMaxLights;   // more lights are read from device memory as the loop needs them
-  if (lds_lights)
-    for (uint32_t i = threadIdx.x; i < nl; i += blockDim.x) {
-      s_pl[i] = a.plights[P.light_base + i];
-      s_light[i] = a.lights[s_pl[i].light];
-    }
   const bool skinned = (flags & PF_SKINNED) != 0;
   const bool lds_bones = skinned && P.bone_count <= kMaxLdsBones;
   if (lds_bones) {
@@ -406,19 +420,12 @@ __global__ __launch_bounds__(256) void k_vertex(FrameArgs a, uint32_t blk0) {
     if (flags & PF_LIGHTING) {
       // vertexLights reset to (0,0,0,1) then every light in order (camera.go:1613-1641)
       float lr = 0, lg = 0, lb = 0;
-      if (lds_lights) {
-        for (uint32_t k = 0; k < nl; k++) {
-          if (!s_pl[k].enabled) continue;
-          light_vertex(s_light[k], s_pl[k], s_light, s_pl, P, flags, vp, vn, lr, lg, lb);
-        }
-      } else {
-        const LightGPU* ls = a.lights + P.light0;
-        const PartLight* pls = a.plights + P.light_base;
-        for (uint32_t k = 0; k < nl; k++) {
-          const PartLight pl = pls[k];
-          if (!pl.enabled) continue;
-          light_vertex(ls[k], pl, ls, pls, P, flags, vp, vn, lr, lg, lb);
-        }
+      const LightGPU* ls = a.lights + P.light0;
+      const PartLight* pls = a.plights + P.light_base;
+      for (uint32_t k = 0; k < nl; k++) {
+        const PartLight pl = load_uniform(pls + k);
+        if (!pl.enabled) continue;
+        light_vertex(load_uniform(ls + k), pl, ls, pls, P, flags, vp, vn, lr, lg, lb);
       }
       cr *= lr;
       cg *= lg;
