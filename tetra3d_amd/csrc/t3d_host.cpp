@@ -238,6 +238,18 @@ uint64_t placed_charge(uint64_t V, uint64_t T) {
          carve_size<float4>(128) + carve_size<float>(V);
 }
 
+// Whether a frame of `pairs` render pairs (or candidates) and T triangles in all is drawn by one workgroup per render
+// pair (k_pair) instead of the chain of passes over all pairs: where no pair is over kPairVertices and kPairTriangles;
+// and up to the larger limits where there are many pairs and their mean is at least half of the largest, so that no
+// workgroup is waited for long.  One sphere of 2,562 vertices: 100 us a frame against the chain's 104; 16 skinned ones
+// 137 against 131; 64 of them 150 against 155; 256 295 against 335.
+bool pairs_fit(const t3d_frame* f, uint64_t pairs, uint64_t T, bool normals, bool groups) {
+  if (normals || groups) return false;
+  const uint64_t v = f->max_vertices, t = f->max_triangles;
+  if (v <= kPairVertices && t <= kPairTriangles) return true;
+  return v <= kPairVerticesMany && t <= kPairTrianglesMany && pairs >= kPairMany && 2 * T >= pairs * t;
+}
+
 // ---------------------------------------------------------------------------
 // camera (camera.go:638-679, 933-983, 1085-1088)
 // ---------------------------------------------------------------------------
@@ -768,6 +780,7 @@ t3d_status t3d_mesh_upload(t3d_ctx* c, const t3d_mesh_desc* d, uint64_t* out_han
     m->max_part = std::max(m->max_part, r.triangle_count);
     m->part_vmin.push_back(lo);
     m->part_vcount.push_back(r.triangle_count ? hi - lo + 1 : 0);
+    m->max_vertices = std::max(m->max_vertices, m->part_vcount.back());
   }
   if (d->bone_indices) {
     m->has_skin = true;
@@ -1074,7 +1087,7 @@ struct ProfScope {
 // batched form).  Block offsets come from the frame's prefix arrays.  The
 // profile charges each kernel its algorithmic bytes: mesh streams read once
 // (k_vertex), triangle indices once (k_cull), outputs (k_assemble, added
-// after the survivor counts are known).
+// after the survivor counts are known); all of them to k_pair where it runs.
 t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t st, bool prof) {
   const FrameArgs& a = f->args;
   struct {
@@ -1110,8 +1123,14 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
     ProfScope ps(c, st, "k_uniforms", 0, prof);
     HIP_TRY(c, launch_uniforms(a, p0, p1 - p0, st));
   }
+  f->ran_pairs = f->small_pairs && p0 == 0 && p1 == f->nparts;
+  if (f->ran_pairs) {
+    ProfScope ps(c, st, "k_pair", tr.vertex + tr.cull + tr.uv, prof);
+    HIP_TRY(c, launch_pairs(a, p1, f->max_vertices, f->max_triangles, st));
+    return T3D_OK;
+  }
   {
-    ProfScope ps(c, st, "k_vertex", tr.vertex, prof);
+    ProfScope ps(c, st, "k_vertex", tr.vertex + tr.uv, prof);
     HIP_TRY(c, launch_vertex(a, vb0, vb1 - vb0, f->vertex_threads, st));
   }
   {
@@ -1136,7 +1155,7 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
     HIP_TRY(c, launch_scatter(a, tb0, tb1 - tb0, c->tuning.scatter_waves, st));
   }
   {
-    ProfScope ps(c, st, "k_assemble", tr.uv, prof);
+    ProfScope ps(c, st, "k_assemble", 0, prof);
     HIP_TRY(c, launch_assemble(a, tb0, tb1 - tb0, c->tuning.store_mode, c->tuning.assemble_split, f->max_triangles, st));
   }
   return T3D_OK;
@@ -1348,7 +1367,7 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   uint64_t pose_bones = 0, pose_roots = 0, npose = 0;
   uint64_t wV = 0, wT = 0, wvch = 0, wtiles = 0, wsb = 0, wps = 0, whist = 0, wpl = 0;
   bool any_normals = false, any_skinned = false;
-  uint32_t max_tri = 0;
+  uint32_t max_tri = 0, max_vert = 0;
   uint64_t last_id = 0;
   Mesh* last = nullptr;
   auto find_mesh = [&](uint64_t id) -> Mesh* {
@@ -1382,6 +1401,7 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
       mesh_worst_case(*m, vchunk, tile);
       const uint32_t np = (uint32_t)m->parts.size();
       max_tri = std::max(max_tri, m->max_part);
+      max_vert = std::max(max_vert, m->max_vertices);
       nm++;
       ncand += np;
       if (md.materials) nmat += np;
@@ -1673,6 +1693,8 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   ms.max_pairs = maxP;
   take_records(sc, a, wV, wT, any_skinned);
   f->max_triangles = max_tri;
+  f->max_vertices = max_vert;
+  f->small_pairs = pairs_fit(f, ncand, wT, any_normals, false);
   a.hist = sc.take<uint32_t>(whist);
   a.bsum = sc.take<uint32_t>(wsb);
   a.tile_count = sc.take<uint32_t>(wtiles);
@@ -2389,8 +2411,12 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   a.sblock_prefix = d_spre;
   a.pscan_prefix = d_ppre;
   take_records(sc, a, sumV, sumT, any_skinned);
-  f->max_triangles = 0;
-  for (const PartGPU& P : f->parts) f->max_triangles = std::max(f->max_triangles, P.tcount);
+  f->max_triangles = f->max_vertices = 0;
+  for (const PartGPU& P : f->parts) {
+    f->max_triangles = std::max(f->max_triangles, P.tcount);
+    f->max_vertices = std::max(f->max_vertices, P.vcount);
+  }
+  f->small_pairs = pairs_fit(f, P_n, sumT, any_normals, ngroups != 0);
   a.stats = sc.take<uint32_t>(4ull * P_n);
   a.hist = sc.take<uint32_t>(sumHist);
   a.bsum = sc.take<uint32_t>(sblocks);
@@ -2461,11 +2487,11 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
     }
   } else if (allow_graph && c->tuning.use_graph && !(profile && c->profiling)) {
     // graph of the whole chain; reused while the launch shape is unchanged
-    std::vector<uint8_t> key(sizeof(FrameArgs) + 10 * sizeof(uint32_t));
-    uint32_t shape[10] = {f->total_vchunks,       f->total_tiles,           f->total_sblocks,
+    std::vector<uint8_t> key(sizeof(FrameArgs) + 12 * sizeof(uint32_t));
+    uint32_t shape[12] = {f->total_vchunks,       f->total_tiles,           f->total_sblocks,
                          f->vertex_threads,      c->tuning.store_mode,     c->tuning.scatter_waves,
                          c->tuning.assemble_split, c->tuning.cull_block,   f->total_pscan,
-                         f->max_triangles};
+                         f->max_triangles,        f->max_vertices,          f->small_pairs ? 1u : 0u};
     std::memcpy(key.data(), &a, sizeof(FrameArgs));
     std::memcpy(key.data() + sizeof(FrameArgs), shape, sizeof shape);
     if (!f->graph_exec || key != f->graph_key) {
@@ -2597,9 +2623,9 @@ void collect_stage(t3d_ctx* c, t3d_frame* f, bool profile) {
     for (uint32_t j = 0; j <= f->stage_jobs; j++) f->job_pair_begin[j] = jp[j];
   if (profile && c->profiling && f->max_pairs) {
     auto w64 = [&](uint32_t lo) { return (uint64_t)cnt[lo] | ((uint64_t)cnt[lo + 1] << 32); };
-    c->prof["k_vertex"].bytes += w64(FC_BYTES_VERTEX_LO);
-    c->prof["k_cull"].bytes += w64(FC_BYTES_CULL_LO);
-    c->prof["k_assemble"].bytes += w64(FC_BYTES_UV_LO);
+    c->prof[f->ran_pairs ? "k_pair" : "k_vertex"].bytes += w64(FC_BYTES_VERTEX_LO);
+    c->prof[f->ran_pairs ? "k_pair" : "k_cull"].bytes += w64(FC_BYTES_CULL_LO);
+    c->prof[f->ran_pairs ? "k_pair" : "k_vertex"].bytes += w64(FC_BYTES_UV_LO);
   }
 }
 
@@ -2624,7 +2650,7 @@ void frame_collect(t3d_ctx* c, t3d_frame* f, bool profile) {
       f->flush[g].survivor_count = n;
     }
   f->total_survivors = total;
-  if (profile && c->profiling) c->prof["k_assemble"].bytes += 300ull * total;   // 3 x (48 B colour + 48 B depth + 4 B index)
+  if (profile && c->profiling) c->prof[f->ran_pairs ? "k_pair" : "k_assemble"].bytes += 300ull * total;   // 3 x (48 B colour + 48 B depth + 4 B index)
 }
 
 // Packing buffer layout: block prefix, source and destination offsets and vertex counts of np pairs, then the

@@ -28,6 +28,9 @@ constexpr uint32_t kBins = 512;        // sortingTriangles.go:166-168
 constexpr uint32_t kMaxLdsBones = 64;  // bone palettes staged in LDS up to this size
 constexpr uint32_t kScanBlock = 2048;  // elements per scan block (256 threads x 8)
 constexpr uint32_t kMaxTile = 2048;    // triangles per tile (keys of a tile are staged in LDS; below 2^16: tri_loc)
+constexpr uint32_t kPairVertices = 1024, kPairTriangles = 2048;  // the largest render pair of a frame k_pair draws ...
+constexpr uint32_t kPairVerticesMany = 2816, kPairTrianglesMany = 5632;  // ... where there are kPairMany of about one size
+constexpr uint32_t kPairMany = 64;
 constexpr uint64_t kTouchVertices = 2400000;  // frames with more vertex records read them ahead of the assembly
 constexpr uint32_t kScanPartMax = 65536;  // histogram matrices up to this size are scanned by one block
 
@@ -401,6 +404,9 @@ hipError_t launch_scatter(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint
 // max_triangles: the largest render pair's (a bound is enough)
 hipError_t launch_assemble(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t mode, uint32_t split,
                            uint32_t max_triangles, hipStream_t s);
+// One workgroup per render pair takes it from its vertices to its lists (frames whose pairs are small, see
+// kPairVertices; no dynamic batches, no normal lists).
+hipError_t launch_pairs(const FrameArgs& a, uint32_t npairs, uint32_t max_vertices, uint32_t max_triangles, hipStream_t s);
 hipError_t launch_pack(const PackArgs& a, uint32_t nblocks, hipStream_t s);
 hipError_t launch_groups(const FrameArgs& a, uint32_t part0, uint32_t part1, hipStream_t s);
 // The model-level stage of a device-built frame (t3d_models.hip): k_models, then k_plist.

@@ -144,106 +144,119 @@ __device__ __forceinline__ const float* volume_cell(const LightGPU& l, V3 p) {
   return i < 0 ? nullptr : l.cells + 4 * i;
 }
 
+// A field of a record: through scalar registers where the whole wavefront
+// reads the same record, else by each lane.  Each is read where it is used:
+// a pair's record, its camera and a light together are more than the 102
+// scalar registers, and held at once a third of the pass's instructions only
+// moved them out of the way and back.
+template <bool kUniform, class T>
+__device__ __forceinline__ T field(const T& r) {
+  if constexpr (kUniform) return load_uniform(&r);
+  else return r;
+}
+
 // VertexLight of an ambient, point or directional light on one vertex
 // (light.go:116-120, 191-258, 332-360), accumulating into rgb in the
-// reference's order.
+// reference's order.  kUniform: l and pl are the same for the whole wavefront.
+template <bool kUniform>
 __device__ __forceinline__ void light_direct(const LightGPU& l, const PartLight& pl, const PartGPU& P, uint32_t flags,
                                              V3 vp, V3 vn, float& r, float& g, float& b) {
   const uint32_t lmode = (flags >> PF_LMODE_SHIFT) & 3u;
-  if (l.type == T3D_LIGHT_AMBIENT) {
-    r += l.amb[0];
-    g += l.amb[1];
-    b += l.amb[2];
-  } else if (l.type == T3D_LIGHT_POINT) {
-    V3 wp = v3(pl.v[0], pl.v[1], pl.v[2]);
+  const int32_t type = field<kUniform>(l.type);
+  float df;
+  if (type == T3D_LIGHT_AMBIENT) {
+    r += field<kUniform>(l.amb[0]);
+    g += field<kUniform>(l.amb[1]);
+    b += field<kUniform>(l.amb[2]);
+    return;
+  } else if (type == T3D_LIGHT_POINT) {
+    const float range_sq = field<kUniform>(l.range_sq);
+    V3 wp = v3(field<kUniform>(pl.v[0]), field<kUniform>(pl.v[1]), field<kUniform>(pl.v[2]));
     float distance = dist_sq(wp, vp);
-    if (l.range > 0) {
-      if (distance > l.range_sq) return;
+    if (field<kUniform>(l.range) > 0) {
+      if (distance > range_sq) return;
     } else {
-      if (fdiv(1.0f, distance) * l.energy < 0.001f) return;
+      if (fdiv(1.0f, distance) * field<kUniform>(l.energy) < 0.001f) return;
     }
     V3 lv = unit(sub(wp, vp));
     V3 n = lmode == T3D_LIGHTING_FIXED_NORMALS ? lv : vn;
     float diffuse = dot(n, lv);
     if (lmode == T3D_LIGHTING_DOUBLE_SIDED) diffuse = fabsf(diffuse);
-    if (diffuse > 0) {
-      float df = diffuse * fdiv(1.0f, 1.0f + (0.1f * distance)) * 2.0f;
-      if (l.range_sq > 0) {
-        float dc = clampf(fdiv(l.range_sq - distance, distance), 0.0f, 1.0f);
-        df *= dc;
-      }
-      r += l.color[0] * df * l.energy;
-      g += l.color[1] * df * l.energy;
-      b += l.color[2] * df * l.energy;
+    if (!(diffuse > 0)) return;
+    df = diffuse * fdiv(1.0f, 1.0f + (0.1f * distance)) * 2.0f;
+    if (range_sq > 0) {
+      float dc = clampf(fdiv(range_sq - distance, distance), 0.0f, 1.0f);
+      df *= dc;
     }
-  } else if (l.type == T3D_LIGHT_DIRECTIONAL) {
-    V3 fwd = v3(l.fwd[0], l.fwd[1], l.fwd[2]);
+  } else if (type == T3D_LIGHT_DIRECTIONAL) {
+    V3 fwd = v3(field<kUniform>(l.fwd[0]), field<kUniform>(l.fwd[1]), field<kUniform>(l.fwd[2]));
     V3 n;
     if (lmode == T3D_LIGHTING_FIXED_NORMALS) n = fwd;
     else if (flags & PF_SKINNED) n = vn;
-    else n = mult_vec(P.rd, vn);
-    float df = dot(n, fwd);
+    else n = mult_vec(load_uniform(&P.rd), vn);
+    df = dot(n, fwd);
     if (lmode == T3D_LIGHTING_DOUBLE_SIDED) df = fabsf(df);
     if (df <= 0) return;
-    r += l.color[0] * df * l.energy;
-    g += l.color[1] * df * l.energy;
-    b += l.color[2] * df * l.energy;
+  } else {
+    return;
   }
+  const float energy = field<kUniform>(l.energy);
+  r += field<kUniform>(l.color[0]) * df * energy;
+  g += field<kUniform>(l.color[1]) * df * energy;
+  b += field<kUniform>(l.color[2]) * df * energy;
 }
 
-// One light of a pair's list on one vertex: light_direct, or a LightVolume
-// (light.go:583-663), whose cell first runs the lights its useLights names
-// (light.go:650-653; entries ls/pls[nest_off + j] of the same list) and then
-// adds its own colour.
-__device__ __forceinline__ void light_vertex(const LightGPU& l, const PartLight& pl, const LightGPU* ls,
+// A LightVolume of a pair's list on one vertex (light.go:583-663): its cell
+// first runs the lights its useLights names (light.go:650-653; entries
+// ls/pls[nest_off + j] of the same list), then adds its own colour.
+__device__ __forceinline__ void light_volume(const LightGPU& lr, const PartLight& pl, const LightGPU* ls,
                                              const PartLight* pls, const PartGPU& P, uint32_t flags, V3 vp, V3 vn,
                                              float& r, float& g, float& b) {
-  if (l.type != T3D_LIGHT_VOLUME) {
-    light_direct(l, pl, P, flags, vp, vn, r, g, b);
+  const uint32_t mode = (flags >> PF_LVMODE_SHIFT) & 3u;
+  if (mode == T3D_LV_OFF) return;                                  // LightVolume.Light, light.go:671-673
+  float c0 = 0, c1 = 0, c2 = 0;
+  if (mode == T3D_LV_PER_OBJECT) {
+    if (load_uniform(&pl.cell_found)) {
+      c0 = load_uniform(&pl.v[0]);
+      c1 = load_uniform(&pl.v[1]);
+      c2 = load_uniform(&pl.v[2]);
+    }
   } else {
-    const uint32_t mode = (flags >> PF_LVMODE_SHIFT) & 3u;
-    if (mode == T3D_LV_OFF) return;                                // LightVolume.Light, light.go:671-673
-    float c0 = 0, c1 = 0, c2 = 0;
-    if (mode == T3D_LV_PER_OBJECT) {
-      if (pl.cell_found) {
-        c0 = pl.v[0];
-        c1 = pl.v[1];
-        c2 = pl.v[2];
-      }
+    const LightGPU l = load_uniform(&lr);
+    V3 halfc = v3(fdiv(l.cell[0], 2.0f), fdiv(l.cell[1], 2.0f), fdiv(l.cell[2], 2.0f));
+    V3 bias = v3(l.bias[0], l.bias[1], l.bias[2]);
+    V3 vpos = v3(0, 0, 0), vpn = v3(0, 0, 0);
+    if (flags & PF_SKINNED) {
+      if (mode == T3D_LV_PER_VERTEX_WITH_NORMAL) vpn = add(add(vpos, hmul(vn, halfc)), bias);
+      else vpos = add(vp, bias);
     } else {
-      V3 halfc = v3(fdiv(l.cell[0], 2.0f), fdiv(l.cell[1], 2.0f), fdiv(l.cell[2], 2.0f));
-      V3 bias = v3(l.bias[0], l.bias[1], l.bias[2]);
-      V3 vpos = v3(0, 0, 0), vpn = v3(0, 0, 0);
-      if (flags & PF_SKINNED) {
-        if (mode == T3D_LV_PER_VERTEX_WITH_NORMAL) vpn = add(add(vpos, hmul(vn, halfc)), bias);
-        else vpos = add(vp, bias);
-      } else {
-        if (mode == T3D_LV_PER_VERTEX_WITH_NORMAL) vpn = add(mult_vec(P.model, add(vp, hmul(vn, halfc))), bias);
-        else vpos = add(mult_vec(P.model, vp), bias);
-      }
-      if (!(vpos.x >= l.vmin[0] && vpos.y >= l.vmin[1] && vpos.z >= l.vmin[2] && vpos.x <= l.vmax[0] &&
-            vpos.y <= l.vmax[1] && vpos.z <= l.vmax[2]))
-        return;                                                      // Dimensions.Contains, mesh.go:80-82
-      const int64_t ci = volume_cell_index(l, mode == T3D_LV_PER_VERTEX_WITH_NORMAL ? vpn : vpos);
-      if (ci >= 0) {
-        const float* cell = l.cells + 4 * ci;
-        c0 = cell[0];
-        c1 = cell[1];
-        c2 = cell[2];
-        if (l.cell_lights) {
-          const uint32_t j1 = l.cell_lights[ci + 1];
-          const uint32_t* ix = l.cell_lights + l.ncells + 1;
-          for (uint32_t j = l.cell_lights[ci]; j < j1; j++) {
-            const uint32_t li = l.nest_off + ix[j];
-            light_direct(ls[li], pls[li], P, flags, vp, vn, r, g, b);
-          }
+      const M4 model = load_uniform(&P.model);
+      if (mode == T3D_LV_PER_VERTEX_WITH_NORMAL) vpn = add(mult_vec(model, add(vp, hmul(vn, halfc))), bias);
+      else vpos = add(mult_vec(model, vp), bias);
+    }
+    if (!(vpos.x >= l.vmin[0] && vpos.y >= l.vmin[1] && vpos.z >= l.vmin[2] && vpos.x <= l.vmax[0] &&
+          vpos.y <= l.vmax[1] && vpos.z <= l.vmax[2]))
+      return;                                                        // Dimensions.Contains, mesh.go:80-82
+    const int64_t ci = volume_cell_index(l, mode == T3D_LV_PER_VERTEX_WITH_NORMAL ? vpn : vpos);
+    if (ci >= 0) {
+      const float* cell = l.cells + 4 * ci;
+      c0 = cell[0];
+      c1 = cell[1];
+      c2 = cell[2];
+      if (l.cell_lights) {
+        const uint32_t j1 = l.cell_lights[ci + 1];
+        const uint32_t* ix = l.cell_lights + l.ncells + 1;
+        for (uint32_t j = l.cell_lights[ci]; j < j1; j++) {
+          const uint32_t li = l.nest_off + ix[j];
+          light_direct<false>(ls[li], pls[li], P, flags, vp, vn, r, g, b);
         }
       }
     }
-    r += l.color[0] * c0 * l.energy;
-    g += l.color[1] * c1 * l.energy;
-    b += l.color[2] * c2 * l.energy;
   }
+  const float energy = load_uniform(&lr.energy);
+  r += load_uniform(&lr.color[0]) * c0 * energy;
+  g += load_uniform(&lr.color[1]) * c1 * energy;
+  b += load_uniform(&lr.color[2]) * c2 * energy;
 }
 
 // ---------------------------------------------------------------------------
@@ -266,7 +279,7 @@ struct VertexRecord {
 // their quotients are one: y / -w is -(y / w) in every rounding.
 __device__ __forceinline__ void place_vertex(const FrameConst& fc, V4 clip, float zd, float2 uv, float src_w,
                                              float src_h, VertexRecord& r) {
-  const bool persp = fc.perspective != 0;
+  const bool persp = load_uniform(&fc.perspective) != 0;
   const float wc = clip.w < 0 ? 0.000001f : clip.w;
   const float nx = fdiv(clip.x, wc), ny = fdiv(clip.y, wc);
   float w = clip.w;                                               // camera.go:1655-1667
@@ -278,7 +291,7 @@ __device__ __forceinline__ void place_vertex(const FrameConst& fc, V4 clip, floa
     qy = fdiv(clip.y, -w);
   }
   float uvU, uvV, c0 = 0.0f;
-  if (fc.pc_tex) {                                                // camera.go:1688-1711
+  if (load_uniform(&fc.pc_tex)) {                                                // camera.go:1688-1711
     uvU = fdiv(uv.x, w) * src_w;
     uvV = fdiv(1.0f - uv.y, w) * src_h;
     c0 = fdiv(1.0f, w);
@@ -287,14 +300,153 @@ __device__ __forceinline__ void place_vertex(const FrameConst& fc, V4 clip, floa
     uvV = (1.0f - uv.y) * src_h;
   }
   float depth = 0.0f;
-  if (fc.render_depth) {                                          // camera.go:1765-1784
-    depth = fdiv(zd + fc.dmp, fc.spread);
+  if (load_uniform(&fc.render_depth)) {                                          // camera.go:1765-1784
+    depth = fdiv(zd + load_uniform(&fc.dmp), load_uniform(&fc.spread));
     if (depth < 0) depth = 0;
     else if (depth > 1) depth = 1;
   }
-  r.a = make_float4(qx * fc.cam_w + fc.half_w, qy * fc.cam_h + fc.half_h, uvU, uvV);
+  r.a = make_float4(qx * load_uniform(&fc.cam_w) + load_uniform(&fc.half_w), qy * load_uniform(&fc.cam_h) + load_uniform(&fc.half_h), uvU, uvV);
   r.q = make_float4(nx, ny, depth, c0);
-  r.zin = clip.z + 1.0f >= fc.near_ && clip.z < fc.far_;          // model.go:883-886
+  r.zin = clip.z + 1.0f >= load_uniform(&fc.near_) && clip.z < load_uniform(&fc.far_);          // model.go:883-886
+}
+
+// bone palette rows in LDS, five float4 per bone (four rows and one of
+// padding): lanes blending different bones then start on different LDS
+// banks instead of two bank groups (a 64-byte stride covers 16 of 32 banks)
+constexpr uint32_t kBoneRows = 5;
+__device__ __forceinline__ void stage_bones(const PartGPU& P, float4* rows) {
+  const float4* src = reinterpret_cast<const float4*>(load_uniform(&P.palette));
+  const uint32_t n = 4u * load_uniform(&P.bone_count);
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) rows[(i / 4) * kBoneRows + i % 4] = src[i];
+}
+
+// One vertex of a pair through shape keys, skinning or MVP transform,
+// snapping, colour, lighting and fog.  rows: the pair's bone rows in LDS, or
+// null (then read from memory); umvp: the unaltered MVP (PF_UNBB pairs).
+__device__ __forceinline__ VertexRecord shade_vertex(const FrameArgs& a, const FrameConst& fc, const PartGPU& P,
+                                                     uint32_t flags, uint32_t v, const float4* rows, const M4& umvp,
+                                                     V3& vp) {
+  const bool skinned = (flags & PF_SKINNED) != 0;
+  const uint32_t nl = (flags & PF_LIGHTING) ? load_uniform(&P.light_count) : 0u;
+  // VertexPositionWithShapeKeys / VertexNormalWithShapeKeys (mesh.go:796-822)
+  V3 pos = ld3(load_uniform(&P.pos), v);
+  V3 nrm = ld3(load_uniform(&P.nrm), v);
+  if (flags & PF_SHAPE_KEYS) {
+    for (uint32_t k = 0; k < load_uniform(&P.shape_keys); k++) {
+      const float w = load_uniform(&P.sk_w)[k];
+      const size_t o = ((size_t)k * load_uniform(&P.mesh_vcount) + v) * 3;
+      pos.x += load_uniform(&P.sk_pos)[o + 0] * w;
+      pos.y += load_uniform(&P.sk_pos)[o + 1] * w;
+      pos.z += load_uniform(&P.sk_pos)[o + 2] * w;
+    }
+    for (uint32_t k = 0; k < load_uniform(&P.shape_keys); k++) {
+      const float w = load_uniform(&P.sk_w)[k];
+      const size_t o = ((size_t)k * load_uniform(&P.mesh_vcount) + v) * 3;
+      nrm.x += load_uniform(&P.sk_nrm)[o + 0] * w;
+      nrm.y += load_uniform(&P.sk_nrm)[o + 1] * w;
+      nrm.z += load_uniform(&P.sk_nrm)[o + 2] * w;
+    }
+  }
+  V3 vn;
+  V4 clip;
+  float zu = 0.0f;                                                // Z of DepthModeUnbillboarded
+  if (skinned) {
+    // Model.skinVertex (model.go:559-596)
+    const ushort4 bi = reinterpret_cast<const ushort4*>(load_uniform(&P.bones))[v];
+    const float4 bw = reinterpret_cast<const float4*>(load_uniform(&P.weights))[v];
+    const uint16_t bidx[4] = {bi.x, bi.y, bi.z, bi.w};
+    const float bwt[4] = {bw.x, bw.y, bw.z, bw.w};
+    M4 S = zero4();
+    for (int k = 0; k < 4; k++) {
+      const float w = bwt[k];
+      if (w == 0) continue;
+      float4 B[4];
+      for (int r = 0; r < 4; r++)
+        B[r] = rows ? rows[bidx[k] * kBoneRows + r]
+                         : reinterpret_cast<const float4*>(load_uniform(&P.palette))[(size_t)bidx[k] * 4 + r];
+      if (w == 1) {
+        for (int r = 0; r < 4; r++) {
+          S.m[r][0] = B[r].x;
+          S.m[r][1] = B[r].y;
+          S.m[r][2] = B[r].z;
+          S.m[r][3] = B[r].w;
+        }
+        break;
+      }
+      for (int r = 0; r < 4; r++) {
+        S.m[r][0] += B[r].x * w;
+        S.m[r][1] += B[r].y * w;
+        S.m[r][2] += B[r].z * w;
+        S.m[r][3] += B[r].w * w;
+      }
+    }
+    vp = mult_vec(S, pos);
+    S.m[3][0] = 0;
+    S.m[3][1] = 0;
+    S.m[3][2] = 0;
+    S.m[3][3] = 1;
+    vn = mult_vec(S, nrm);
+    clip = mult_vec_w(load_uniform(&fc.vp), vp);                                 // model.go:772-775
+  } else {
+    vp = pos;
+    vn = nrm;
+    clip = mult_vec_w(load_uniform(&P.mvp), pos);                                // model.go:795-798
+    if (flags & PF_UNBB) zu = mult_vec_w(umvp, pos).z;          // model.go:800-803, not snapped
+  }
+  const float snap = load_uniform(&fc.snap);
+  if (snap > 0) {                                                 // model.go:807-812
+    clip.x = fdiv(roundf(clip.x * snap), snap);
+    clip.y = fdiv(roundf(clip.y * snap), snap);
+    clip.z = fdiv(roundf(clip.z * snap), snap);
+  }
+  // vertex colour (camera.go:1750-1768)
+  float cr, cg, cb, ca;
+  if (flags & PF_HAS_COLOR) {
+    const float4 vc = reinterpret_cast<const float4*>(load_uniform(&P.col))[v];
+    cr = vc.x * load_uniform(&P.mp[0]);
+    cg = vc.y * load_uniform(&P.mp[1]);
+    cb = vc.z * load_uniform(&P.mp[2]);
+    ca = vc.w * load_uniform(&P.mp[3]);
+  } else {
+    cr = load_uniform(&P.mp[0]);
+    cg = load_uniform(&P.mp[1]);
+    cb = load_uniform(&P.mp[2]);
+    ca = load_uniform(&P.mp[3]);
+  }
+  if (flags & PF_LIGHTING) {
+    // vertexLights reset to (0,0,0,1) then every light in order (camera.go:1613-1641)
+    float lr = 0, lg = 0, lb = 0;
+    const LightGPU* ls = a.lights + load_uniform(&P.light0);
+    const PartLight* pls = a.plights + load_uniform(&P.light_base);
+    for (uint32_t k = 0; k < nl; k++) {
+      if (!load_uniform(&pls[k].enabled)) continue;
+      if (load_uniform(&ls[k].type) == T3D_LIGHT_VOLUME) light_volume(ls[k], pls[k], ls, pls, P, flags, vp, vn, lr, lg, lb);
+      else light_direct<true>(ls[k], pls[k], P, flags, vp, vn, lr, lg, lb);
+    }
+    cr *= lr;
+    cg *= lg;
+    cb *= lb;
+  }
+  if (load_uniform(&fc.fog_active)) {                                            // camera.go:1786-1810
+    float depth = fdiv(clip.z + load_uniform(&fc.dmp), load_uniform(&fc.spread));
+    if (depth < 0) depth = 0;
+    else if (depth > 1) depth = 1;
+    depth = load_uniform(&fc.fog_range[0]) + ((load_uniform(&fc.fog_range[1]) - load_uniform(&fc.fog_range[0])) * 1.0f - depth);
+    if (load_uniform(&fc.fog_mode) == T3D_FOG_ADD) {
+      cr += load_uniform(&fc.fog_color[0]) * depth;
+      cg += load_uniform(&fc.fog_color[1]) * depth;
+      cb += load_uniform(&fc.fog_color[2]) * depth;
+    } else if (load_uniform(&fc.fog_mode) == T3D_FOG_SUB) {
+      cr *= load_uniform(&fc.fog_color[0]) * depth;
+      cg *= load_uniform(&fc.fog_color[1]) * depth;
+      cb *= load_uniform(&fc.fog_color[2]) * depth;
+    }
+  }
+  const float2 uv = (flags & PF_HAS_UV) ? reinterpret_cast<const float2*>(load_uniform(&P.uv))[v] : make_float2(0.0f, 0.0f);
+  VertexRecord r;
+  place_vertex(fc, clip, (flags & PF_UNBB) ? zu : clip.z, uv, load_uniform(&P.src_w), load_uniform(&P.src_h), r);
+  r.b = make_float4(cr, cg, cb, ca);
+  return r;
 }
 
 // Its vertices move about 105 bytes each (3.9 M of them: 410 MB in 94 us, 4.4
@@ -307,155 +459,33 @@ __global__ __launch_bounds__(256, 8) void k_vertex(FrameArgs a, uint32_t blk0) {
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
   const uint32_t p = a.vchunk_part[b];
-  const PartGPU P = a.parts[p];        // by value: read once, before any store
-  const uint32_t flags = P.flags;
+  const PartGPU& P = a.parts[p];
+  const uint32_t flags = load_uniform(&P.flags);
 
-  // bone palette rows in LDS, five float4 per bone (four rows and one of
-  // padding): lanes blending different bones then start on different LDS
-  // banks instead of two bank groups (a 64-byte stride covers 16 of 32 banks)
-  constexpr uint32_t kBoneRows = 5;
   __shared__ float4 s_bone_rows[kMaxLdsBones * kBoneRows];
-
-  const uint32_t nl = (flags & PF_LIGHTING) ? P.light_count : 0u;
   const bool skinned = (flags & PF_SKINNED) != 0;
-  const bool lds_bones = skinned && P.bone_count <= kMaxLdsBones;
-  if (lds_bones) {
-    const float4* src = reinterpret_cast<const float4*>(P.palette);
-    for (uint32_t i = threadIdx.x; i < 4u * P.bone_count; i += blockDim.x) s_bone_rows[(i / 4) * kBoneRows + i % 4] = src[i];
-  }
+  const bool lds_bones = skinned && load_uniform(&P.bone_count) <= kMaxLdsBones;
+  if (lds_bones) stage_bones(P, s_bone_rows);
   __shared__ M4 s_umvp;                  // unaltered MVP of DepthModeUnbillboarded (model.go:697-703)
-  if ((flags & PF_UNBB) && threadIdx.x == 0) s_umvp = mult(P.model, a.fc[P.cam].vp);
+  if ((flags & PF_UNBB) && threadIdx.x == 0) s_umvp = mult(load_uniform(&P.model), load_uniform(&a.fc[load_uniform(&P.cam)].vp));
   __syncthreads();
 
-  const FrameConst fc = a.fc[P.cam];
+  const FrameConst& fc = a.fc[load_uniform(&P.cam)];
+  const uint32_t vbase = load_uniform(&P.vbase), vmin = load_uniform(&P.vmin);
+  const bool normals = load_uniform(&fc.render_normals) != 0;
   const uint32_t first = (b - a.vchunk_prefix[p]) * a.vchunk;
-  const uint32_t last = min(first + a.vchunk, P.vcount);
+  const uint32_t last = min(first + a.vchunk, load_uniform(&P.vcount));
   bool out_of_range = false;
   for (uint32_t i = first + threadIdx.x; i < last; i += blockDim.x) {
-    const uint32_t v = P.vmin + i;
-    // VertexPositionWithShapeKeys / VertexNormalWithShapeKeys (mesh.go:796-822)
-    V3 pos = ld3(P.pos, v);
-    V3 nrm = ld3(P.nrm, v);
-    if (flags & PF_SHAPE_KEYS) {
-      for (uint32_t k = 0; k < P.shape_keys; k++) {
-        const float w = P.sk_w[k];
-        const size_t o = ((size_t)k * P.mesh_vcount + v) * 3;
-        pos.x += P.sk_pos[o + 0] * w;
-        pos.y += P.sk_pos[o + 1] * w;
-        pos.z += P.sk_pos[o + 2] * w;
-      }
-      for (uint32_t k = 0; k < P.shape_keys; k++) {
-        const float w = P.sk_w[k];
-        const size_t o = ((size_t)k * P.mesh_vcount + v) * 3;
-        nrm.x += P.sk_nrm[o + 0] * w;
-        nrm.y += P.sk_nrm[o + 1] * w;
-        nrm.z += P.sk_nrm[o + 2] * w;
-      }
-    }
-    V3 vp, vn;
-    V4 clip;
-    float zu = 0.0f;                                                // Z of DepthModeUnbillboarded
-    if (skinned) {
-      // Model.skinVertex (model.go:559-596)
-      const ushort4 bi = reinterpret_cast<const ushort4*>(P.bones)[v];
-      const float4 bw = reinterpret_cast<const float4*>(P.weights)[v];
-      const uint16_t bidx[4] = {bi.x, bi.y, bi.z, bi.w};
-      const float bwt[4] = {bw.x, bw.y, bw.z, bw.w};
-      M4 S = zero4();
-      for (int k = 0; k < 4; k++) {
-        const float w = bwt[k];
-        if (w == 0) continue;
-        float4 B[4];
-        for (int r = 0; r < 4; r++)
-          B[r] = lds_bones ? s_bone_rows[bidx[k] * kBoneRows + r]
-                           : reinterpret_cast<const float4*>(P.palette)[(size_t)bidx[k] * 4 + r];
-        if (w == 1) {
-          for (int r = 0; r < 4; r++) {
-            S.m[r][0] = B[r].x;
-            S.m[r][1] = B[r].y;
-            S.m[r][2] = B[r].z;
-            S.m[r][3] = B[r].w;
-          }
-          break;
-        }
-        for (int r = 0; r < 4; r++) {
-          S.m[r][0] += B[r].x * w;
-          S.m[r][1] += B[r].y * w;
-          S.m[r][2] += B[r].z * w;
-          S.m[r][3] += B[r].w * w;
-        }
-      }
-      vp = mult_vec(S, pos);
-      S.m[3][0] = 0;
-      S.m[3][1] = 0;
-      S.m[3][2] = 0;
-      S.m[3][3] = 1;
-      vn = mult_vec(S, nrm);
-      clip = mult_vec_w(fc.vp, vp);                                 // model.go:772-775
-    } else {
-      vp = pos;
-      vn = nrm;
-      clip = mult_vec_w(P.mvp, pos);                                // model.go:795-798
-      if (flags & PF_UNBB) zu = mult_vec_w(s_umvp, pos).z;          // model.go:800-803, not snapped
-    }
-    if (fc.snap > 0) {                                              // model.go:807-812
-      clip.x = fdiv(roundf(clip.x * fc.snap), fc.snap);
-      clip.y = fdiv(roundf(clip.y * fc.snap), fc.snap);
-      clip.z = fdiv(roundf(clip.z * fc.snap), fc.snap);
-    }
-    // vertex colour (camera.go:1750-1768)
-    float cr, cg, cb, ca;
-    if (flags & PF_HAS_COLOR) {
-      const float4 vc = reinterpret_cast<const float4*>(P.col)[v];
-      cr = vc.x * P.mp[0];
-      cg = vc.y * P.mp[1];
-      cb = vc.z * P.mp[2];
-      ca = vc.w * P.mp[3];
-    } else {
-      cr = P.mp[0];
-      cg = P.mp[1];
-      cb = P.mp[2];
-      ca = P.mp[3];
-    }
-    if (flags & PF_LIGHTING) {
-      // vertexLights reset to (0,0,0,1) then every light in order (camera.go:1613-1641)
-      float lr = 0, lg = 0, lb = 0;
-      const LightGPU* ls = a.lights + P.light0;
-      const PartLight* pls = a.plights + P.light_base;
-      for (uint32_t k = 0; k < nl; k++) {
-        const PartLight pl = load_uniform(pls + k);
-        if (!pl.enabled) continue;
-        light_vertex(load_uniform(ls + k), pl, ls, pls, P, flags, vp, vn, lr, lg, lb);
-      }
-      cr *= lr;
-      cg *= lg;
-      cb *= lb;
-    }
-    if (fc.fog_active) {                                            // camera.go:1786-1810
-      float depth = fdiv(clip.z + fc.dmp, fc.spread);
-      if (depth < 0) depth = 0;
-      else if (depth > 1) depth = 1;
-      depth = fc.fog_range[0] + ((fc.fog_range[1] - fc.fog_range[0]) * 1.0f - depth);
-      if (fc.fog_mode == T3D_FOG_ADD) {
-        cr += fc.fog_color[0] * depth;
-        cg += fc.fog_color[1] * depth;
-        cb += fc.fog_color[2] * depth;
-      } else if (fc.fog_mode == T3D_FOG_SUB) {
-        cr *= fc.fog_color[0] * depth;
-        cg *= fc.fog_color[1] * depth;
-        cb *= fc.fog_color[2] * depth;
-      }
-    }
-    const uint32_t o = P.vbase + i;
-    if (fc.render_normals) {   // model.go:814-818: the rotation applied to the position; colour camera.go:1718-1720
-      const V3 tn = mult_vec(P.nrot, vp);
+    const uint32_t o = vbase + i;
+    V3 vp;
+    const VertexRecord r = shade_vertex(a, fc, P, flags, vmin + i, lds_bones ? s_bone_rows : nullptr, s_umvp, vp);
+    if (normals) {   // model.go:814-818: the rotation applied to the position; colour camera.go:1718-1720
+      const V3 tn = mult_vec(load_uniform(&P.nrot), vp);
       a.vnrm[o] = make_float4(tn.x * 0.5f + 0.5f, tn.y * 0.5f + 0.5f, tn.z * 0.5f + 0.5f, 0.0f);
     }
-    const float2 uv = (flags & PF_HAS_UV) ? reinterpret_cast<const float2*>(P.uv)[v] : make_float2(0.0f, 0.0f);
-    VertexRecord r;
-    place_vertex(fc, clip, (flags & PF_UNBB) ? zu : clip.z, uv, P.src_w, P.src_h, r);
     a.vab[2 * (size_t)o + 0] = r.a;
-    a.vab[2 * (size_t)o + 1] = make_float4(cr, cg, cb, ca);
+    a.vab[2 * (size_t)o + 1] = r.b;
     a.vq[o] = r.q;
     a.vz[o] = r.zin ? 1 : 0;
     out_of_range |= !r.zin;
@@ -1361,6 +1391,244 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(FrameArgs a, uint32_t 
   }
 }
 
+// ---------------------------------------------------------------------------
+// k_pair
+// ---------------------------------------------------------------------------
+
+// The chain from the vertices to the lists for frames of small meshes: one
+// workgroup takes a whole render pair through k_vertex, k_cull, the sort and
+// k_assemble, with the cull's screen positions, the keys, the histogram and
+// the draw order in LDS and barriers where the chain has launches.  Each step
+// is the chain's own (same functions, same order), so the lists are the same
+// bit for bit.  Only the colour half of the vertex records and the skinned
+// positions go through memory (the workgroup's own, read back by the same
+// CU); tri_vo is written for t3d_frame_download_triangles.
+//
+// kThreads, kV and kT: threads, and the most vertices and triangles a pair may
+// have (launch_pairs chooses).  LDS per block: 17 B a vertex, 8 B a triangle
+// and 1 KB a wavefront; 112 KB at the largest.
+//
+// What bounds it: instructions and latency while a workgroup shades (10 us a
+// round of 1,024 skinned vertices under six lights; 7 us before the first, of
+// cold loads), then the stores of the lists.  642 vertices alone: 19 us, where
+// the chain's six launches take 44; 4,096 cubes 16 us against 52; 256 skinned
+// characters of 2,562 vertices 83 us against 125.  Where one pair is much
+// larger than the others its workgroup is what the frame waits for (200
+// uneven models of up to 4,000 vertices: 151 us a frame against 141 with the
+// chain), so larger pairs come here only in even company (pairs_fit).
+template <uint32_t kThreads, uint32_t kV, uint32_t kT>
+__global__ __launch_bounds__(kThreads) void k_pair(FrameArgs a) {
+  if (past_count(a, FC_PAIRS)) return;
+  const uint32_t p = blockIdx.x;
+  const PartGPU& R = a.parts[p];
+  const uint32_t flags = load_uniform(&R.flags), vcount = load_uniform(&R.vcount), tcount = load_uniform(&R.tcount);
+  const uint32_t vbase = load_uniform(&R.vbase), vmin = load_uniform(&R.vmin);
+  if (tcount == 0 || tcount > kT || vcount > kV) return;   // k_uniforms has set its count to 0
+  const FrameConst& fc = a.fc[load_uniform(&R.cam)];
+  constexpr uint32_t kWaves = kThreads / 64;
+  static_assert(kT % 64 == 0 && kT <= 65536 && kV <= 65536, "16-bit places");
+  __shared__ float4 s_q[kV];
+  __shared__ uint8_t s_z[kV];
+  __shared__ uint32_t s_u[kT * 6 / 4];            // keys and triangles of the survivors; then their corners in draw order
+  __shared__ uint16_t s_slot[kT];                 // triangles in draw order
+  __shared__ uint32_t s_off[kWaves][kBins / 2];   // per wavefront and bin, two to a word: counts, then next slots
+  __shared__ float4 s_bone_rows[kThreads > 64 ? kMaxLdsBones * kBoneRows : 1];
+  __shared__ M4 s_umvp;
+  __shared__ uint32_t s_w[kWaves];
+  __shared__ float s_mn[kWaves], s_mx[kWaves];
+  float* s_key = reinterpret_cast<float*>(s_u);
+  uint16_t* s_tri = reinterpret_cast<uint16_t*>(s_u + kT);
+  uint16_t* s_vo = reinterpret_cast<uint16_t*>(s_u);
+  const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+
+  // vertices
+  const bool skinned = (flags & PF_SKINNED) != 0;
+  const bool lds_bones = kThreads > 64 && skinned && load_uniform(&R.bone_count) <= kMaxLdsBones;
+  if (lds_bones) stage_bones(R, s_bone_rows);
+  if ((flags & PF_UNBB) && tid == 0) s_umvp = mult(load_uniform(&R.model), load_uniform(&fc.vp));
+  for (uint32_t i = tid; i < kWaves * (kBins / 2); i += kThreads) (&s_off[0][0])[i] = 0;
+  __syncthreads();
+  for (uint32_t i = tid; i < vcount; i += kThreads) {
+    V3 vp;
+    const VertexRecord r = shade_vertex(a, fc, R, flags, vmin + i, lds_bones ? s_bone_rows : nullptr, s_umvp, vp);
+    const uint32_t o = vbase + i;
+    a.vab[2 * (size_t)o + 0] = r.a;
+    a.vab[2 * (size_t)o + 1] = r.b;
+    if (skinned) a.vpos[o] = make_float4(vp.x, vp.y, vp.z, 0.0f);
+    s_q[i] = r.q;
+    s_z[i] = r.zin ? 1 : 0;
+  }
+  __syncthreads();
+
+  // cull: survivors in triangle order
+  const bool backface = (flags & PF_BACKFACE) != 0;
+  const bool all = (flags & PF_ALL) != 0;         // processOnlyVisible false: no test removes a triangle
+  const PartGPU P = load_uniform(&R);              // what the passes over triangles read of it
+  const V3 camPos = v3(load_uniform(&fc.campos[0]), load_uniform(&fc.campos[1]), load_uniform(&fc.campos[2]));
+  const V3 icp = v3(P.icp[0], P.icp[1], P.icp[2]);
+  float mn = kMaxF32, mx = 0.0f;
+  uint32_t n = 0;                                 // survivors so far, block-uniform
+  for (uint32_t base = 0; base < tcount; base += kThreads) {
+    const uint32_t t = base + tid;
+    bool keep = false;
+    float depth = -1.0f;
+    if (t < tcount) {
+      uint32_t ov[3];
+      corner_records(P, t, ov);
+      float4 cc[3];
+      V3 q[3];
+      bool zin = false;
+      if (skinned) {
+        for (int k = 0; k < 3; k++) {
+          const float4 x = a.vpos[ov[k]];
+          q[k] = v3(x.x, x.y, x.z);
+        }
+      } else {
+        const float* cp = P.ctr + 3 * (size_t)t;
+        q[0] = v3(cp[0], cp[1], cp[2]);
+      }
+      for (int k = 0; k < 3; k++) {
+        cc[k] = s_q[ov[k] - P.vbase];
+        zin |= s_z[ov[k] - P.vbase] != 0;
+      }
+      keep = all || visible(cc, zin, backface);
+      if (keep) {                                                       // model.go:941-960
+        depth = depth_key(skinned, camPos, icp, q);
+        if (!all && (isnan(depth) || isinf(depth))) keep = false;
+      }
+    }
+    const uint64_t m = __ballot(keep);
+    if (lane == 0) s_w[wave] = (uint32_t)__popcll(m);
+    __syncthreads();
+    uint32_t before = 0, tot = 0;
+    for (uint32_t w = 0; w < kWaves; w++) {
+      if (w < wave) before += s_w[w];
+      tot += s_w[w];
+    }
+    if (keep) {
+      const uint32_t at = n + before + (uint32_t)__popcll(m & lt_mask);
+      s_key[at] = depth;
+      s_tri[at] = (uint16_t)t;
+      mn = fminf(mn, depth);
+      mx = fmaxf(mx, depth);
+    }
+    n += tot;
+    __syncthreads();                              // s_w is rewritten next round
+  }
+  mn = wave_min(mn);
+  mx = wave_max(mx);
+  if (lane == 0) {
+    s_mn[wave] = mn;
+    s_mx[wave] = mx;
+  }
+  __syncthreads();
+  mn = s_mn[0];
+  mx = s_mx[0];
+  for (uint32_t w = 1; w < kWaves; w++) {
+    mn = fminf(mn, s_mn[w]);
+    mx = fmaxf(mx, s_mx[w]);
+  }
+  if (tid == 0) a.stats[4 * p + 2] = n;
+  if (n == 0) return;                             // block-uniform
+  float rd = mx - mn;
+  if (rd == 0) rd += 0.001f;                                            // sortingTriangles.go:43-46
+
+  // sort: each wavefront counts, then ranks, a contiguous share of the
+  // survivors' 64s, as in k_scatter4
+  const uint32_t mode = (flags >> PF_SORT_SHIFT) & 3u;
+  const uint32_t nchunks = (n + 63) / 64;
+  const uint32_t ch0 = wave * nchunks / kWaves, ch1 = (wave + 1) * nchunks / kWaves;
+  for (uint32_t c = ch0; c < ch1; c++) {
+    const uint32_t i = c * 64 + lane;
+    if (i < n) {
+      const uint32_t bin = visit_bin(s_key[i], mn, rd, mode);
+      atomicAdd(&s_off[wave][bin / 2], 1u << (16 * (bin % 2)));
+    }
+  }
+  __syncthreads();
+  uint16_t* off16 = reinterpret_cast<uint16_t*>(&s_off[0][0]);
+  {
+    constexpr uint32_t kPer = kThreads < kBins ? kBins / kThreads : 1;   // bins per thread
+    uint32_t sum = 0;
+    if (tid * kPer < kBins)
+      for (uint32_t k = tid * kPer; k < (tid + 1) * kPer; k++)
+        for (uint32_t w = 0; w < kWaves; w++) sum += off16[w * kBins + k];
+    uint32_t x = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(x, o);
+      if (lane >= (uint32_t)o) x += y;
+    }
+    if (lane == 63) s_w[wave] = x;
+    __syncthreads();
+    uint32_t next = x - sum;
+    for (uint32_t w = 0; w < wave; w++) next += s_w[w];
+    if (tid * kPer < kBins)
+      for (uint32_t k = tid * kPer; k < (tid + 1) * kPer; k++)
+        for (uint32_t w = 0; w < kWaves; w++) {
+          const uint32_t c = off16[w * kBins + k];
+          off16[w * kBins + k] = (uint16_t)next;
+          next += c;
+        }
+  }
+  __syncthreads();
+  uint16_t* off = off16 + wave * kBins;           // only this wavefront's from here on
+  for (uint32_t c = ch0; c < ch1; c++) {          // wave-uniform
+    const uint32_t i = c * 64 + lane;
+    const bool valid = i < n;
+    const uint64_t vmask = __ballot(valid);
+    const uint32_t bin = valid ? visit_bin(s_key[i], mn, rd, mode) : 0xFFFFu;
+    const uint64_t peers = bin_peers(bin, vmask);
+    const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
+    uint32_t slot = 0;
+    if (valid) slot = off[bin] + rank;
+    __builtin_amdgcn_wave_barrier();
+    if (valid && rank == 0) off[bin] = (uint16_t)(slot + (uint32_t)__popcll(peers));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (valid) s_slot[slot] = s_tri[i];
+  }
+  __syncthreads();
+  for (uint32_t k = tid; k < n; k += kThreads) {  // corners in draw order, over the keys
+    const uint4 r = slot_record(P, s_slot[k]);
+    a.tri_vo[P.tbase + k] = r;
+    s_vo[3 * k + 0] = (uint16_t)(r.x - P.vbase);
+    s_vo[3 * k + 1] = (uint16_t)(r.y - P.vbase);
+    s_vo[3 * k + 2] = (uint16_t)(r.z - P.vbase);
+  }
+  __syncthreads();
+
+  // lists, in the chunks of k_assemble
+  const float da = load_uniform(&fc.render_depth) ? 1.0f : 0.0f;
+  const float4* vab = a.vab + 2 * (size_t)P.vbase;   // this block's own stores, before the last barriers
+  float4* __restrict__ out_c = a.out_color + 3 * P.out_base;
+  float4* __restrict__ out_d = a.out_depth + 3 * P.out_base;
+  uint32_t* __restrict__ out_i = a.out_idx + P.out_base;
+  const int32_t end = 9 * (int32_t)n;
+  constexpr int32_t kPer = 9, kChunk = 64 * kPer;
+  for (int32_t c0 = -(int32_t)(3 * P.out_base % 64) + (int32_t)wave * kChunk; c0 < end; c0 += (int32_t)kWaves * kChunk) {
+    float4 v[kPer];
+    float4 w[kPer];
+#pragma unroll
+    for (int32_t q = 0; q < kPer; q++) {
+      const uint32_t g = (uint32_t)min(max(c0 + q * 64 + (int32_t)lane, 0), end - 1);   // an active float4
+      const uint32_t corner = g / 3, piece = g % 3, o = s_vo[corner];
+      w[q] = s_q[o];
+      if (piece != 2) v[q] = vab[2 * o + piece];
+    }
+#pragma unroll
+    for (int32_t q = 0; q < kPer; q++) {
+      const int32_t g = c0 + q * 64 + (int32_t)lane;
+      if (g < 0 || g >= end) continue;
+      const uint32_t piece = (uint32_t)g % 3;
+      const float4 custom = make_float4(w[q].w, 0.0f, 0.0f, 0.0f);
+      store4<true>(&out_c[g], piece == 2 ? custom : v[q]);
+      store4<true>(&out_d[g], piece == 2 ? custom : piece == 1 ? make_float4(w[q].z, w[q].z, w[q].z, da) : v[q]);
+    }
+  }
+  for (uint32_t i = tid; i < 3 * n; i += kThreads) store1<true>(&out_i[i], P.idx_base + i);   // camera.go:1816
+}
+
 // Fill of a word array (test poisoning of outputs: unwritten entries show up).
 __global__ __launch_bounds__(256) void k_fill(uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
@@ -1515,6 +1783,24 @@ hipError_t launch_assemble(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uin
     case 1: hipLaunchKernelGGL((k_assemble<false, true>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
     case 2: hipLaunchKernelGGL((k_assemble<true, false>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
     default: hipLaunchKernelGGL((k_assemble<true, true>), g, dim3(kAsmThreads), 0, s, b, blk0, sub, per); break;
+  }
+  return hipGetLastError();
+}
+// The workgroup: one wavefront for pairs of at most 128 vertices and triangles;
+// four for larger ones when there are more pairs than CUs can take at sixteen
+// wavefronts each; else sixteen.
+hipError_t launch_pairs(const FrameArgs& a, uint32_t npairs, uint32_t max_vertices, uint32_t max_triangles, hipStream_t s) {
+  if (!npairs) return hipSuccess;
+  const uint32_t V = max_vertices, T = max_triangles;
+  const dim3 g(npairs);
+  if (V <= 128 && T <= 128) hipLaunchKernelGGL((k_pair<64, 128, 128>), g, dim3(64), 0, s, a);
+  else if (V <= kPairVertices && T <= kPairTriangles) {
+    if (npairs > 512) hipLaunchKernelGGL((k_pair<256, kPairVertices, kPairTriangles>), g, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((k_pair<1024, kPairVertices, kPairTriangles>), g, dim3(1024), 0, s, a);
+  } else if (V <= kPairVerticesMany && T <= kPairTrianglesMany) {
+    hipLaunchKernelGGL((k_pair<1024, kPairVerticesMany, kPairTrianglesMany>), g, dim3(1024), 0, s, a);
+  } else {
+    return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }

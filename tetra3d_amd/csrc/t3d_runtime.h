@@ -37,7 +37,7 @@ struct Mesh {
   const uint16_t* idx16 = nullptr; // ... or uint16 when the mesh has at most 65,536 vertices
   const float* ctr = nullptr;      // Triangle.Center per triangle, xyz (mesh.go:1980-1982, kept as AddTriangles does)
   uint32_t V = 0, T = 0, K = 0;
-  uint32_t max_part = 0;           // triangles of its largest part
+  uint32_t max_part = 0, max_vertices = 0;   // most triangles and vertices of a part
   std::vector<t3d_part_range> parts;
   std::vector<uint32_t> part_vmin, part_vcount;
   float dmin[3], dmax[3];
@@ -140,7 +140,9 @@ struct t3d_frame {
   const t3d::MaterialGPU* stage_mats = nullptr;
   uint64_t table_bytes = 0;
   uint64_t total_triangles = 0;
-  uint32_t max_triangles = 0;      // of one render pair (with the device stage: of any MeshPart)
+  uint32_t max_triangles = 0, max_vertices = 0;   // of one render pair (with the device stage: of any MeshPart)
+  bool small_pairs = false;        // may be drawn by one workgroup per render pair
+  bool ran_pairs = false;          // the last launch was (the profile's names)
   uint32_t nparts = 0;
   uint32_t total_vchunks = 0, total_tiles = 0, total_sblocks = 0;
   std::vector<uint32_t> vchunk_prefix, tile_prefix, sblock_prefix, pscan_prefix;
