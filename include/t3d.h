@@ -487,7 +487,7 @@ t3d_status t3d_profile_read(t3d_ctx* ctx, t3d_kernel_time* per_kernel, uint32_t 
  * tables and scratch come from a static per-GPU device array of
  * T3D_NOALLOC_SCRATCH_BYTES and the outputs are the caller's device arrays,
  * each holding vertex_capacity entries.  Calls no hipMalloc, hipHostMalloc or
- * hipFree and builds no graph; the tables go up from pageable host memory
+ * hipFree and builds no graph; the tables go up from host memory
  * and the call waits for the frame.  Pair p's results occupy vertices
  * [vertex_offset, vertex_offset + 3*survivor_count) of the caller's arrays
  * (t3d_frame_pairs), so the arrays must hold 3 x the triangles of every drawn
@@ -519,7 +519,9 @@ typedef struct {
   uint32_t model_stage;              /* 1: the batched form runs the model-level stage (frustum test, render
                                         pairs and their order, per-pair slices) on the device when the
                                         frame allows it: no dynamic batch, RenderDepth on, every model at a
-                                        finite distance from its camera; 0: always on the host */
+                                        finite distance from its camera; 0: always on the host.  Until a
+                                        shape is set or autotuned, 1 leaves frames of up to 640 models
+                                        to the host */
 } t3d_tuning;
 t3d_status t3d_get_tuning(const t3d_ctx* ctx, t3d_tuning* out);
 t3d_status t3d_set_tuning(t3d_ctx* ctx, const t3d_tuning* tuning);

@@ -12,6 +12,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <limits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -21,6 +22,7 @@
 #include <vector>
 
 #include "t3d_runtime.h"
+#include "t3d_stage.h"
 
 using namespace t3d;
 
@@ -239,15 +241,15 @@ uint64_t placed_charge(uint64_t V, uint64_t T) {
 }
 
 // Whether a frame of `pairs` render pairs (or candidates) and T triangles in all is drawn by one workgroup per render
-// pair (k_pair) instead of the chain of passes over all pairs: where no pair is over kPairVertices and kPairTriangles;
-// and up to the larger limits where there are many pairs and their mean is at least half of the largest, so that no
-// workgroup is waited for long.  One sphere of 2,562 vertices: 100 us a frame against the chain's 104; 16 skinned ones
-// 137 against 131; 64 of them 150 against 155; 256 295 against 335.
-bool pairs_fit(const t3d_frame* f, uint64_t pairs, uint64_t T, bool normals, bool groups) {
+// pair (k_pair) instead of the chain of passes over all pairs: where no pair is over kPairVertices and kPairTriangles; and
+// up to the larger limits where there are only a few, none skinned (one sphere of 2,562 vertices: 45 us a frame, 53 with
+// the chain; five uneven models 43 and 60; two skinned spheres 86 and 80), or many whose mean is at least half of the
+// largest, so that no workgroup is waited for long (64 skinned spheres 150 and 155, 256 of them 295 and 335).
+bool pairs_fit(const t3d_frame* f, uint64_t pairs, uint64_t T, bool skinned, bool normals, bool groups) {
   if (normals || groups) return false;
   const uint64_t v = f->max_vertices, t = f->max_triangles;
   if (v <= kPairVertices && t <= kPairTriangles) return true;
-  return v <= kPairVerticesMany && t <= kPairTrianglesMany && pairs >= kPairMany && 2 * T >= pairs * t;
+  return v <= kPairVerticesMany && t <= kPairTrianglesMany && ((pairs <= kPairFew && !skinned) || (pairs >= kPairMany && 2 * T >= pairs * t));
 }
 
 // ---------------------------------------------------------------------------
@@ -708,10 +710,17 @@ t3d_status t3d_ctx_create(int32_t device, uint64_t hbm_budget_bytes, t3d_ctx** o
     delete c;
     return T3D_ERR_DEVICE;
   }
+  if (hipHostMalloc((void**)&c->pinned, kPinnedTables + 16ull * kHostUniforms, hipHostMallocDefault) != hipSuccess) {
+    (void)hipStreamDestroy(c->stream);
+    (void)hipStreamDestroy(c->copy_stream);
+    delete c;
+    return T3D_ERR_DEVICE;
+  }
   // this device's copy of the scratch array of t3d_render_noalloc, looked up with the device current
   if (noalloc_scratch_address(device, &c->noalloc_scratch) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     (void)hipStreamDestroy(c->copy_stream);
+    (void)hipHostFree(c->pinned);
     delete c;
     return T3D_ERR_DEVICE;
   }
@@ -731,6 +740,7 @@ t3d_status t3d_ctx_destroy(t3d_ctx* c) {
   }
   (void)hipStreamDestroy(c->stream);
   (void)hipStreamDestroy(c->copy_stream);
+  (void)hipHostFree(c->pinned);
   delete c;
   return T3D_OK;
 }
@@ -1119,7 +1129,7 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
     ProfScope ps(c, st, "k_palettes", f->bytes_palettes, prof);
     HIP_TRY(c, launch_palettes(a, st));
   }
-  {
+  if (!f->host_uniforms) {
     ProfScope ps(c, st, "k_uniforms", 0, prof);
     HIP_TRY(c, launch_uniforms(a, p0, p1 - p0, st));
   }
@@ -1278,8 +1288,27 @@ namespace {
 // RenderDepth on (its solids then keep model order), and no drawable model is
 // at a NaN distance from its camera (the transparents' comparator is then a
 // strict weak order, so a stable sort by it is Go's SliceStable's order).
+// A frame of at most kHostModels models and MeshParts: its pairs are built on the host, at about 0.1 us each, where the
+// stage's two kernels take 15 us and more on the device, and the readback of what they built another ten: 500 cubes
+// 80 us a frame and 96, 300 uneven models 345 and 358, 512 of them 535 and 554.  Past that the host's part is longer
+// than what it saves (4,096 cubes: 0.25 ms against 0.21).
+bool few_models(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
+  uint64_t pairs = 0;
+  for (uint32_t j = 0; j < ndesc; j++) {
+    const t3d_render_desc* d = descs[j];
+    if (!d || d->exec_mode != T3D_EXEC_BATCHED || (d->model_count && !d->models) || d->model_count > kHostModels)
+      return false;
+    for (uint32_t mi = 0; mi < d->model_count; mi++) {
+      auto it = c->meshes.find(d->models[mi].mesh);
+      if (it != c->meshes.end()) pairs += it->second->parts.size();
+    }
+  }
+  return pairs <= kHostModels;
+}
+
 bool stage_applies(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
   if (!c->tuning.model_stage) return false;
+  if (c->stage_auto && few_models(c, descs, ndesc)) return false;
   for (uint32_t j = 0; j < ndesc; j++) {
     const t3d_render_desc* d = descs[j];
     if (!d || !d->camera || !d->camera->render_depth || d->process_all_triangles) return false;
@@ -1694,7 +1723,7 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   take_records(sc, a, wV, wT, any_skinned);
   f->max_triangles = max_tri;
   f->max_vertices = max_vert;
-  f->small_pairs = pairs_fit(f, ncand, wT, any_normals, false);
+  f->small_pairs = pairs_fit(f, ncand, wT, any_skinned, any_normals, false);
   a.hist = sc.take<uint32_t>(whist);
   a.bsum = sc.take<uint32_t>(wsb);
   a.tile_count = sc.take<uint32_t>(wtiles);
@@ -1749,6 +1778,7 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
                        const Placement* place, bool device_stage) {
   auto wall0 = std::chrono::steady_clock::now();
   if (!c || !f || !descs || ndesc == 0) return fail(c, T3D_ERR_INVALID_ARGUMENT, "render: null argument");
+  f->host_uniforms = f->host_stats = false;
   if (device_stage && !place && stage_applies(c, descs, ndesc)) {
     t3d_status sst = frame_build_stage(c, f, descs, ndesc);
     if (sst != T3D_ERR_UNSUPPORTED) return sst;   // else too large for the worst case: sized by what is drawn
@@ -2241,16 +2271,41 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   }
   const uint32_t npose = (uint32_t)pose_jobs.size();
 
+  bool any_skinned = false;
+  f->max_triangles = f->max_vertices = 0;
+  for (const PartGPU& P : f->parts) {
+    f->max_triangles = std::max(f->max_triangles, P.tcount);
+    f->max_vertices = std::max(f->max_vertices, P.vcount);
+    any_skinned = any_skinned || (P.flags & PF_SKINNED);
+  }
+  f->small_pairs = pairs_fit(f, P_n, sumT, any_skinned, any_normals, ngroups != 0);
+  // few pairs: their uniforms and per-light values are computed here, instead of by k_uniforms (but for a volume's
+  // cell at a model's position, which is on the device)
+  f->host_uniforms = P_n && P_n <= kHostUniforms && n_plights <= kHostLights && !ngroups;
+  for (uint32_t j = 0; j < ndesc; j++) f->host_uniforms = f->host_uniforms && descs[j]->exec_mode == T3D_EXEC_BATCHED;
+  for (const PartGPU& P : f->parts)
+    for (uint32_t k = 0; k < P.light_count; k++)
+      if (lights[P.light0 + k].type == T3D_LIGHT_VOLUME && ((P.flags >> PF_LVMODE_SHIFT) & 3u) == T3D_LV_PER_OBJECT)
+        f->host_uniforms = false;
+  f->host_stats = !ngroups && P_n && (!place || P_n <= kHostUniforms);
+  for (uint32_t j = 0; j < ndesc; j++) f->host_stats = f->host_stats && descs[j]->exec_mode == T3D_EXEC_BATCHED;
+  const uint64_t host_plights = f->host_uniforms ? n_plights : 0;
+  const uint64_t host_pairs = f->host_uniforms ? P_n : 0;
+  // the chain's block -> pair maps, where there are more pairs than its blocks search among
+  const uint64_t host_tiles = host_pairs > kSearchPairs && !f->small_pairs ? f->tile_prefix.back() : 0;
+  const uint64_t host_chunks = host_tiles ? f->vchunk_prefix.back() : 0;
+  const uint64_t host_bytes = carve_size<PartLight>(host_plights) + carve_size<uint4>(host_pairs) +
+                              carve_size<uint32_t>(host_tiles) + carve_size<uint32_t>(host_chunks);
+
   // device tables: FrameConst[jobs], parts, lights, prefixes, palettes, shape-key weights
   const uint64_t tbytes = carve_size<FrameConst>(ndesc) + carve_size<PartGPU>(P_n) + carve_size<LightGPU>(lights.size()) +
                           4 * carve_size<uint32_t>(P_n + 1) +
                           carve_size<float>(pal_floats) + carve_size<float>(skw_floats) +
                           carve_size<t3d_bone_pose>(pose_bones) + carve_size<M4>(pose_roots) +
-                          carve_size<PaletteJob>(npose) + carve_size<uint2>(ngroups);
+                          carve_size<PaletteJob>(npose) + carve_size<uint2>(ngroups) +
+                          host_bytes;
   // scratch: vertex records, skinned positions, keys, survivor records, stats, histograms, block sums
   const uint32_t ntiles_total = f->tile_prefix.back();
-  bool any_skinned = false;
-  for (uint32_t i = 0; i < P_n && !any_skinned; i++) any_skinned = (f->parts[i].flags & PF_SKINNED) != 0;
   const uint64_t rest = carve_size<uint32_t>(4ull * P_n) + carve_size<uint32_t>(sumHist) +
                         carve_size<uint32_t>(sblocks) + 2 * carve_size<uint32_t>(ntiles_total) +
                         carve_size<uint32_t>(f->vchunk_prefix.back()) + carve_size<PartLight>(n_plights) +
@@ -2264,7 +2319,7 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
       return fail(c, T3D_ERR_UNSUPPORTED, "render_noalloc: Camera.RenderNormals needs a normal vertex array, which "
                                           "this entry point does not take");
     // no allocation: tables and scratch carved from the placement's scratch, outputs the caller's
-    const uint64_t charge = tbytes + rest + placed_charge(sumV, sumT);
+    const uint64_t charge = tbytes - host_bytes + rest + placed_charge(sumV, sumT);
     if (charge > place->scratch_bytes)
       return fail(c, T3D_ERR_BUDGET, "render_noalloc: the frame needs %llu bytes of scratch, the static scratch holds %llu",
                   (unsigned long long)charge, (unsigned long long)place->scratch_bytes);
@@ -2275,10 +2330,10 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
       return fail(c, T3D_ERR_INVALID_ARGUMENT, "render_noalloc: outputs hold %llu vertices, the frame needs %llu",
                   (unsigned long long)place->capacity, (unsigned long long)(3 * sumT));
     if (f->host_tables.size() < tbytes) f->host_tables.resize(tbytes);
-    if (f->host_stats.size() < 4ull * P_n) f->host_stats.resize(4ull * P_n);
+    if (f->host_stats_copy.size() < 4ull * P_n) f->host_stats_copy.resize(4ull * P_n);
     tables_dev = place->scratch;
     scratch_dev = place->scratch + tbytes;   // tbytes is a sum of 256-byte-aligned slices
-    tables_host = f->host_tables.data();
+    tables_host = tbytes <= kPinnedTables ? place->pinned_tables : f->host_tables.data();
     out_color = place->color;
     out_depth = place->depth;
     out_idx = place->idx;
@@ -2345,7 +2400,33 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   PaletteJob* h_pjobs = host.take<PaletteJob>(npose);
   uint2* d_groups = dev.take<uint2>(ngroups);
   uint2* h_groups = host.take<uint2>(ngroups);
+  PartLight* d_plights = dev.take<PartLight>(host_plights);
+  PartLight* h_plights = host.take<PartLight>(host_plights);
+  uint4* d_stats = dev.take<uint4>(host_pairs);
+  uint4* h_stats = host.take<uint4>(host_pairs);
+  uint32_t* d_tpart = dev.take<uint32_t>(host_tiles);
+  uint32_t* h_tpart = host.take<uint32_t>(host_tiles);
+  uint32_t* d_vpart = dev.take<uint32_t>(host_chunks);
+  uint32_t* h_vpart = host.take<uint32_t>(host_chunks);
+  if (host_tiles)
+    for (uint32_t i = 0; i < P_n; i++) {
+      std::fill(h_tpart + f->tile_prefix[i], h_tpart + f->tile_prefix[i + 1], i);
+      std::fill(h_vpart + f->vchunk_prefix[i], h_vpart + f->vchunk_prefix[i + 1], i);
+    }
   if (ngroups) std::memcpy(h_groups, f->groups.data(), sizeof(uint2) * ngroups);
+  if (f->host_uniforms) {
+    for (uint32_t i = 0; i < P_n; i++) {
+      PartGPU& P = f->parts[i];
+      const ModelInverse inv = model_inverse(P.model);
+      for (uint32_t k = 0; k < P.light_count; k++)
+        h_plights[P.light_base + k] = pair_light(P, inv, lights[P.light0 + k], P.light0 + k);
+      complete_pair(P, inv, f->fcs[P.cam]);
+      uint4 st = make_uint4(0, 0, 0, 0);
+      const float none = std::numeric_limits<float>::max();   // minDepth = MaxFloat32 (model.go:702)
+      std::memcpy(&st.x, &none, 4);
+      h_stats[i] = st;
+    }
+  }
   uint64_t pal_off = 0, skw_off = 0;
   for (uint32_t i = 0; i < P_n; i++) {
     PartGPU& P = f->parts[i];
@@ -2411,12 +2492,6 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   a.sblock_prefix = d_spre;
   a.pscan_prefix = d_ppre;
   take_records(sc, a, sumV, sumT, any_skinned);
-  f->max_triangles = f->max_vertices = 0;
-  for (const PartGPU& P : f->parts) {
-    f->max_triangles = std::max(f->max_triangles, P.tcount);
-    f->max_vertices = std::max(f->max_vertices, P.vcount);
-  }
-  f->small_pairs = pairs_fit(f, P_n, sumT, any_normals, ngroups != 0);
   a.stats = sc.take<uint32_t>(4ull * P_n);
   a.hist = sc.take<uint32_t>(sumHist);
   a.bsum = sc.take<uint32_t>(sblocks);
@@ -2424,6 +2499,16 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   a.tile_part = sc.take<uint32_t>(ntiles_total);
   a.vchunk_part = sc.take<uint32_t>(f->vchunk_prefix.back());
   a.plights = sc.take<PartLight>(n_plights);
+  if (f->host_stats) {      // k_pair or k_assemble puts the survivor counts where the host reads them
+    a.host_stats = place ? place->pinned_stats : f->pinned_stats;
+    for (uint32_t i = 0; i < P_n; i++) a.host_stats[4 * i + 2] = 0;
+  }
+  if (f->host_uniforms) {   // from the tables
+    a.plights = d_plights;
+    a.stats = reinterpret_cast<uint32_t*>(d_stats);
+    a.tile_part = host_tiles ? d_tpart : nullptr;
+    a.vchunk_part = host_tiles ? d_vpart : nullptr;
+  }
   a.pose_world = sc.take<M4>(pose_bones);
   a.vnrm = sc.take<float4>(any_normals ? sumV : 1);
   a.out_normal = reinterpret_cast<float4*>(out_normal);
@@ -2464,11 +2549,13 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
 // Sends the tables and enqueues the chain (graph replay when allowed) and the
 // survivor-count readback on `stream`; returns without waiting.
 t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_t copy_stream, int32_t exec_mode,
-                        bool allow_graph, bool profile) {
+                        bool allow_graph, bool profile, bool alone) {
   const uint32_t P_n = f->nparts;
   const FrameArgs& a = f->args;
   if (!f->done) HIP_TRY(c, hipEventCreateWithFlags(&f->done, hipEventDisableTiming));
   if (!f->tables_ready) HIP_TRY(c, hipEventCreateWithFlags(&f->tables_ready, hipEventDisableTiming));
+  // where nothing runs that the copy could overlap, or for a few KB, the wait between the streams takes longer
+  if (alone || f->host_uniforms) copy_stream = stream;
   HIP_TRY(c, hipMemcpyAsync(f->tables.ptr, f->pinned, f->table_bytes, hipMemcpyHostToDevice, copy_stream));
   if (copy_stream != stream) {
     HIP_TRY(c, hipEventRecord(f->tables_ready, copy_stream));
@@ -2485,7 +2572,7 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
       st = run_chain(c, f, i, i + 1, stream, profile);
       if (st) return st;
     }
-  } else if (allow_graph && c->tuning.use_graph && !(profile && c->profiling)) {
+  } else if (allow_graph && c->tuning.use_graph && !f->host_uniforms && !(profile && c->profiling)) {
     // graph of the whole chain; reused while the launch shape is unchanged
     std::vector<uint8_t> key(sizeof(FrameArgs) + 12 * sizeof(uint32_t));
     uint32_t shape[12] = {f->total_vchunks,       f->total_tiles,           f->total_sblocks,
@@ -2521,6 +2608,8 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
   if (f->device_stage) {   // counts, the jobs' first pairs, the pairs and their stats in one copy
     HIP_TRY(c, hipMemcpyAsync(f->pinned_rb, f->rb_dev, f->rb_bytes, hipMemcpyDeviceToHost, stream));
     f->stats_host = reinterpret_cast<const uint32_t*>(f->pinned_rb + f->rb_stats);
+  } else if (f->host_stats) {
+    f->stats_host = f->pinned_stats;   // written there by the chain
   } else {
     HIP_TRY(c, hipMemcpyAsync(f->pinned_stats, a.stats, 16ull * P_n, hipMemcpyDeviceToHost, stream));
     f->stats_host = f->pinned_stats;
@@ -2532,7 +2621,8 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
 t3d_status frame_run_placed(t3d_ctx* c, t3d_frame* f, hipStream_t stream, int32_t exec_mode) {
   const uint32_t P_n = f->nparts;
   const FrameArgs& a = f->args;
-  HIP_TRY(c, hipMemcpyAsync(f->tables_dev, f->host_tables.data(), f->table_bytes, hipMemcpyHostToDevice, stream));
+  const uint8_t* tables = f->table_bytes <= kPinnedTables ? c->pinned : f->host_tables.data();
+  HIP_TRY(c, hipMemcpyAsync(f->tables_dev, tables, f->table_bytes, hipMemcpyHostToDevice, stream));
   if (c->poison && f->total_triangles) {
     const uint64_t nv = 3 * f->total_triangles;
     HIP_TRY(c, launch_fill(a.out_color, nv * sizeof(t3d_vertex), c->poison, stream));
@@ -2549,10 +2639,11 @@ t3d_status frame_run_placed(t3d_ctx* c, t3d_frame* f, hipStream_t stream, int32_
       t3d_status st = run_chain(c, f, 0, P_n, stream, false);
       if (st) return st;
     }
-    HIP_TRY(c, hipMemcpyAsync(f->host_stats.data(), a.stats, 16ull * P_n, hipMemcpyDeviceToHost, stream));
+    if (!f->host_stats)
+      HIP_TRY(c, hipMemcpyAsync(f->host_stats_copy.data(), a.stats, 16ull * P_n, hipMemcpyDeviceToHost, stream));
   }
   HIP_TRY(c, hipStreamSynchronize(stream));
-  f->stats_host = f->host_stats.data();
+  f->stats_host = f->host_stats ? reinterpret_cast<const uint32_t*>(c->pinned + kPinnedTables) : f->host_stats_copy.data();
   frame_collect(c, f, false);
   return T3D_OK;
 }
@@ -2843,7 +2934,7 @@ t3d_status frame_finish(t3d_ctx* c, t3d_frame* f) {
   return T3D_OK;
 }
 
-t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc) {
+t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, bool alone) {
   const auto wall0 = std::chrono::steady_clock::now();
   t3d_status st = frame_finish(c, f);
   if (st) return st;
@@ -2856,7 +2947,7 @@ t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc) 
     f->device_stage = false;
     return st;
   }
-  st = frame_launch(c, f, f->stream ? f->stream : c->stream, c->copy_stream, desc->exec_mode, true, true);
+  st = frame_launch(c, f, f->stream ? f->stream : c->stream, c->copy_stream, desc->exec_mode, true, true, alone);
   if (st) return st;
   f->submitted = wall0;
   f->inflight = true;
@@ -2868,7 +2959,7 @@ t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc) 
 extern "C" t3d_status t3d_render(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc) {
   if (!c || !f || !desc) return fail(c, T3D_ERR_INVALID_ARGUMENT, "render: null argument");
   std::lock_guard<std::mutex> lk(c->mu);
-  t3d_status st = render_submit(c, f, desc);
+  t3d_status st = render_submit(c, f, desc, true);
   if (st) return st;
   return frame_finish(c, f);
 }
@@ -2876,7 +2967,7 @@ extern "C" t3d_status t3d_render(t3d_ctx* c, t3d_frame* f, const t3d_render_desc
 extern "C" t3d_status t3d_render_async(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc) {
   if (!c || !f || !desc) return fail(c, T3D_ERR_INVALID_ARGUMENT, "render: null argument");
   std::lock_guard<std::mutex> lk(c->mu);
-  return render_submit(c, f, desc);
+  return render_submit(c, f, desc, false);
 }
 
 extern "C" t3d_status t3d_frame_wait(t3d_ctx* c, t3d_frame* f) {
@@ -3039,6 +3130,7 @@ t3d_status t3d_set_tuning(t3d_ctx* c, const t3d_tuning* t) {
     return fail(c, T3D_ERR_INVALID_ARGUMENT, "tuning: cull_block is 256, 512 or 1024");
   if (t->model_stage > 1) return fail(c, T3D_ERR_INVALID_ARGUMENT, "tuning: model_stage is 0 or 1");
   c->tuning = *t;
+  c->stage_auto = false;
   return T3D_OK;
 }
 
@@ -3049,6 +3141,8 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
   if (!c || !f || !desc) return T3D_ERR_INVALID_ARGUMENT;
   reps = std::max<uint32_t>(reps, 1);
   const t3d_tuning base = c->tuning;
+  const bool base_auto = c->stage_auto;
+  c->stage_auto = false;   // a candidate's model_stage is what it says
   t3d_render_desc d = *desc;
   d.exec_mode = T3D_EXEC_BATCHED;
   auto valid = [](const t3d_tuning& t) {
@@ -3111,6 +3205,7 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
       {&t3d_tuning::xcd_swizzle, {0, 1}},
       {&t3d_tuning::cull_block, {256, 512, 1024}},
       {&t3d_tuning::model_stage, {0, 1}},
+      {&t3d_tuning::use_graph, {0, 1}},
   };
   t3d_tuning best = base;
   if (!valid(best)) best.assemble_split = 1;
@@ -3156,6 +3251,7 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
   if (f2) (void)t3d_frame_destroy(c, f2);
   if (st) {
     c->tuning = base;
+    c->stage_auto = base_auto;
     return st;
   }
   c->tuning = best;

@@ -31,6 +31,8 @@ constexpr uint32_t kMaxTile = 2048;    // triangles per tile (keys of a tile are
 constexpr uint32_t kPairVertices = 1024, kPairTriangles = 2048;  // the largest render pair of a frame k_pair draws ...
 constexpr uint32_t kPairVerticesMany = 2816, kPairTrianglesMany = 5632;  // ... where there are kPairMany of about one size
 constexpr uint32_t kPairMany = 64;
+constexpr uint32_t kPairFew = 16;      // ... or at most so many, none skinned
+constexpr uint32_t kSearchPairs = 4;   // a host-built frame's blocks search among this many pairs; more have maps
 constexpr uint64_t kTouchVertices = 2400000;  // frames with more vertex records read them ahead of the assembly
 constexpr uint32_t kScanPartMax = 65536;  // histogram matrices up to this size are scanned by one block
 
@@ -314,9 +316,10 @@ struct FrameArgs {
   float* key;
   uint16_t* tri_loc;            // [sumT] survivors, triangle order: the triangle's place in its tile
   uint4* tri_vo;                // [sumT] survivors, output-slot order: {vertex-record offsets x3, triangle}
+  uint32_t* host_stats;         // where the host reads survivor counts, [P][4] (a frame built on the host), or null
   uint32_t* stats;              // [P][4]: min bits, max bits, survivors, 1 when some vertex's Z is out of range
   uint32_t* tile_count;         // [tiles] survivors of each tile (compacted at the tile's front)
-  uint32_t* tile_part;          // [tiles] render pair of each tile (written by k_uniforms)
+  uint32_t* tile_part;          // [tiles] render pair of each tile (written by k_uniforms); null: few pairs, searched for
   uint32_t* vchunk_part;        // [vertex chunks] render pair of each vertex-kernel block (k_uniforms)
   uint32_t* hist;
   uint32_t* bsum;

@@ -48,6 +48,12 @@ __device__ __forceinline__ uint32_t find_part(const uint32_t* __restrict__ prefi
   return lo;
 }
 
+// The pair of block b: from k_uniforms' map, or, in a frame of few pairs that
+// has none, from the prefix itself.
+__device__ __forceinline__ uint32_t pair_of(const uint32_t* map, const uint32_t* prefix, uint32_t n, uint32_t b) {
+  return map ? map[b] : find_part(prefix, n, b);
+}
+
 // Workgroups of a launch are dealt round-robin to the 8 XCDs (workgroup i to
 // XCD i % 8), each with its own L2.  With the swizzle on, the workgroups an
 // XCD receives take consecutive logical block numbers, so the blocks of one
@@ -458,7 +464,7 @@ __global__ __launch_bounds__(256, 8) void k_vertex(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_VCHUNKS, 1);
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
-  const uint32_t p = a.vchunk_part[b];
+  const uint32_t p = pair_of(a.vchunk_part, a.vchunk_prefix, a.nparts, b);
   const PartGPU& P = a.parts[p];
   const uint32_t flags = load_uniform(&P.flags);
 
@@ -628,31 +634,12 @@ __global__ __launch_bounds__(kUniformThreads) void k_uniforms(FrameArgs a, uint3
   const uint32_t nl = (flags & PF_LIGHTING) ? P.light_count : 0u;
   if (k > 0 && k >= nl) return;
   const FrameConst& fc = a.fc[P.cam];
-  const M4 M = P.model;
-  V3 dp, ds;
-  M4 dr;
-  decompose(inverted(M), dp, ds, dr);
-  const V3 is = v3(fdiv(1.0f, ds.x), fdiv(1.0f, ds.y), fdiv(1.0f, ds.z));
+  const ModelInverse inv = model_inverse(P.model);
   for (uint32_t kk = k; kk < nl; kk += 64) {
-    const bool skinned = (flags & PF_SKINNED) != 0;
-    const uint32_t lvmode = (flags >> PF_LVMODE_SHIFT) & 3u;
-    const V3 modelPos = row3(M);
-    PartLight pl{};
-    pl.light = P.light0 + kk;
-    const LightGPU& L = a.lights[pl.light];
-    pl.enabled = L.nested ? 0u : 1u;   // a volume's cell light runs from its cells only, unskipped
-    if (L.type == T3D_LIGHT_POINT) {
-      const V3 wp = v3(L.pos[0], L.pos[1], L.pos[2]);
-      const V3 w = skinned ? wp : add(mult_vec(dr, wp), hmul(dp, is));
-      pl.v[0] = w.x;
-      pl.v[1] = w.y;
-      pl.v[2] = w.z;
-      if (L.range > 0 && !L.nested) {
-        const float dist = P.max_span + L.range;
-        if (dist_sq(modelPos, wp) > dist * dist) pl.enabled = 0;
-      }
-    } else if (L.type == T3D_LIGHT_VOLUME && lvmode == T3D_LV_PER_OBJECT) {
-      const float* cell = volume_cell(L, modelPos);
+    const LightGPU& L = a.lights[P.light0 + kk];
+    PartLight pl = pair_light(P, inv, L, P.light0 + kk);
+    if (L.type == T3D_LIGHT_VOLUME && ((flags >> PF_LVMODE_SHIFT) & 3u) == T3D_LV_PER_OBJECT) {
+      const float* cell = volume_cell(L, row3(P.model));
       if (cell) {
         pl.cell_found = 1;
         pl.v[0] = cell[0];
@@ -668,18 +655,7 @@ __global__ __launch_bounds__(kUniformThreads) void k_uniforms(FrameArgs a, uint3
     st[1] = 0u;                        // max over non-negative keys
     st[2] = 0u;                        // survivors
     st[3] = 0u;
-    P.mvp = mult(P.mvp, fc.vp);          // the uploaded base (model.go:634-695)
-    if (fc.render_normals) {             // mvJustRForNormals (model.go:705-708)
-      V3 np, ns;
-      M4 nr;
-      decompose(mult(M, fc.view), np, ns, nr);
-      P.nrot = nr;
-    }
-    const V3 icp = add(mult_vec(dr, v3(fc.campos[0], fc.campos[1], fc.campos[2])), hmul(dp, is));
-    P.icp[0] = icp.x;
-    P.icp[1] = icp.y;
-    P.icp[2] = icp.z;
-    if (flags & PF_NEED_RD) P.rd = transposed(inverted(P.rd));
+    complete_pair(P, inv, fc);
   }
 }
 
@@ -752,7 +728,7 @@ __global__ __launch_bounds__(kThreads) void k_cull(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_TILES, 1);
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
-  const uint32_t p = a.tile_part[b];
+  const uint32_t p = pair_of(a.tile_part, a.tile_prefix, a.nparts, b);
   const PartGPU P = a.parts[p];        // by value: read once, before any store
   const uint32_t flags = P.flags;
   const FrameConst fc = a.fc[P.cam];
@@ -888,7 +864,7 @@ __global__ __launch_bounds__(kHistThreads) void k_hist(FrameArgs a, uint32_t blk
   const uint32_t lb = frame_block(a, FC_TILES, 1);
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
-  const uint32_t p = a.tile_part[b];
+  const uint32_t p = pair_of(a.tile_part, a.tile_prefix, a.nparts, b);
   const PartGPU P = a.parts[p];        // by value: read once, before any store
   if (P.ntiles <= 1) return;
   __shared__ uint32_t h[kBins];
@@ -1080,7 +1056,7 @@ __global__ __launch_bounds__(64) void k_scatter(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_TILES, 1);
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
-  const uint32_t p = a.tile_part[b];
+  const uint32_t p = pair_of(a.tile_part, a.tile_prefix, a.nparts, b);
   const PartGPU P = a.parts[p];        // by value: read once, before any store
   if (a.stats[4 * p + 2] == 0) return;
   const uint32_t tl = b - a.tile_prefix[p];
@@ -1159,7 +1135,7 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_TILES, 1);
   if (lb == kNoBlock) return;
   const uint32_t b = blk0 + lb;
-  const uint32_t p = a.tile_part[b];
+  const uint32_t p = pair_of(a.tile_part, a.tile_prefix, a.nparts, b);
   const PartGPU P = a.parts[p];        // by value: read once, before any store
   if (a.stats[4 * p + 2] == 0) return;
   const uint32_t tl = b - a.tile_prefix[p];
@@ -1324,8 +1300,9 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(FrameArgs a, uint32_t 
   const uint32_t li = frame_block<true>(a, FC_TILES, per);
   if (li == kNoBlock) return;
   const uint32_t b = blk0 + li / per;
-  const uint32_t p = a.tile_part[b];
+  const uint32_t p = pair_of(a.tile_part, a.tile_prefix, a.nparts, b);
   const uint32_t S = a.stats[4 * p + 2];
+  if (a.host_stats && b == a.tile_prefix[p] && li % per == 0 && threadIdx.x == 0) a.host_stats[4 * p + 2] = S;
   if (S == 0) return;
   const PartGPU& P = a.parts[p];
   // read before the first store, which may alias these tables as far as the compiler knows
@@ -1416,6 +1393,11 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(FrameArgs a, uint32_t 
 // larger than the others its workgroup is what the frame waits for (200
 // uneven models of up to 4,000 vertices: 151 us a frame against 141 with the
 // chain), so larger pairs come here only in even company (pairs_fit).
+__device__ __forceinline__ void publish_count(const FrameArgs& a, uint32_t p, uint32_t n) {
+  a.stats[4 * p + 2] = n;
+  if (a.host_stats) a.host_stats[4 * p + 2] = n;
+}
+
 template <uint32_t kThreads, uint32_t kV, uint32_t kT>
 __global__ __launch_bounds__(kThreads) void k_pair(FrameArgs a) {
   if (past_count(a, FC_PAIRS)) return;
@@ -1423,7 +1405,10 @@ __global__ __launch_bounds__(kThreads) void k_pair(FrameArgs a) {
   const PartGPU& R = a.parts[p];
   const uint32_t flags = load_uniform(&R.flags), vcount = load_uniform(&R.vcount), tcount = load_uniform(&R.tcount);
   const uint32_t vbase = load_uniform(&R.vbase), vmin = load_uniform(&R.vmin);
-  if (tcount == 0 || tcount > kT || vcount > kV) return;   // k_uniforms has set its count to 0
+  if (tcount == 0 || tcount > kT || vcount > kV) {
+    if (threadIdx.x == 0) publish_count(a, p, 0);
+    return;
+  }
   const FrameConst& fc = a.fc[load_uniform(&R.cam)];
   constexpr uint32_t kWaves = kThreads / 64;
   static_assert(kT % 64 == 0 && kT <= 65536 && kV <= 65536, "16-bit places");
@@ -1529,7 +1514,7 @@ __global__ __launch_bounds__(kThreads) void k_pair(FrameArgs a) {
     mn = fminf(mn, s_mn[w]);
     mx = fmaxf(mx, s_mx[w]);
   }
-  if (tid == 0) a.stats[4 * p + 2] = n;
+  if (tid == 0) publish_count(a, p, n);
   if (n == 0) return;                             // block-uniform
   float rd = mx - mn;
   if (rd == 0) rd += 0.001f;                                            // sortingTriangles.go:43-46

@@ -70,6 +70,8 @@ extern "C" t3d_status t3d_render_noalloc(t3d_ctx* c, t3d_frame* f, const t3d_ren
   pl.scratch = reinterpret_cast<uint8_t*>(c->noalloc_scratch);
   pl.scratch_bytes = T3D_NOALLOC_SCRATCH_BYTES;
   pl.scratch_room = kNoallocRoom;
+  pl.pinned_tables = c->pinned;
+  pl.pinned_stats = reinterpret_cast<uint32_t*>(c->pinned + kPinnedTables);
   pl.color = color_vertices;
   pl.depth = depth_vertices;
   pl.idx = indices;

@@ -90,10 +90,10 @@ struct t3d_frame {
   uint64_t pinned_cap = 0;
   uint32_t* pinned_stats = nullptr;
   uint64_t pinned_stats_cap = 0;
-  // a render placed in external memory (t3d_render_noalloc): pageable host staging of the tables and of the
+  // a render placed in external memory (t3d_render_noalloc): host staging of tables over kPinnedTables and of the
   // stats readback, and where the last render's stats were read back to
   std::vector<uint8_t> host_tables;
-  std::vector<uint32_t> host_stats;
+  std::vector<uint32_t> host_stats_copy;
   const uint32_t* stats_host = nullptr;
   uint8_t* tables_dev = nullptr;   // device table block of the last build (own or placed)
   bool any_normals = false;        // the last build fills the normal vertex list (Camera.RenderNormals)
@@ -142,6 +142,8 @@ struct t3d_frame {
   uint64_t total_triangles = 0;
   uint32_t max_triangles = 0, max_vertices = 0;   // of one render pair (with the device stage: of any MeshPart)
   bool small_pairs = false;        // may be drawn by one workgroup per render pair
+  bool host_uniforms = false;      // few pairs: uniforms built on the host
+  bool host_stats = false;         // survivor counts written to pinned memory by the chain's last pass
   bool ran_pairs = false;          // the last launch was (the profile's names)
   uint32_t nparts = 0;
   uint32_t total_vchunks = 0, total_tiles = 0, total_sblocks = 0;
@@ -172,7 +174,11 @@ struct t3d_ctx {
   std::map<uint64_t, std::unique_ptr<t3d::Animation>> animations;
   std::map<uint64_t, std::unique_ptr<t3d::Texture>> textures;
   std::string err;
-  t3d_tuning tuning{256, 1, 2048, 4, 1, 2, 8, 1, 0, 256, 1};
+  // Launch shape.  No graph: replaying one puts about 13 us before a frame's first kernel (512 mixed models 549 us a
+  // frame with it, 535 without; 4,096 cubes 219 and 207), and the chain's launches are enqueued faster than they run.
+  t3d_tuning tuning{256, 1, 2048, 4, 0, 2, 8, 1, 0, 256, 1};
+  // until a launch shape is set by hand or autotuned: frames of few models don't use the model stage
+  bool stage_auto = true;
   // Guards resources, the budget and err between callers and the serving
   // thread; frame builds hold it, device work runs outside it.
   std::mutex mu;
@@ -180,6 +186,8 @@ struct t3d_ctx {
   uint32_t poison = 0;
   // this device's copy of the static scratch array of t3d_render_noalloc (looked up at context creation)
   void* noalloc_scratch = nullptr;
+  // pinned staging of its tables (kPinnedTables bytes) and survivor counts (kHostUniforms pairs), used under mu
+  uint8_t* pinned = nullptr;
   // profiling (synchronous render path)
   bool profiling = false;
   struct Prof {
@@ -196,6 +204,10 @@ t3d_status fail(t3d_ctx* c, t3d_status st, const char* fmt, ...);
 // Device address of `device`'s copy of the no-allocation scratch array (t3d_noalloc.hip); the device must be
 // current.  Looked up once per device.
 hipError_t noalloc_scratch_address(int device, void** out);
+// Frames of at most this many render pairs (and per-light values) have their uniforms built on the host too.
+constexpr uint32_t kHostUniforms = 192, kHostLights = 2048;
+constexpr uint32_t kHostModels = 640;   // frames of at most so many models have their pairs built on the host
+constexpr uint64_t kPinnedTables = 64 << 10;
 // Its size: a quarter over the limit that frames are counted against.
 constexpr uint64_t kNoallocRoom = T3D_NOALLOC_SCRATCH_BYTES + T3D_NOALLOC_SCRATCH_BYTES / 4;
 t3d_status dev_alloc(t3d_ctx* c, DevBuf& b, uint64_t bytes);
@@ -219,6 +231,8 @@ struct Placement {
   uint8_t* scratch = nullptr;
   uint64_t scratch_bytes = 0;    // what a frame may count (T3D_NOALLOC_SCRATCH_BYTES)
   uint64_t scratch_room = 0;     // bytes at `scratch`
+  uint8_t* pinned_tables = nullptr;   // the context's pinned staging, kPinnedTables bytes ...
+  uint32_t* pinned_stats = nullptr;   // ... and 16 bytes for each of kHostUniforms pairs
   t3d_vertex* color = nullptr;
   t3d_vertex* depth = nullptr;
   uint32_t* idx = nullptr;
@@ -228,20 +242,23 @@ struct Placement {
 // One frame of one or more Camera.Render calls: build (host work, caller
 // holds ctx->mu), launch (enqueue on `stream`), collect (after completion).
 // With `place`, nothing is allocated: the frame's device memory is the
-// placement's, its table staging pageable host memory.
+// placement's, its table staging the context's pinned block or pageable host
+// memory.
 // With device_stage, a frame that allows it (and whose tuning asks for it) has its model-level stage run on the
 // device: frustum tests, render pairs and their slices are then known only after the frame (frame_collect).
 t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* descs, uint32_t ndesc,
                        const Placement* place = nullptr, bool device_stage = false);
 // Runs a frame built with a placement on `stream` and waits for it: table
-// upload from pageable memory, the chain (per pair for the plain form, one
+// upload, the chain (per pair for the plain form, one
 // chain for the batched form; never a graph), stats readback.  Calls no
 // allocating HIP routine.
 t3d_status frame_run_placed(t3d_ctx* c, t3d_frame* f, hipStream_t stream, int32_t exec_mode);
 // The table upload goes on `copy_stream` (may equal `stream`); `stream` waits
 // for it, runs the chain and the survivor readback, then records f->done.
+// alone: the caller waits for this frame before its next (the upload then
+// goes on `stream` itself).
 t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_t copy_stream, int32_t exec_mode,
-                        bool allow_graph, bool profile);
+                        bool allow_graph, bool profile, bool alone = false);
 void frame_collect(t3d_ctx* c, t3d_frame* f, bool profile);
 // Device bytes frame_download_range needs in `pack` for pairs [p0, p1) (0 when none survive).
 uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool normals = false);

@@ -7,6 +7,60 @@
 
 namespace t3d {
 
+// ---- a pair's uniforms, for k_uniforms and for the host's build of small frames (the same float32 functions, so the
+// same values) ----
+
+// The inverse of a model's transform, taken apart (model.go:629-630, light.go:175-189).
+struct ModelInverse {
+  V3 pos, inv_scale;
+  M4 rot;
+};
+T3D_HD ModelInverse model_inverse(const M4& model) {
+  ModelInverse r;
+  V3 s;
+  decompose(inverted(model), r.pos, s, r.rot);
+  r.inv_scale = v3(fdiv(1.0f, s.x), fdiv(1.0f, s.y), fdiv(1.0f, s.z));
+  return r;
+}
+T3D_HD V3 into_model(const ModelInverse& inv, V3 world) {
+  return add(mult_vec(inv.rot, world), hmul(inv.pos, inv.inv_scale));
+}
+// A light's values for one pair: beginModel's working position and the
+// per-model point-light skip (light.go:175-189, camera.go:1592, 1625-1629).
+T3D_HD PartLight pair_light(const PartGPU& P, const ModelInverse& inv, const LightGPU& L, uint32_t index) {
+  PartLight pl{};
+  pl.light = index;
+  pl.enabled = L.nested ? 0u : 1u;   // a volume's cell light runs from its cells only, unskipped
+  if (L.type == T3D_LIGHT_POINT) {
+    const V3 wp = v3(L.pos[0], L.pos[1], L.pos[2]);
+    const V3 w = (P.flags & PF_SKINNED) ? wp : into_model(inv, wp);
+    pl.v[0] = w.x;
+    pl.v[1] = w.y;
+    pl.v[2] = w.z;
+    if (L.range > 0 && !L.nested) {
+      const float dist = P.max_span + L.range;
+      if (dist_sq(row3(P.model), wp) > dist * dist) pl.enabled = 0;
+    }
+  }
+  return pl;
+}
+// MVP from the uploaded base (model.go:634-695), invertedCamPos (model.go:629-630), the normal list's rotation
+// (model.go:705-708) and the directional working rotation (light.go:326-330).
+T3D_HD void complete_pair(PartGPU& P, const ModelInverse& inv, const FrameConst& fc) {
+  P.mvp = mult(P.mvp, fc.vp);
+  if (fc.render_normals) {
+    V3 np, ns;
+    M4 nr;
+    decompose(mult(P.model, fc.view), np, ns, nr);
+    P.nrot = nr;
+  }
+  const V3 icp = into_model(inv, v3(fc.campos[0], fc.campos[1], fc.campos[2]));
+  P.icp[0] = icp.x;
+  P.icp[1] = icp.y;
+  P.icp[2] = icp.z;
+  if (P.flags & PF_NEED_RD) P.rd = transposed(inverted(P.rd));
+}
+
 // part_material (a material array whose entry is present), or null
 __device__ __forceinline__ const MaterialGPU* stage_material(const ModelStage& ms, const ModelGPU& M, uint32_t part) {
   if (!(M.flags & MF_MATERIALS)) return nullptr;
