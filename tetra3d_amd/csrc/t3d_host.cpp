@@ -2744,29 +2744,32 @@ void frame_collect(t3d_ctx* c, t3d_frame* f, bool profile) {
   if (profile && c->profiling) c->prof[f->ran_pairs ? "k_pair" : "k_assemble"].bytes += 300ull * total;   // 3 x (48 B colour + 48 B depth + 4 B index)
 }
 
-// Packing buffer layout: block prefix, source and destination offsets and vertex counts of np pairs, then the
-// packed colour and depth vertices and indices of `verts` corners.
-static uint64_t pack_layout_bytes(uint64_t np, uint64_t verts, bool normals) {
-  return carve_size<uint32_t>(np + 1) + 2 * carve_size<uint64_t>(np) + carve_size<uint32_t>(np) +
-         2 * carve_size<t3d_vertex>(verts) + carve_size<uint32_t>(verts) +
+// Packing buffer layout: block prefix, source and destination offsets, vertex counts and triangle sources of np pairs,
+// then the packed colour and depth vertices and indices, and the normals, of `verts` corners.  Packed triangles take no
+// room here: they go over the frame's depth keys, which nothing reads after the sort.
+static uint64_t pack_table_bytes(uint64_t np) {
+  return carve_size<uint32_t>(np + 1) + 2 * carve_size<uint64_t>(np) + 3 * carve_size<uint32_t>(np);
+}
+static uint64_t pack_layout_bytes(uint64_t np, uint64_t verts, bool lists, bool normals) {
+  return pack_table_bytes(np) + (lists ? 2 * carve_size<t3d_vertex>(verts) + carve_size<uint32_t>(verts) : 0) +
          (normals ? carve_size<t3d_vertex>(verts) : 0);
 }
 
-uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool normals) {
+uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool lists, bool normals) {
   uint64_t np = 0, verts = 0;
   for (uint32_t i = p0; i < p1; i++)
     if (f->pairs[i].survivor_count) {
       np++;
       verts += 3ull * f->pairs[i].survivor_count;
     }
-  return verts ? pack_layout_bytes(np, verts, normals) : 0;
+  return verts ? pack_layout_bytes(np, verts, lists, normals) : 0;
 }
 
 t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t stream,
                                 t3d_vertex* cv, t3d_vertex* dv, uint32_t* idx, uint32_t* tri_ids, t3d_vertex* nv,
-                                DevBuf* pack, uint64_t* pack_cap, std::string* err_out) {
-  // Every exit after the first asynchronous copy waits for the stream, so no copy is still writing into `recs`
-  // or the caller's buffers when this returns; the message goes to *err_out when given, else to ctx->err.
+                                PackBuf& pack, std::string* err_out) {
+  // Every exit after the first asynchronous copy waits for the stream, so no copy is still writing into the caller's
+  // buffers when this returns; the message goes to *err_out when given, else to ctx->err.
   bool enqueued = false;
   auto bail = [&](t3d_status st, const std::string& msg) {
     if (enqueued) (void)hipStreamSynchronize(stream);
@@ -2780,89 +2783,107 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
     if (e_ != hipSuccess) return bail(T3D_ERR_DEVICE, std::string(#expr ": ") + hipGetErrorString(e_)); \
     enqueued = true;                                                                       \
   } while (0)
-  uint64_t off = 0, toff = 0;
-  uint64_t nrec = 0;
-  for (uint32_t i = p0; i < p1; i++) nrec += f->pairs[i].survivor_count;
-  std::vector<uint4> recs(tri_ids ? std::max<uint64_t>(nrec, 1) : 0);
-  // vertices and indices: the pairs' survivors packed on the device (k_pack), then one copy per stream
-  std::vector<uint32_t> blk(1, 0), nvert;
-  std::vector<uint64_t> src, dst;
   if (nv && !f->args.out_normal) return bail(T3D_ERR_NOT_FOUND, "download: the render has no normal list (Camera.RenderNormals off)");
-  if ((cv || dv || idx || nv) && !pack) return bail(T3D_ERR_INVALID_ARGUMENT, "download: no packing buffer");
-  if (cv || dv || idx || nv)
+  uint32_t np = 0, only = 0;
+  uint64_t verts = 0;
+  for (uint32_t i = p0; i < p1; i++)
+    if (f->pairs[i].survivor_count) {
+      np++;
+      only = i;
+      verts += 3ull * f->pairs[i].survivor_count;
+    }
+  if (np == 1 && !tri_ids) {   // one pair's lists are contiguous as they are
+    const uint64_t v = f->pairs[only].vertex_offset;
+    if (cv) DL_TRY(hipMemcpyAsync(cv, f->args.out_color + 3 * v, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+    if (dv) DL_TRY(hipMemcpyAsync(dv, f->args.out_depth + 3 * v, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+    if (idx) DL_TRY(hipMemcpyAsync(idx, f->args.out_idx + v, verts * 4, hipMemcpyDeviceToHost, stream));
+    if (nv) DL_TRY(hipMemcpyAsync(nv, f->args.out_normal + 3 * v, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+  } else if (np && (cv || dv || idx || nv || tri_ids)) {
+    // the pairs' survivors packed on the device (k_pack), then one copy per stream; the tables go up in one copy from
+    // pinned memory
+    const bool lists = cv || dv || idx;
+    const uint64_t need = pack_layout_bytes(np, verts, lists, nv != nullptr);
+    if (need > pack.cap) {
+      if (err_out) return bail(T3D_ERR_INVALID_ARGUMENT, "download: packing buffer too small");   // grown by the caller
+      t3d_status st = ensure(c, pack.dev, pack.cap, need);
+      if (st) return st;
+    }
+    const uint64_t tbytes = pack_table_bytes(np);
+    if (tbytes > pack.host_cap) {
+      if (pack.host) (void)hipHostFree(pack.host);
+      pack.host = nullptr;
+      pack.host_cap = 0;
+      const uint64_t cap = align_up(tbytes + tbytes / 4, 1 << 16);
+      DL_TRY(hipHostMalloc(&pack.host, cap, hipHostMallocDefault));
+      pack.host_cap = cap;
+    }
+    Carve pc{reinterpret_cast<uint8_t*>(pack.dev.ptr)};
+    Carve hc{reinterpret_cast<uint8_t*>(pack.host)};
+    PackArgs pa{};
+    uint32_t* h_blk = hc.take<uint32_t>(np + 1);
+    uint64_t* h_src = hc.take<uint64_t>(np);
+    uint64_t* h_dst = hc.take<uint64_t>(np);
+    uint32_t* h_nv = hc.take<uint32_t>(np);
+    uint32_t* h_tsrc = hc.take<uint32_t>(np);
+    uint32_t* h_tfirst = hc.take<uint32_t>(np);
+    pa.blk_prefix = pc.take<uint32_t>(np + 1);
+    pa.src = pc.take<uint64_t>(np);
+    pa.dst = pc.take<uint64_t>(np);
+    pa.nvert = pc.take<uint32_t>(np);
+    pa.tsrc = pc.take<uint32_t>(np);
+    pa.tfirst = pc.take<uint32_t>(np);
+    uint64_t off = 0;
+    uint32_t k = 0, blocks = 0;
     for (uint32_t i = p0; i < p1; i++) {
       const uint64_t n = 3ull * f->pairs[i].survivor_count;
       if (!n) continue;
-      src.push_back(f->pairs[i].vertex_offset);
-      dst.push_back(off);
-      nvert.push_back((uint32_t)n);
-      blk.push_back(blk.back() + (uint32_t)((3 * n + 255) / 256));   // 3 float4 per vertex, 256 to a block
+      h_blk[k] = blocks;
+      h_src[k] = f->pairs[i].vertex_offset;
+      h_dst[k] = off;
+      h_nv[k] = (uint32_t)n;
+      h_tsrc[k] = f->pair_tbase[i];
+      h_tfirst[k] = f->part_first_tri[i];
+      blocks += (uint32_t)((3 * n + 255) / 256);   // 3 float4 per vertex, 256 to a block
       off += n;
+      k++;
     }
-  if (off) {
-    const uint32_t np = (uint32_t)nvert.size();
-    const uint64_t need = pack_layout_bytes(np, off, nv != nullptr);
-    if (need > *pack_cap) {
-      if (err_out) return bail(T3D_ERR_INVALID_ARGUMENT, "download: packing buffer too small");   // grown by the caller
-      t3d_status st = ensure(c, *pack, *pack_cap, need);
-      if (st) return st;
-    }
-    Carve pc{reinterpret_cast<uint8_t*>(pack->ptr)};
-    PackArgs pa{};
-    uint32_t* d_blk = pc.take<uint32_t>(np + 1);
-    uint64_t* d_src = pc.take<uint64_t>(np);
-    uint64_t* d_dst = pc.take<uint64_t>(np);
-    uint32_t* d_nv = pc.take<uint32_t>(np);
-    DL_TRY(hipMemcpyAsync(d_blk, blk.data(), 4ull * (np + 1), hipMemcpyHostToDevice, stream));
-    DL_TRY(hipMemcpyAsync(d_src, src.data(), 8ull * np, hipMemcpyHostToDevice, stream));
-    DL_TRY(hipMemcpyAsync(d_dst, dst.data(), 8ull * np, hipMemcpyHostToDevice, stream));
-    DL_TRY(hipMemcpyAsync(d_nv, nvert.data(), 4ull * np, hipMemcpyHostToDevice, stream));
-    pa.blk_prefix = d_blk;
-    pa.src = d_src;
-    pa.dst = d_dst;
-    pa.nvert = d_nv;
+    h_blk[np] = blocks;
+    DL_TRY(hipMemcpyAsync(pack.dev.ptr, pack.host, tbytes, hipMemcpyHostToDevice, stream));
     pa.npairs = np;
     pa.color = f->args.out_color;
     pa.depth = f->args.out_depth;
     pa.idx = f->args.out_idx;
-    float4* pcol = reinterpret_cast<float4*>(pc.take<t3d_vertex>(off));
-    float4* pdep = reinterpret_cast<float4*>(pc.take<t3d_vertex>(off));
-    uint32_t* pidx = pc.take<uint32_t>(off);
-    float4* pnrm = nv ? reinterpret_cast<float4*>(pc.take<t3d_vertex>(off)) : nullptr;
+    float4* pcol = lists ? reinterpret_cast<float4*>(pc.take<t3d_vertex>(verts)) : nullptr;
+    float4* pdep = lists ? reinterpret_cast<float4*>(pc.take<t3d_vertex>(verts)) : nullptr;
+    uint32_t* pidx = lists ? pc.take<uint32_t>(verts) : nullptr;
+    float4* pnrm = nv ? reinterpret_cast<float4*>(pc.take<t3d_vertex>(verts)) : nullptr;
+    uint32_t* ptri = tri_ids ? reinterpret_cast<uint32_t*>(f->args.key) + f->pair_tbase[p0] : nullptr;
     pa.pcolor = cv ? pcol : nullptr;   // only the arrays asked for are packed
     pa.pdepth = dv ? pdep : nullptr;
     pa.pidx = idx ? pidx : nullptr;
     pa.normal = f->args.out_normal;
     pa.pnormal = pnrm;
-    DL_TRY(launch_pack(pa, blk.back(), stream));
-    if (cv) DL_TRY(hipMemcpyAsync(cv, pcol, off * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
-    if (dv) DL_TRY(hipMemcpyAsync(dv, pdep, off * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
-    if (idx) DL_TRY(hipMemcpyAsync(idx, pidx, off * 4, hipMemcpyDeviceToHost, stream));
-    if (nv) DL_TRY(hipMemcpyAsync(nv, pnrm, off * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+    pa.tri_vo = f->args.tri_vo;
+    pa.ptri = ptri;
+    DL_TRY(launch_pack(pa, blocks, stream));
+    if (cv) DL_TRY(hipMemcpyAsync(cv, pcol, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+    if (dv) DL_TRY(hipMemcpyAsync(dv, pdep, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+    if (idx) DL_TRY(hipMemcpyAsync(idx, pidx, verts * 4, hipMemcpyDeviceToHost, stream));
+    if (nv) DL_TRY(hipMemcpyAsync(nv, pnrm, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
+    if (tri_ids) DL_TRY(hipMemcpyAsync(tri_ids, ptri, verts / 3 * 4, hipMemcpyDeviceToHost, stream));
   }
-  if (tri_ids)
-    for (uint32_t i = p0; i < p1; i++) {
-      const auto& p = f->pairs[i];
-      if (!p.survivor_count) continue;
-      DL_TRY(hipMemcpyAsync(recs.data() + toff, f->args.tri_vo + f->pair_tbase[i], 16ull * p.survivor_count,
-                            hipMemcpyDeviceToHost, stream));
-      toff += p.survivor_count;
-    }
-  {
-    hipError_t e = hipStreamSynchronize(stream);
-    enqueued = false;
-    if (e != hipSuccess) return bail(T3D_ERR_DEVICE, std::string("download: ") + hipGetErrorString(e));
-  }
+  const hipError_t e = hipStreamSynchronize(stream);
+  enqueued = false;
+  if (e != hipSuccess) return bail(T3D_ERR_DEVICE, std::string("download: ") + hipGetErrorString(e));
 #undef DL_TRY
-  if (tri_ids) {
-    toff = 0;
-    for (uint32_t i = p0; i < p1; i++) {
-      const auto& p = f->pairs[i];
-      for (uint32_t k = 0; k < p.survivor_count; k++) tri_ids[toff + k] = recs[toff + k].w + f->part_first_tri[i];
-      toff += p.survivor_count;
-    }
-  }
   return T3D_OK;
+}
+
+void pack_release(t3d_ctx* c, PackBuf& pack) {
+  dev_free(c, pack.dev);
+  if (pack.host) (void)hipHostFree(pack.host);
+  pack.host = nullptr;
+  pack.cap = pack.host_cap = 0;
 }
 
 uint64_t estimate_job_bytes(t3d_ctx* c, const t3d_render_desc* desc) {
@@ -2895,12 +2916,12 @@ void frame_release(t3d_ctx* c, t3d_frame* f) {
   dev_free(c, f->tables);
   dev_free(c, f->scratch);
   dev_free(c, f->outputs);
-  dev_free(c, f->pack);
+  pack_release(c, f->pack);
   dev_free(c, f->raster_buf);
   dev_free(c, f->raster_buf2);
   dev_free(c, f->raster_buf3);
   dev_free(c, f->images);
-  f->tables_cap = f->scratch_cap = f->outputs_cap = f->pack_cap = 0;
+  f->tables_cap = f->scratch_cap = f->outputs_cap = 0;
   f->raster_cap = f->raster_cap2 = f->raster_cap3 = f->images_cap = 0;
   f->image_color = f->image_depth = nullptr;
   if (f->pinned) (void)hipHostFree(f->pinned);
@@ -3011,7 +3032,7 @@ t3d_status t3d_frame_download(t3d_ctx* c, const t3d_frame* f, t3d_vertex* cv, t3
   (void)hipSetDevice(c->device);
   t3d_frame* fm = const_cast<t3d_frame*>(f);   // the staging buffer only; the frame's results are untouched
   return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, cv, dv, idx, nullptr, nullptr,
-                              &fm->pack, &fm->pack_cap);
+                              fm->pack);
 }
 
 t3d_status t3d_frame_download_normals(t3d_ctx* c, const t3d_frame* f, t3d_vertex* nv) {
@@ -3021,7 +3042,7 @@ t3d_status t3d_frame_download_normals(t3d_ctx* c, const t3d_frame* f, t3d_vertex
   (void)hipSetDevice(c->device);
   t3d_frame* fm = const_cast<t3d_frame*>(f);
   return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, nullptr, nullptr, nullptr, nullptr, nv,
-                              &fm->pack, &fm->pack_cap);
+                              fm->pack);
 }
 
 t3d_status t3d_frame_download_triangles(t3d_ctx* c, const t3d_frame* f, uint32_t* ids) {
@@ -3029,7 +3050,9 @@ t3d_status t3d_frame_download_triangles(t3d_ctx* c, const t3d_frame* f, uint32_t
   std::lock_guard<std::mutex> lk(c->mu);
   if (f->inflight) return fail(c, T3D_ERR_NOT_READY, "frame_download: render in flight (t3d_frame_wait first)");
   (void)hipSetDevice(c->device);
-  return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, nullptr, nullptr, nullptr, ids, nullptr);
+  t3d_frame* fm = const_cast<t3d_frame*>(f);
+  return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, nullptr, nullptr, nullptr, ids, nullptr,
+                              fm->pack);
 }
 
 t3d_status t3d_debug_model_spheres(const t3d_mat4* transforms, const float* dims, const uint8_t* skinned, uint32_t n,

@@ -342,13 +342,16 @@ struct FrameArgs {
 
 // Packing of a range of render pairs' survivors for download: pair j of the
 // range copies its first nvert[j] output vertices (and indices) from vertex
-// src[j] of the frame outputs to vertex dst[j] of the packed arrays; blocks
+// src[j] of the frame outputs to vertex dst[j] of the packed arrays, and the
+// mesh triangles of its slots (tri_vo from tsrc[j] on, plus tfirst[j]); blocks
 // [blk_prefix[j], blk_prefix[j+1]) cover its 3 * nvert float4 words, 256 each.
 struct PackArgs {
   const uint32_t* blk_prefix;   // [npairs + 1]
   const uint64_t* src;          // [npairs]
   const uint64_t* dst;          // [npairs]
   const uint32_t* nvert;        // [npairs]
+  const uint32_t* tsrc;         // [npairs]
+  const uint32_t* tfirst;       // [npairs]
   uint32_t npairs, pad;
   const float4* color;          // frame outputs, t3d_vertex as 3 float4
   const float4* depth;
@@ -358,6 +361,8 @@ struct PackArgs {
   uint32_t* pidx;
   const float4* normal;         // frame normal vertices and their packed copy (both null: none packed)
   float4* pnormal;
+  const uint4* tri_vo;          // slot records and the packed triangles (both null: none packed)
+  uint32_t* ptri;
 };
 
 // Raster sink (t3d_raster.hip): the state a flush's draw reads (camera.go:1829-2048).

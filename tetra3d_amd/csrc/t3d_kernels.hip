@@ -1642,6 +1642,7 @@ __global__ __launch_bounds__(256) void k_pack(PackArgs a) {
   if (a.pdepth) a.pdepth[3 * d + e] = a.depth[3 * s + e];
   if (a.pnormal) a.pnormal[3 * d + e] = a.normal[3 * s + e];
   if (a.pidx && e < n) a.pidx[d + e] = a.idx[s + e];
+  if (a.ptri && e < n / 3) a.ptri[d / 3 + e] = a.tri_vo[a.tsrc[lo] + e].w + a.tfirst[lo];
 }
 
 // Dynamic batches (camera.go:2075-2099): the render pairs of one flush write

@@ -21,6 +21,14 @@ struct DevBuf {
   uint64_t bytes = 0;
 };
 
+// Download staging: the packed survivors on the device (its size accounted), the pairs' tables in pinned memory.
+struct PackBuf {
+  DevBuf dev;
+  uint64_t cap = 0;
+  void* host = nullptr;
+  uint64_t host_cap = 0;
+};
+
 // A resident mesh (mesh.go:260-302) and its MeshPart ranges.
 struct Mesh {
   uint64_t handle = 0;
@@ -84,8 +92,7 @@ struct t3d_frame {
   uint64_t tables_cap = 0, scratch_cap = 0, outputs_cap = 0;
   // download staging of t3d_frame_download: the survivors packed back to back, so the copy to the host is one
   // transfer per stream (grown on demand, kept with the frame)
-  t3d::DevBuf pack;
-  uint64_t pack_cap = 0;
+  t3d::PackBuf pack;
   void* pinned = nullptr;          // host staging of the tables
   uint64_t pinned_cap = 0;
   uint32_t* pinned_stats = nullptr;
@@ -217,7 +224,7 @@ void dev_free(t3d_ctx* c, DevBuf& b);
 void frame_release(t3d_ctx* c, t3d_frame* f);
 // Device bytes a frame holds between renders (tables, scratch, outputs, download packing).
 inline uint64_t frame_capacity(const t3d_frame* f) {
-  return f->tables.bytes + f->scratch.bytes + f->outputs.bytes + f->pack.bytes + f->raster_buf.bytes +
+  return f->tables.bytes + f->scratch.bytes + f->outputs.bytes + f->pack.dev.bytes + f->raster_buf.bytes +
          f->raster_buf2.bytes + f->raster_buf3.bytes + f->images.bytes;
 }
 
@@ -261,16 +268,16 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
                         bool allow_graph, bool profile, bool alone = false);
 void frame_collect(t3d_ctx* c, t3d_frame* f, bool profile);
 // Device bytes frame_download_range needs in `pack` for pairs [p0, p1) (0 when none survive).
-uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool normals = false);
-// Copy pairs [p0, p1) of a frame, concatenated, to host memory (any output may be null).  Vertices and
-// indices are first packed on the device into `pack`, so they cross to the host in one copy per stream.
-// Without err_out, `pack` is grown here when too small (needs ctx->mu) and errors go to ctx->err; with it,
-// the caller has grown `pack` to download_pack_bytes already and the message goes to *err_out (no ctx state
-// is touched).  Returns only after every copy it enqueued has finished.
+uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool lists, bool normals);
+// Copy pairs [p0, p1) of a frame, concatenated, to host memory (any output may be null): vertices, indices and
+// triangles packed on the device into `pack`, so that they cross to the host in one copy per stream (a single pair's
+// lists are copied as they lie).  Without err_out, `pack` is grown here when too small (needs ctx->mu) and errors go
+// to ctx->err; with it, the caller has grown `pack` to download_pack_bytes already and the message goes to *err_out
+// (no ctx state is touched).  Returns only after every copy it enqueued has finished.
 t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t stream,
                                 t3d_vertex* cv, t3d_vertex* dv, uint32_t* idx, uint32_t* tri_ids, t3d_vertex* nv,
-                                t3d::DevBuf* pack = nullptr, uint64_t* pack_cap = nullptr,
-                                std::string* err_out = nullptr);
+                                PackBuf& pack, std::string* err_out = nullptr);
+void pack_release(t3d_ctx* c, PackBuf& pack);
 // Frame memory a job may need (scratch + outputs + tables), before frustum culling.
 uint64_t estimate_job_bytes(t3d_ctx* c, const t3d_render_desc* desc);
 

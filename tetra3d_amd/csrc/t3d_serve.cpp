@@ -109,8 +109,7 @@ struct t3d_server {
   std::mutex dl_mu;
   // download packing buffer of t3d_job_download, shared by all jobs: grown under dl_mu and ctx->mu, its size
   // readable under mu (counted with the frames the server holds)
-  t3d::DevBuf pack;
-  uint64_t pack_cap = 0;
+  t3d::PackBuf pack;
   std::atomic<uint64_t> pack_bytes{0};
   uint64_t wakeups = 0;                  // slot completions signalled from the slot streams
   std::thread worker;
@@ -587,7 +586,7 @@ t3d_status t3d_server_destroy(t3d_server* s) {
     }
     (void)hipStreamSynchronize(s->dl_stream);
     (void)hipStreamDestroy(s->dl_stream);
-    dev_free(s->ctx, s->pack);
+    pack_release(s->ctx, s->pack);
     for (t3d_frame* f : frames) {
       frame_release(s->ctx, f);
       delete f;
@@ -731,17 +730,16 @@ t3d_status job_download(t3d_server* s, uint64_t job, t3d_pair_result* pairs, t3d
     (void)hipSetDevice(s->ctx->device);
     std::lock_guard<std::mutex> dl(s->dl_mu);   // one download at a time on the download stream
     // the server's packing buffer: grown under ctx->mu (memory accounting), used under dl_mu only
-    const uint64_t need = (cv || dv || idx || nv) ? download_pack_bytes(f, p0, p1, nv != nullptr) : 0;
-    if (need > s->pack_cap) {
+    const uint64_t need = download_pack_bytes(f, p0, p1, cv || dv || idx, nv != nullptr);
+    if (need > s->pack.cap) {
       std::lock_guard<std::mutex> cl(s->ctx->mu);
-      st = ensure(s->ctx, s->pack, s->pack_cap, need);
-      s->pack_bytes = s->pack.bytes;
+      st = ensure(s->ctx, s->pack.dev, s->pack.cap, need);
+      s->pack_bytes = s->pack.dev.bytes;
     }
     if (!st) {
       // errors are reported into a local string (the worker may be writing ctx->err under ctx->mu)
       std::string err;
-      st = frame_download_range(s->ctx, f, p0, p1, s->dl_stream, cv, dv, idx, tri_ids, nv, &s->pack, &s->pack_cap,
-                                &err);
+      st = frame_download_range(s->ctx, f, p0, p1, s->dl_stream, cv, dv, idx, tri_ids, nv, s->pack, &err);
       if (st) {
         std::lock_guard<std::mutex> cl(s->ctx->mu);
         s->ctx->err = err;
