@@ -1,0 +1,41 @@
+"""Frames at and one past the model counts where the pairs stop being built on the host, the uniforms stop coming from
+it and the tile tables start, on a context whose tuning nobody has set, against the oracle bit for bit; and their
+lists downloaded with and without the triangle ids."""
+import numpy as np
+import pytest
+
+from tetra3d_amd import workloads as W
+from tetra3d_amd.runtime import Context
+from tetra3d_amd.scene import Camera, Model, Scene
+from tests.parity import compare_frames
+from tests.test_gpu_pairs import _mesh
+
+
+@pytest.fixture(scope="module")
+def fresh_ctx():
+    with Context(0) as c:
+        c.poison_outputs(0x7FC0DEAD)
+        yield c
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("large", [False, True], ids=["small", "large"])
+@pytest.mark.parametrize("count", [1, 4, 5, 16, 17, 192, 193, 640, 641])
+def test_model_counts(fresh_ctx, oracle, count, large):
+    r = np.random.default_rng(count)
+    meshes = [_mesh(64, 60, 1), _mesh(300, 500, 2), _mesh(3000, 5000, 3)][: 3 if large else 2]
+    models = []
+    for i in range(count):
+        m = Model("m%d" % i, meshes[-1 if i % 40 == 0 else i % 2])
+        m.set_local_position(*(r.uniform(-4, 4, 3) - [0, 0, 6]))
+        m.color = np.array([*r.random(3), 0.5 if i % 11 == 3 else 1.0], dtype=np.float32)
+        m.shadeless = i % 7 == 5
+        models.append(m)
+    W._skin(models[count // 2], W.SplitMix64(5), bones=8)
+    wl = W.Workload("few", Camera("camera", 800, 450), Scene("few", W._world(0.2)), W.icosphere_scene().lights, models)
+    print("few models", count, large, flush=True)
+    got, want = fresh_ctx.render_workload(wl), oracle.render_workload(wl)
+    compare_frames(got, want)
+    lists = fresh_ctx.download(triangles=False)
+    for name in ("color", "depth"):
+        np.testing.assert_array_equal(getattr(lists, name).view(np.uint32), getattr(want, name).view(np.uint32))
