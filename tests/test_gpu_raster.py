@@ -122,3 +122,20 @@ def test_mixed_512_full_size(gpu_ctx, oracle):
     gc, gd, oc, od = _both(gpu_ctx, oracle, wl.camera, wl.scene, wl.lights, wl.models)
     _same(gc, gd, oc, od, "mixed_512")
     assert np.count_nonzero(gd[..., 3]) > 100000
+
+
+@pytest.mark.parametrize("kind", ["opaque", "half", "hidden"])
+@pytest.mark.parametrize("layers", [1, 63, 64, 65, 255, 256, 257, 700])
+def test_runs_of_one_flush(gpu_ctx, oracle, layers, kind):
+    """Every pixel of a rectangle holds one fragment of each layer of a mesh: runs that end inside, at and past a
+    wavefront and a workgroup of the fragment passes; alone, blended, and behind an earlier flush."""
+    r = np.random.default_rng(layers)
+    m = R._flat(R._square(100, 40, 107, 45) * layers, z=-5, color=(0.7, 0.5, 0.3, 0.5 if kind == "half" else 1.0))
+    m.mesh.positions[:, 2] = np.repeat(r.uniform(-2, 2, layers).astype(np.float32), 6)
+    models = [m]
+    if kind == "hidden":
+        models.append(R._flat(R._square(98, 38, 104, 47), z=-1, color=(0, 1, 0, 1)))
+    w = R._world(fog_on=True, fog_color=np.array([0.25, 0.5, 1, 1], dtype=np.float32),
+                 fog_range=np.array([0.0, 0.5], dtype=np.float32))
+    print("raster runs", layers, kind, flush=True)
+    _same(*_both(gpu_ctx, oracle, R.ortho_camera(), Scene("s", w), [], models), "%d layers, %s" % (layers, kind))
