@@ -243,17 +243,19 @@ __device__ __forceinline__ uint32_t pair_of(const RArgs& a, uint32_t t) {
   return lo;
 }
 
-__device__ void load_tri(const RArgs& a, uint32_t t, STri& s) {
-  const RasterPair rp = a.pairs[pair_of(a, t)];
-  const uint64_t v0 = rp.vertex + 3ull * (t - rp.tri0);
+__device__ __forceinline__ void load_corners(const RArgs& a, uint64_t v0, STri& s) {
   for (int k = 0; k < 3; k++) {
-    const float4 p = a.color[3 * (v0 + k) + 0];
-    const float4 c = a.color[3 * (v0 + k) + 1];
-    const float4 q = a.color[3 * (v0 + k) + 2];
+    const float4 p = a.color[3 * (v0 + k)];
     s.x[k] = p.x;
     s.y[k] = p.y;
     s.sx[k] = p.z;
     s.sy[k] = p.w;
+  }
+}
+__device__ __forceinline__ void load_attributes(const RArgs& a, uint64_t v0, STri& s) {
+  for (int k = 0; k < 3; k++) {
+    const float4 c = a.color[3 * (v0 + k) + 1];
+    const float4 q = a.color[3 * (v0 + k) + 2];
     s.r[k] = c.x;
     s.g[k] = c.y;
     s.b[k] = c.z;
@@ -261,7 +263,6 @@ __device__ void load_tri(const RArgs& a, uint32_t t, STri& s) {
     s.c0[k] = q.x;
     s.dz[k] = a.rf.render_depth ? a.depth[3 * (v0 + k) + 1].x : 0.0f;
   }
-  s.flush = rp.flush;
 }
 
 // ---- shading ---------------------------------------------------------------------
@@ -321,19 +322,26 @@ __device__ __forceinline__ void base3d_fog(const RasterFrame& rf, float d, float
 
 // ---- fragments -------------------------------------------------------------------
 
-// per drawn triangle: its record and the number of pixels of its box (its fragment slots)
+// per drawn triangle: the number of pixels of its box (its fragment slots) and, if it has any, its record. One
+// without pixels owns no slot, so nothing reads its record: it is not stored, nor the attributes for it read.
 __global__ __launch_bounds__(256) void k_rsetup(RArgs a) {
   const uint32_t t = blockIdx.x * 256 + threadIdx.x;
   if (t > a.ntri) return;
   uint64_t n = 0;
   if (t < a.ntri) {
     STri s;
-    load_tri(a, t, s);
-    if (setup(s, a.rf.width, a.rf.height)) n = (uint64_t)(s.bx1 - s.bx0 + 1) * (uint64_t)(s.by1 - s.by0 + 1);
-    s.pad[0] = s.pad[1] = s.pad[2] = 0;
-    const float4* src = reinterpret_cast<const float4*>(&s);
-    float4* dst = reinterpret_cast<float4*>(a.recs + t);
-    for (int k = 0; k < 10; k++) dst[k] = src[k];
+    const RasterPair rp = a.pairs[pair_of(a, t)];
+    const uint64_t v0 = rp.vertex + 3ull * (t - rp.tri0);
+    load_corners(a, v0, s);
+    if (setup(s, a.rf.width, a.rf.height)) {
+      n = (uint64_t)(s.bx1 - s.bx0 + 1) * (uint64_t)(s.by1 - s.by0 + 1);
+      load_attributes(a, v0, s);
+      s.flush = rp.flush;
+      s.pad[0] = s.pad[1] = s.pad[2] = 0;
+      const float4* src = reinterpret_cast<const float4*>(&s);
+      float4* dst = reinterpret_cast<float4*>(a.recs + t);
+      for (int k = 0; k < 10; k++) dst[k] = src[k];
+    }
   }
   a.counts[t] = n;   // counts[ntri] = 0 closes the scan
 }
