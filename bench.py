@@ -4,8 +4,8 @@ cull, 512-bin depth sort, ebiten vertex assembly) on one MI355X.
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload mixed]
 
 A step is one Camera.Render frame of the workload, in the batched form (one
-launch chain for all render pairs, replayed from a HIP graph), with all
-meshes, bone palettes and light volumes resident in HBM before timing.
+launch chain for all render pairs), with all meshes, bone palettes and light
+volumes resident in HBM before timing.
 Prints one JSON line.
 """
 import argparse
@@ -590,7 +590,7 @@ def main():
         "data": "synthetic (seeded SplitMix64 scene, seed 0x7e7a3d)",
         "config": {"workload": wname, "description": wdesc, "triangles_per_frame": tris,
                    "vertices_per_frame": wl.vertex_count, "render_pairs": len(pairs), "drawn_triangles": survivors,
-                   "exec": "batched, HIP graph, two frames in flight", "tuning": tuning},
+                   "exec": "batched, two frames in flight", "tuning": tuning},
         "latency_ms": {"p50": p50, "p99": p99, "mean": sync_ms,
                        "note": "synchronous frames: submit -> outputs complete in HBM",
                        "with_d2h_p50": d2h50, "with_d2h_p99": d2h99,

@@ -82,7 +82,7 @@ enum { T3D_LIGHT_AMBIENT = 0, T3D_LIGHT_POINT = 1, T3D_LIGHT_DIRECTIONAL = 2, T3
 /* Execution forms of t3d_render */
 enum {
   T3D_EXEC_PLAIN = 0,   /* one kernel chain per render pair, like one ProcessVertices+flush each */
-  T3D_EXEC_BATCHED = 1  /* all render pairs of the frame in one launch chain, replayed from a HIP graph */
+  T3D_EXEC_BATCHED = 1  /* all render pairs of the frame in one launch chain */
 };
 
 /* Matrix4 (matrix.go:9-10): m[row][col], row vectors, translation in row 3. */
