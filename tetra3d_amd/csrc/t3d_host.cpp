@@ -710,9 +710,16 @@ t3d_status t3d_ctx_create(int32_t device, uint64_t hbm_budget_bytes, t3d_ctx** o
     delete c;
     return T3D_ERR_DEVICE;
   }
+  if (hipStreamCreateWithFlags(&c->large_stream, hipStreamNonBlocking) != hipSuccess) {
+    (void)hipStreamDestroy(c->stream);
+    (void)hipStreamDestroy(c->copy_stream);
+    delete c;
+    return T3D_ERR_DEVICE;
+  }
   if (hipHostMalloc((void**)&c->pinned, kPinnedTables + 16ull * kHostUniforms, hipHostMallocDefault) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     (void)hipStreamDestroy(c->copy_stream);
+    (void)hipStreamDestroy(c->large_stream);
     delete c;
     return T3D_ERR_DEVICE;
   }
@@ -720,6 +727,7 @@ t3d_status t3d_ctx_create(int32_t device, uint64_t hbm_budget_bytes, t3d_ctx** o
   if (noalloc_scratch_address(device, &c->noalloc_scratch) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     (void)hipStreamDestroy(c->copy_stream);
+    (void)hipStreamDestroy(c->large_stream);
     (void)hipHostFree(c->pinned);
     delete c;
     return T3D_ERR_DEVICE;
@@ -733,6 +741,7 @@ t3d_status t3d_ctx_destroy(t3d_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   (void)hipStreamSynchronize(c->copy_stream);
+  (void)hipStreamSynchronize(c->large_stream);
   for (auto& kv : c->meshes) dev_free(c, kv.second->buf);
   for (auto& kv : c->volumes) {
     dev_free(c, kv.second->buf);
@@ -740,6 +749,7 @@ t3d_status t3d_ctx_destroy(t3d_ctx* c) {
   }
   (void)hipStreamDestroy(c->stream);
   (void)hipStreamDestroy(c->copy_stream);
+  (void)hipStreamDestroy(c->large_stream);
   (void)hipHostFree(c->pinned);
   delete c;
   return T3D_OK;
@@ -1051,6 +1061,7 @@ t3d_status t3d_frame_destroy(t3d_ctx* c, t3d_frame* f) {
   std::lock_guard<std::mutex> lk(c->mu);
   if (f->stream) (void)hipStreamSynchronize(f->stream);
   (void)hipStreamSynchronize(c->stream);
+  (void)hipStreamSynchronize(c->large_stream);
   frame_release(c, f);
   if (f->stream) (void)hipStreamDestroy(f->stream);
   delete f;
@@ -1283,11 +1294,6 @@ t3d_status validate_desc(t3d_ctx* c, const t3d_render_desc* desc) {
 
 namespace {
 
-// Whether the model-level stage of these descriptors can run on the device:
-// the tuning asks for it, no model is dynamically batched, every camera has
-// RenderDepth on (its solids then keep model order), and no drawable model is
-// at a NaN distance from its camera (the transparents' comparator is then a
-// strict weak order, so a stable sort by it is Go's SliceStable's order).
 // A frame of at most kHostModels models and MeshParts: its pairs are built on the host, at about 0.1 us each, where the
 // stage's two kernels take 15 us and more on the device, and the readback of what they built another ten: 500 cubes
 // 80 us a frame and 96, 300 uneven models 345 and 358, 512 of them 535 and 554.  Past that the host's part is longer
@@ -1306,6 +1312,12 @@ bool few_models(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t 
   return pairs <= kHostModels;
 }
 
+// Whether the model-level stage of these descriptors can run on the device:
+// the tuning asks for it, no model is dynamically batched, every camera has
+// RenderDepth on (its solids then keep model order), and no drawable model is
+// at a NaN distance from its camera (the transparents' comparator is then a
+// strict weak order, so a stable sort by it is Go's SliceStable's order).  Until a shape is
+// set or autotuned, a frame of few models is left to the host.
 bool stage_applies(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
   if (!c->tuning.model_stage) return false;
   if (c->stage_auto && few_models(c, descs, ndesc)) return false;
@@ -2968,7 +2980,12 @@ t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, 
     f->device_stage = false;
     return st;
   }
-  st = frame_launch(c, f, f->stream ? f->stream : c->stream, c->copy_stream, desc->exec_mode, true, true, alone);
+  // Frames in flight together overlap on the device, but not large ones: each holds more vertex records than the
+  // memory-side cache keeps of two, so side by side they push out each other's and the assemblies wait for HBM (512
+  // uneven models, two frames in flight: 471 us a frame one after the other, 497 side by side).
+  hipStream_t stream = f->stream ? f->stream : c->stream;
+  if (f->args.touch_records) stream = c->large_stream;
+  st = frame_launch(c, f, stream, c->copy_stream, desc->exec_mode, true, true, alone);
   if (st) return st;
   f->submitted = wall0;
   f->inflight = true;
