@@ -39,3 +39,33 @@ def test_model_counts(fresh_ctx, oracle, count, large):
     lists = fresh_ctx.download(triangles=False)
     for name in ("color", "depth"):
         np.testing.assert_array_equal(getattr(lists, name).view(np.uint32), getattr(want, name).view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [799, 801])
+def test_large_frames_in_flight(fresh_ctx, oracle, count):
+    """Two frames of just under and just over 2.4 million vertices in flight, which overlap on the device or run in
+    turn: each equals the oracle's."""
+    mesh = _mesh(3000, 5000, 3)
+    r = np.random.default_rng(count)
+    models = []
+    for i in range(count):
+        m = Model("m%d" % i, mesh)
+        m.set_local_position(*(r.uniform(-4, 4, 3) - [0, 0, 6]))
+        models.append(m)
+    lights = W.icosphere_scene().lights
+    frames = [fresh_ctx.frame, fresh_ctx.new_frame()]
+    wls = []
+    for k in range(2):
+        cam = Camera("camera%d" % k, 800, 450)
+        cam.set_local_position(0.3 * k, 0, 0)
+        wls.append(W.Workload("large", cam, Scene("large", W._world(0.2)), lights, models))
+    fresh_ctx.prepare(wls[0])
+    inputs = [fresh_ctx.inputs(w.camera, w.scene, w.lights, w.models) for w in wls]
+    print("large frames in flight", count, flush=True)
+    for _ in range(2):
+        for f, inp in zip(frames, inputs):
+            fresh_ctx.render_async(inp, f)
+    for f, w in zip(frames, wls):
+        fresh_ctx.wait(f)
+        compare_frames(fresh_ctx.download(frame=f), oracle.render_workload(w))
