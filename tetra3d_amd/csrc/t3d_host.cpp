@@ -710,16 +710,9 @@ t3d_status t3d_ctx_create(int32_t device, uint64_t hbm_budget_bytes, t3d_ctx** o
     delete c;
     return T3D_ERR_DEVICE;
   }
-  if (hipStreamCreateWithFlags(&c->large_stream, hipStreamNonBlocking) != hipSuccess) {
-    (void)hipStreamDestroy(c->stream);
-    (void)hipStreamDestroy(c->copy_stream);
-    delete c;
-    return T3D_ERR_DEVICE;
-  }
   if (hipHostMalloc((void**)&c->pinned, kPinnedTables + 16ull * kHostUniforms, hipHostMallocDefault) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     (void)hipStreamDestroy(c->copy_stream);
-    (void)hipStreamDestroy(c->large_stream);
     delete c;
     return T3D_ERR_DEVICE;
   }
@@ -727,7 +720,6 @@ t3d_status t3d_ctx_create(int32_t device, uint64_t hbm_budget_bytes, t3d_ctx** o
   if (noalloc_scratch_address(device, &c->noalloc_scratch) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
     (void)hipStreamDestroy(c->copy_stream);
-    (void)hipStreamDestroy(c->large_stream);
     (void)hipHostFree(c->pinned);
     delete c;
     return T3D_ERR_DEVICE;
@@ -741,7 +733,6 @@ t3d_status t3d_ctx_destroy(t3d_ctx* c) {
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
   (void)hipStreamSynchronize(c->copy_stream);
-  (void)hipStreamSynchronize(c->large_stream);
   for (auto& kv : c->meshes) dev_free(c, kv.second->buf);
   for (auto& kv : c->volumes) {
     dev_free(c, kv.second->buf);
@@ -749,7 +740,6 @@ t3d_status t3d_ctx_destroy(t3d_ctx* c) {
   }
   (void)hipStreamDestroy(c->stream);
   (void)hipStreamDestroy(c->copy_stream);
-  (void)hipStreamDestroy(c->large_stream);
   (void)hipHostFree(c->pinned);
   delete c;
   return T3D_OK;
@@ -1061,7 +1051,6 @@ t3d_status t3d_frame_destroy(t3d_ctx* c, t3d_frame* f) {
   std::lock_guard<std::mutex> lk(c->mu);
   if (f->stream) (void)hipStreamSynchronize(f->stream);
   (void)hipStreamSynchronize(c->stream);
-  (void)hipStreamSynchronize(c->large_stream);
   frame_release(c, f);
   if (f->stream) (void)hipStreamDestroy(f->stream);
   delete f;
@@ -2982,9 +2971,12 @@ t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, 
   }
   // Frames in flight together overlap on the device, but not large ones: each holds more vertex records than the
   // memory-side cache keeps of two, so side by side they push out each other's and the assemblies wait for HBM (512
-  // uneven models, two frames in flight: 471 us a frame one after the other, 497 side by side).
+  // uneven models, two frames in flight: 471 us a frame one after the other, 497 side by side).  They take the context's
+  // stream, not one more: a process has four hardware queues, and with five streams (this one, the copies' and two
+  // frames' besides) two frames shared a queue and ran in turn whatever their size (20 uneven models 79 us a frame with
+  // five, 54 with four; a 1024 x 1024 grid 131 and 93).
   hipStream_t stream = f->stream ? f->stream : c->stream;
-  if (f->args.touch_records) stream = c->large_stream;
+  if (f->args.touch_records) stream = c->stream;
   st = frame_launch(c, f, stream, c->copy_stream, desc->exec_mode, true, true, alone);
   if (st) return st;
   f->submitted = wall0;

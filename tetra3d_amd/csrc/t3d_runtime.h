@@ -174,7 +174,6 @@ struct t3d_ctx {
   int device = 0;
   hipStream_t stream = nullptr;        // kernel chains of t3d_render / t3d_render_async
   hipStream_t copy_stream = nullptr;   // table uploads, so they overlap the previous frame's kernels
-  hipStream_t large_stream = nullptr;  // frames too large to overlap (render_submit)
   uint64_t budget = 0, used = 0;
   uint64_t next_handle = 1;
   std::map<uint64_t, std::unique_ptr<t3d::Mesh>> meshes;
