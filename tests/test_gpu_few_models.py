@@ -52,6 +52,7 @@ def test_large_frames_in_flight(fresh_ctx, oracle, count):
     for i in range(count):
         m = Model("m%d" % i, mesh)
         m.set_local_position(*(r.uniform(-4, 4, 3) - [0, 0, 6]))
+        m.frustum_culling = False          # all of them drawn: what counts is the drawn pairs' vertices
         models.append(m)
     lights = W.icosphere_scene().lights
     frames = [fresh_ctx.frame, fresh_ctx.new_frame()]

@@ -1098,7 +1098,8 @@ struct ProfScope {
 // profile charges each kernel its algorithmic bytes: mesh streams read once
 // (k_vertex), triangle indices once (k_cull), outputs (k_assemble, added
 // after the survivor counts are known); all of them to k_pair where it runs.
-t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t st, bool prof) {
+t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t st, bool prof,
+                     hipEvent_t gate = nullptr) {
   const FrameArgs& a = f->args;
   struct {
     uint64_t vertex = 0, cull = 0, uv = 0;
@@ -1133,6 +1134,7 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
     ProfScope ps(c, st, "k_uniforms", 0, prof);
     HIP_TRY(c, launch_uniforms(a, p0, p1 - p0, st));
   }
+  if (gate) HIP_TRY(c, hipStreamWaitEvent(st, gate, 0));
   f->ran_pairs = f->small_pairs && p0 == 0 && p1 == f->nparts;
   if (f->ran_pairs) {
     ProfScope ps(c, st, "k_pair", tr.vertex + tr.cull + tr.uv, prof);
@@ -2529,6 +2531,7 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   f->total_sblocks = sblocks;
   f->total_pscan = f->pscan_prefix.back();
   f->total_triangles = sumT;
+  f->drawn_vertices = sumV;
   if (c->profiling) {   // the caller holds ctx->mu
     const auto wall2 = std::chrono::steady_clock::now();
     auto& hp = c->prof["host:prologue"];
@@ -2568,9 +2571,10 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
     return T3D_OK;
   }
   t3d_status st = T3D_OK;
+  const hipEvent_t gate = f->in_turn && c->large_on != stream ? c->large_done : nullptr;
   if (exec_mode == T3D_EXEC_PLAIN && !f->device_stage) {
     for (uint32_t i = 0; i < P_n; i++) {
-      st = run_chain(c, f, i, i + 1, stream, profile);
+      st = run_chain(c, f, i, i + 1, stream, profile, i ? nullptr : gate);
       if (st) return st;
     }
   } else if (allow_graph && c->tuning.use_graph && !f->host_uniforms && !(profile && c->profiling)) {
@@ -2601,10 +2605,17 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
       if (ie != hipSuccess) return fail(c, T3D_ERR_DEVICE, "graph instantiate: %s", hipGetErrorString(ie));
       f->graph_key = key;
     }
+    if (gate) HIP_TRY(c, hipStreamWaitEvent(stream, gate, 0));
     HIP_TRY(c, hipGraphLaunch(f->graph_exec, stream));
   } else {
-    st = run_chain(c, f, 0, P_n, stream, profile);
+    st = run_chain(c, f, 0, P_n, stream, profile, gate);
     if (st) return st;
+  }
+  hipEvent_t ran = f->done;   // a device-built frame's readback lies between its last kernel and `done`
+  if (f->in_turn && f->device_stage) {
+    if (!f->ran) HIP_TRY(c, hipEventCreateWithFlags(&f->ran, hipEventDisableTiming));
+    ran = f->ran;
+    HIP_TRY(c, hipEventRecord(ran, stream));
   }
   if (f->device_stage) {   // counts, the jobs' first pairs, the pairs and their stats in one copy
     HIP_TRY(c, hipMemcpyAsync(f->pinned_rb, f->rb_dev, f->rb_bytes, hipMemcpyDeviceToHost, stream));
@@ -2616,6 +2627,10 @@ t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_
     f->stats_host = f->pinned_stats;
   }
   HIP_TRY(c, hipEventRecord(f->done, stream));
+  if (f->in_turn) {
+    c->large_done = ran;
+    c->large_on = stream;
+  }
   return T3D_OK;
 }
 
@@ -2658,6 +2673,7 @@ namespace {
 void collect_stage(t3d_ctx* c, t3d_frame* f, bool profile) {
   const uint32_t* cnt = reinterpret_cast<const uint32_t*>(f->pinned_rb);
   const uint32_t P = f->max_pairs ? cnt[FC_PAIRS] : 0u;
+  f->drawn_vertices = P ? cnt[FC_SUMV] : 0;
   const uint32_t* jp = reinterpret_cast<const uint32_t*>(f->pinned_rb + f->rb_jobs);
   const PairOut* po = reinterpret_cast<const PairOut*>(f->pinned_rb + f->rb_pairs);
   f->nparts = P;
@@ -2935,6 +2951,12 @@ void frame_release(t3d_ctx* c, t3d_frame* f) {
   f->device_stage = false;
   if (f->graph_exec) (void)hipGraphExecDestroy(f->graph_exec);
   f->graph_exec = nullptr;
+  if (c->large_done && (c->large_done == f->done || c->large_done == f->ran)) {
+    c->large_done = nullptr;
+    c->large_on = nullptr;
+  }
+  if (f->ran) (void)hipEventDestroy(f->ran);
+  f->ran = nullptr;
   if (f->done) (void)hipEventDestroy(f->done);
   if (f->tables_ready) (void)hipEventDestroy(f->tables_ready);
   f->done = f->tables_ready = nullptr;
@@ -2971,12 +2993,17 @@ t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, 
   }
   // Frames in flight together overlap on the device, but not large ones: each holds more vertex records than the
   // memory-side cache keeps of two, so side by side they push out each other's and the assemblies wait for HBM (512
-  // uneven models, two frames in flight: 471 us a frame one after the other, 497 side by side).  They take the context's
-  // stream, not one more: a process has four hardware queues, and with five streams (this one, the copies' and two
-  // frames' besides) two frames shared a queue and ran in turn whatever their size (20 uneven models 79 us a frame with
-  // five, 54 with four; a 1024 x 1024 grid 131 and 93).
-  hipStream_t stream = f->stream ? f->stream : c->stream;
-  if (f->args.touch_records) stream = c->stream;
+  // uneven models, two frames in flight: 471 us a frame one after the other, 497 side by side).  What counts is what the
+  // camera sees.  For a frame built on the device that is not known here: its handle's last render stands in, and a
+  // wrong guess costs time only.
+  // Frames built on the host take the context's stream then, not one more: a process has four hardware queues, and with
+  // five streams (this one, the copies' and two frames' besides) two frames shared a queue and ran in turn whatever
+  // their size (20 uneven models 79 us a frame with five, 54 with four; a 1024 x 1024 grid 131 and 93).  One built on
+  // the device keeps its own, where its model stage, palettes and uniforms run beside the frame before, and waits for
+  // that frame's kernels ahead of its vertices (700 uneven models 704 us a frame, 738 all in turn; 1,000 of them 1,128
+  // and 1,160; but on the host, with less to overlap, 512 of them 474 and 470).
+  f->in_turn = !alone && f->drawn_vertices > kTouchVertices;
+  hipStream_t stream = f->stream && (f->device_stage || !f->in_turn) ? f->stream : c->stream;
   st = frame_launch(c, f, stream, c->copy_stream, desc->exec_mode, true, true, alone);
   if (st) return st;
   f->submitted = wall0;

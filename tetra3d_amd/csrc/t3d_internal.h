@@ -33,7 +33,8 @@ constexpr uint32_t kPairVerticesMany = 2816, kPairTrianglesMany = 5632;  // ... 
 constexpr uint32_t kPairMany = 64;
 constexpr uint32_t kPairFew = 16;      // ... or at most so many, none skinned
 constexpr uint32_t kSearchPairs = 4;   // a host-built frame's blocks search among this many pairs; more have maps
-constexpr uint64_t kTouchVertices = 2400000;  // frames with more vertex records read them ahead of the assembly
+constexpr uint64_t kTouchVertices = 2400000;  // frames that draw more vertices read them ahead of the assembly and, in
+                                              // flight together, run one after the other
 constexpr uint32_t kScanPartMax = 65536;  // histogram matrices up to this size are scanned by one block
 
 // PartGPU.flags
@@ -301,7 +302,8 @@ struct FrameArgs {
   uint32_t vchunk;              // vertices per vertex-kernel block
   uint32_t tile;                // triangles per tile
   uint32_t xcd_swizzle;         // 1: give each XCD a contiguous range of blocks (see block_index_n)
-  uint32_t touch_records;       // 1: more vertex records than the memory-side cache keeps (see k_scatter4)
+  uint32_t touch_records;       // 1: more vertex records than the memory-side cache keeps (see k_scatter4; a frame
+                                // built on the device has their count in counts[FC_SUMV] instead)
   uint32_t pad0;
   const LightGPU* lights;
   PartLight* plights;

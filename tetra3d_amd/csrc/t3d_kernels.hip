@@ -1169,7 +1169,7 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
   // less they are still cached and reading them only costs (113 and 110
   // against 35 and 25).
   float touch = 0.0f;
-  if (a.touch_records) {
+  if (a.counts ? a.counts[FC_SUMV] > kTouchVertices : a.touch_records != 0) {
     constexpr uint32_t kLine = 128 / sizeof(float);
     const uint32_t v0 = (uint32_t)((uint64_t)P.vcount * tl / P.ntiles);
     const uint32_t nv = (uint32_t)((uint64_t)P.vcount * (tl + 1) / P.ntiles) - v0;

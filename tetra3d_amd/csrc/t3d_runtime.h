@@ -147,6 +147,8 @@ struct t3d_frame {
   const t3d::MaterialGPU* stage_mats = nullptr;
   uint64_t table_bytes = 0;
   uint64_t total_triangles = 0;
+  uint64_t drawn_vertices = 0;     // vertex records of the pairs drawn (built on the device: of the last frame read back)
+  bool in_turn = false;            // the last launch: a large frame, run after the kernels of the one before
   uint32_t max_triangles = 0, max_vertices = 0;   // of one render pair (with the device stage: of any MeshPart)
   bool small_pairs = false;        // may be drawn by one workgroup per render pair
   bool host_uniforms = false;      // few pairs: uniforms built on the host
@@ -165,6 +167,7 @@ struct t3d_frame {
   // asynchronous renders: tables uploaded / whole frame done, and whether a
   // launch is outstanding
   hipEvent_t tables_ready = nullptr, done = nullptr;
+  hipEvent_t ran = nullptr;        // after the kernels of a large device-built frame, before its readback
   hipStream_t stream = nullptr;    // the frame's own chain stream (null: the caller's)
   bool inflight = false;
   std::chrono::steady_clock::time_point submitted;
@@ -174,6 +177,9 @@ struct t3d_ctx {
   int device = 0;
   hipStream_t stream = nullptr;        // kernel chains of t3d_render / t3d_render_async
   hipStream_t copy_stream = nullptr;   // table uploads, so they overlap the previous frame's kernels
+  // the last large frame that t3d_render_async launched (render_submit): recorded after its kernels, and its stream
+  hipEvent_t large_done = nullptr;
+  hipStream_t large_on = nullptr;
   uint64_t budget = 0, used = 0;
   uint64_t next_handle = 1;
   std::map<uint64_t, std::unique_ptr<t3d::Mesh>> meshes;
