@@ -135,3 +135,32 @@ def test_noalloc_refusals():
             assert ref.survivors > 0
         finally:
             arrays.free()
+
+
+def _triangle_ids(ctx, frame):
+    ids = np.zeros(sum(p[3] for p in ctx.pairs(frame)), dtype=np.uint32)
+    ctx._check(ctx.L.t3d_frame_download_triangles(ctx.ctx, frame, ids.ctypes.data_as(C.POINTER(C.c_uint32))))
+    return ids
+
+
+@pytest.mark.gpu
+def test_noalloc_triangles_leave_other_frames_alone():
+    """Two frames rendered one after the other into the GPU's one static array: downloading the first one's triangles
+    (they are no longer there) changes nothing of the second, whose triangles are then the allocating render's.  The
+    sizes put the first one's depth keys where the second's slot records lie."""
+    first, second = W.heightfield_scene(n=59), W.icosphere_scene(level=4)
+    first.camera.process_only_visible = False      # all its triangles are drawn
+    hip = _hip()
+    with Context(0) as ctx:
+        ref = ctx.render_workload(second)
+        ctx.prepare(first)
+        frames = [ctx.new_frame(), ctx.new_frame()]
+        arrays = DeviceArrays(hip, max(_max_vertices(first), _max_vertices(second)))
+        try:
+            print("noalloc triangles", flush=True)
+            for wl, f in ((first, frames[0]), (second, frames[1])):
+                _noalloc_frame(ctx, wl, arrays, f, A.EXEC_BATCHED)
+            _triangle_ids(ctx, frames[0])
+            np.testing.assert_array_equal(_triangle_ids(ctx, frames[1]), ref.triangle_ids)
+        finally:
+            arrays.free()

@@ -1749,6 +1749,7 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   f->any_normals = any_normals;
   f->tables_dev = tables_dev;
   f->device_stage = true;
+  f->placed = false;
   f->max_pairs = maxP;
   f->stage_jobs = ndesc;
   f->nparts = maxP;
@@ -1787,6 +1788,7 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
     if (sst != T3D_ERR_UNSUPPORTED) return sst;   // else too large for the worst case: sized by what is drawn
   }
   f->device_stage = false;
+  f->placed = place != nullptr;
   f->max_pairs = 0;
   f->stage_models = nullptr;
   f->stage_mats = nullptr;
@@ -2761,30 +2763,46 @@ void frame_collect(t3d_ctx* c, t3d_frame* f, bool profile) {
   if (profile && c->profiling) c->prof[f->ran_pairs ? "k_pair" : "k_assemble"].bytes += 300ull * total;   // 3 x (48 B colour + 48 B depth + 4 B index)
 }
 
-// Packing buffer layout: block prefix, source and destination offsets, vertex counts and triangle sources of np pairs,
-// then the packed colour and depth vertices and indices, and the normals, of `verts` corners.  Packed triangles take no
-// room here: they go over the frame's depth keys, which nothing reads after the sort.
-static uint64_t pack_table_bytes(uint64_t np) {
-  return carve_size<uint32_t>(np + 1) + 2 * carve_size<uint64_t>(np) + 3 * carve_size<uint32_t>(np);
+// Packing buffer layout: block prefix, source and destination offsets and vertex counts of np pairs (and, where their
+// triangles are packed too, the triangles' sources), then the packed colour and depth vertices and indices, and the
+// normals, of `verts` corners.  Packed triangles take no room here: they go over the frame's depth keys, which nothing
+// reads after the sort.
+static uint64_t pack_table_bytes(uint64_t np, bool ids) {
+  return carve_size<uint32_t>(np + 1) + 2 * carve_size<uint64_t>(np) + (ids ? 3 : 1) * carve_size<uint32_t>(np);
 }
-static uint64_t pack_layout_bytes(uint64_t np, uint64_t verts, bool lists, bool normals) {
-  return pack_table_bytes(np) + (lists ? 2 * carve_size<t3d_vertex>(verts) + carve_size<uint32_t>(verts) : 0) +
-         (normals ? carve_size<t3d_vertex>(verts) : 0);
+static uint64_t pack_layout_bytes(uint64_t np, uint64_t verts, const DownloadParts& d) {
+  return pack_table_bytes(np, d.pack_ids) +
+         (d.lists ? 2 * carve_size<t3d_vertex>(verts) + carve_size<uint32_t>(verts) : 0) +
+         (d.normals ? carve_size<t3d_vertex>(verts) : 0);
 }
 
-uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool lists, bool normals) {
+DownloadParts download_parts(const t3d_frame* f, bool lists, bool normals, bool ids) {
+  DownloadParts d;
+  d.lists = lists;
+  d.normals = normals;
+  d.pack_ids = ids && !f->placed;   // a placed frame's keys lie in an array that other frames use after it
+  return d;
+}
+
+uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, const DownloadParts& d) {
   uint64_t np = 0, verts = 0;
   for (uint32_t i = p0; i < p1; i++)
     if (f->pairs[i].survivor_count) {
       np++;
       verts += 3ull * f->pairs[i].survivor_count;
     }
-  return verts ? pack_layout_bytes(np, verts, lists, normals) : 0;
+  if (!d.pack_ids && (np <= 1 || !(d.lists || d.normals))) return 0;   // copied as they lie
+  return verts ? pack_layout_bytes(np, verts, d) : 0;
+}
+
+t3d_status download_pack_grow(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, DownloadParts& d, PackBuf& pack) {
+  const uint64_t need = download_pack_bytes(f, p0, p1, d);
+  return need > pack.cap ? ensure(c, pack.dev, pack.cap, need) : T3D_OK;
 }
 
 t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t stream,
                                 t3d_vertex* cv, t3d_vertex* dv, uint32_t* idx, uint32_t* tri_ids, t3d_vertex* nv,
-                                PackBuf& pack, std::string* err_out) {
+                                const DownloadParts& parts, PackBuf& pack, std::string* err_out) {
   // Every exit after the first asynchronous copy waits for the stream, so no copy is still writing into the caller's
   // buffers when this returns; the message goes to *err_out when given, else to ctx->err.
   bool enqueued = false;
@@ -2809,23 +2827,21 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
       only = i;
       verts += 3ull * f->pairs[i].survivor_count;
     }
-  if (np == 1 && !tri_ids) {   // one pair's lists are contiguous as they are
+  const bool pack_ids = tri_ids && parts.pack_ids;
+  std::vector<uint4> recs;
+  if (np == 1 && !pack_ids) {   // one pair's lists are contiguous as they are
     const uint64_t v = f->pairs[only].vertex_offset;
     if (cv) DL_TRY(hipMemcpyAsync(cv, f->args.out_color + 3 * v, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
     if (dv) DL_TRY(hipMemcpyAsync(dv, f->args.out_depth + 3 * v, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
     if (idx) DL_TRY(hipMemcpyAsync(idx, f->args.out_idx + v, verts * 4, hipMemcpyDeviceToHost, stream));
     if (nv) DL_TRY(hipMemcpyAsync(nv, f->args.out_normal + 3 * v, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
-  } else if (np && (cv || dv || idx || nv || tri_ids)) {
+  } else if (np && (cv || dv || idx || nv || pack_ids)) {
     // the pairs' survivors packed on the device (k_pack), then one copy per stream; the tables go up in one copy from
     // pinned memory
-    const bool lists = cv || dv || idx;
-    const uint64_t need = pack_layout_bytes(np, verts, lists, nv != nullptr);
-    if (need > pack.cap) {
-      if (err_out) return bail(T3D_ERR_INVALID_ARGUMENT, "download: packing buffer too small");   // grown by the caller
-      t3d_status st = ensure(c, pack.dev, pack.cap, need);
-      if (st) return st;
-    }
-    const uint64_t tbytes = pack_table_bytes(np);
+    const bool lists = parts.lists;
+    if (pack_layout_bytes(np, verts, parts) > pack.cap)   // grown by the caller
+      return bail(T3D_ERR_INVALID_ARGUMENT, "download: packing buffer too small");
+    const uint64_t tbytes = pack_table_bytes(np, pack_ids);
     if (tbytes > pack.host_cap) {
       if (pack.host) (void)hipHostFree(pack.host);
       pack.host = nullptr;
@@ -2841,14 +2857,14 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
     uint64_t* h_src = hc.take<uint64_t>(np);
     uint64_t* h_dst = hc.take<uint64_t>(np);
     uint32_t* h_nv = hc.take<uint32_t>(np);
-    uint32_t* h_tsrc = hc.take<uint32_t>(np);
-    uint32_t* h_tfirst = hc.take<uint32_t>(np);
+    uint32_t* h_tsrc = pack_ids ? hc.take<uint32_t>(np) : nullptr;
+    uint32_t* h_tfirst = pack_ids ? hc.take<uint32_t>(np) : nullptr;
     pa.blk_prefix = pc.take<uint32_t>(np + 1);
     pa.src = pc.take<uint64_t>(np);
     pa.dst = pc.take<uint64_t>(np);
     pa.nvert = pc.take<uint32_t>(np);
-    pa.tsrc = pc.take<uint32_t>(np);
-    pa.tfirst = pc.take<uint32_t>(np);
+    pa.tsrc = pack_ids ? pc.take<uint32_t>(np) : nullptr;
+    pa.tfirst = pack_ids ? pc.take<uint32_t>(np) : nullptr;
     uint64_t off = 0;
     uint32_t k = 0, blocks = 0;
     for (uint32_t i = p0; i < p1; i++) {
@@ -2858,8 +2874,10 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
       h_src[k] = f->pairs[i].vertex_offset;
       h_dst[k] = off;
       h_nv[k] = (uint32_t)n;
-      h_tsrc[k] = f->pair_tbase[i];
-      h_tfirst[k] = f->part_first_tri[i];
+      if (pack_ids) {
+        h_tsrc[k] = f->pair_tbase[i];
+        h_tfirst[k] = f->part_first_tri[i];
+      }
       blocks += (uint32_t)((3 * n + 255) / 256);   // 3 float4 per vertex, 256 to a block
       off += n;
       k++;
@@ -2874,7 +2892,7 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
     float4* pdep = lists ? reinterpret_cast<float4*>(pc.take<t3d_vertex>(verts)) : nullptr;
     uint32_t* pidx = lists ? pc.take<uint32_t>(verts) : nullptr;
     float4* pnrm = nv ? reinterpret_cast<float4*>(pc.take<t3d_vertex>(verts)) : nullptr;
-    uint32_t* ptri = tri_ids ? reinterpret_cast<uint32_t*>(f->args.key) + f->pair_tbase[p0] : nullptr;
+    uint32_t* ptri = pack_ids ? reinterpret_cast<uint32_t*>(f->args.key) + f->pair_tbase[p0] : nullptr;
     pa.pcolor = cv ? pcol : nullptr;   // only the arrays asked for are packed
     pa.pdepth = dv ? pdep : nullptr;
     pa.pidx = idx ? pidx : nullptr;
@@ -2887,12 +2905,27 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
     if (dv) DL_TRY(hipMemcpyAsync(dv, pdep, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
     if (idx) DL_TRY(hipMemcpyAsync(idx, pidx, verts * 4, hipMemcpyDeviceToHost, stream));
     if (nv) DL_TRY(hipMemcpyAsync(nv, pnrm, verts * sizeof(t3d_vertex), hipMemcpyDeviceToHost, stream));
-    if (tri_ids) DL_TRY(hipMemcpyAsync(tri_ids, ptri, verts / 3 * 4, hipMemcpyDeviceToHost, stream));
+    if (pack_ids) DL_TRY(hipMemcpyAsync(tri_ids, ptri, verts / 3 * 4, hipMemcpyDeviceToHost, stream));
+  }
+  if (tri_ids && !pack_ids && verts) {   // the slot records as they lie
+    recs.resize(verts / 3);
+    uint64_t at = 0;
+    for (uint32_t i = p0; i < p1; i++) {
+      const uint32_t n = f->pairs[i].survivor_count;
+      if (!n) continue;
+      DL_TRY(hipMemcpyAsync(recs.data() + at, f->args.tri_vo + f->pair_tbase[i], 16ull * n, hipMemcpyDeviceToHost, stream));
+      at += n;
+    }
   }
   const hipError_t e = hipStreamSynchronize(stream);
   enqueued = false;
   if (e != hipSuccess) return bail(T3D_ERR_DEVICE, std::string("download: ") + hipGetErrorString(e));
 #undef DL_TRY
+  if (!recs.empty()) {
+    uint64_t at = 0;
+    for (uint32_t i = p0; i < p1; i++)
+      for (uint32_t k = 0; k < f->pairs[i].survivor_count; k++, at++) tri_ids[at] = recs[at].w + f->part_first_tri[i];
+  }
   return T3D_OK;
 }
 
@@ -3067,8 +3100,11 @@ t3d_status t3d_frame_download(t3d_ctx* c, const t3d_frame* f, t3d_vertex* cv, t3
   if (f->inflight) return fail(c, T3D_ERR_NOT_READY, "frame_download: render in flight (t3d_frame_wait first)");
   (void)hipSetDevice(c->device);
   t3d_frame* fm = const_cast<t3d_frame*>(f);   // the staging buffer only; the frame's results are untouched
-  return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, cv, dv, idx, nullptr, nullptr,
-                              fm->pack);
+  const uint32_t np = (uint32_t)f->pairs.size();
+  DownloadParts parts = download_parts(f, cv || dv || idx, false, false);
+  t3d_status st = download_pack_grow(c, f, 0, np, parts, fm->pack);
+  if (st) return st;
+  return frame_download_range(c, f, 0, np, c->stream, cv, dv, idx, nullptr, nullptr, parts, fm->pack);
 }
 
 t3d_status t3d_frame_download_normals(t3d_ctx* c, const t3d_frame* f, t3d_vertex* nv) {
@@ -3077,8 +3113,11 @@ t3d_status t3d_frame_download_normals(t3d_ctx* c, const t3d_frame* f, t3d_vertex
   if (f->inflight) return fail(c, T3D_ERR_NOT_READY, "frame_download: render in flight (t3d_frame_wait first)");
   (void)hipSetDevice(c->device);
   t3d_frame* fm = const_cast<t3d_frame*>(f);
-  return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, nullptr, nullptr, nullptr, nullptr, nv,
-                              fm->pack);
+  const uint32_t np = (uint32_t)f->pairs.size();
+  DownloadParts parts = download_parts(f, false, true, false);
+  t3d_status st = download_pack_grow(c, f, 0, np, parts, fm->pack);
+  if (st) return st;
+  return frame_download_range(c, f, 0, np, c->stream, nullptr, nullptr, nullptr, nullptr, nv, parts, fm->pack);
 }
 
 t3d_status t3d_frame_download_triangles(t3d_ctx* c, const t3d_frame* f, uint32_t* ids) {
@@ -3087,8 +3126,11 @@ t3d_status t3d_frame_download_triangles(t3d_ctx* c, const t3d_frame* f, uint32_t
   if (f->inflight) return fail(c, T3D_ERR_NOT_READY, "frame_download: render in flight (t3d_frame_wait first)");
   (void)hipSetDevice(c->device);
   t3d_frame* fm = const_cast<t3d_frame*>(f);
-  return frame_download_range(c, f, 0, (uint32_t)f->pairs.size(), c->stream, nullptr, nullptr, nullptr, ids, nullptr,
-                              fm->pack);
+  const uint32_t np = (uint32_t)f->pairs.size();
+  DownloadParts parts = download_parts(f, false, false, true);
+  t3d_status st = download_pack_grow(c, f, 0, np, parts, fm->pack);
+  if (st) return st;
+  return frame_download_range(c, f, 0, np, c->stream, nullptr, nullptr, nullptr, ids, nullptr, parts, fm->pack);
 }
 
 t3d_status t3d_debug_model_spheres(const t3d_mat4* transforms, const float* dims, const uint8_t* skinned, uint32_t n,

@@ -102,6 +102,7 @@ struct t3d_frame {
   std::vector<uint8_t> host_tables;
   std::vector<uint32_t> host_stats_copy;
   const uint32_t* stats_host = nullptr;
+  bool placed = false;             // the last build's memory is external (t3d_render_noalloc)
   uint8_t* tables_dev = nullptr;   // device table block of the last build (own or placed)
   bool any_normals = false;        // the last build fills the normal vertex list (Camera.RenderNormals)
   t3d::FrameArgs args{};
@@ -273,16 +274,24 @@ t3d_status frame_run_placed(t3d_ctx* c, t3d_frame* f, hipStream_t stream, int32_
 t3d_status frame_launch(t3d_ctx* c, t3d_frame* f, hipStream_t stream, hipStream_t copy_stream, int32_t exec_mode,
                         bool allow_graph, bool profile, bool alone = false);
 void frame_collect(t3d_ctx* c, t3d_frame* f, bool profile);
-// Device bytes frame_download_range needs in `pack` for pairs [p0, p1) (0 when none survive).
-uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, bool lists, bool normals);
+// What a download takes: vertex and index lists, normals; and whether triangles are packed on the device with them (over
+// the frame's depth keys) or copied from its slot records as they lie.
+struct DownloadParts {
+  bool lists = false, normals = false, pack_ids = false;
+};
+DownloadParts download_parts(const t3d_frame* f, bool lists, bool normals, bool ids);
+// Device bytes frame_download_range needs in `pack` for pairs [p0, p1) (0 where nothing is packed).
+uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, const DownloadParts& d);
+// Grows `pack` to that (the caller holds ctx->mu).
+t3d_status download_pack_grow(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, DownloadParts& d, PackBuf& pack);
 // Copy pairs [p0, p1) of a frame, concatenated, to host memory (any output may be null): vertices, indices and
-// triangles packed on the device into `pack`, so that they cross to the host in one copy per stream (a single pair's
-// lists are copied as they lie).  Without err_out, `pack` is grown here when too small (needs ctx->mu) and errors go
-// to ctx->err; with it, the caller has grown `pack` to download_pack_bytes already and the message goes to *err_out
-// (no ctx state is touched).  Returns only after every copy it enqueued has finished.
+// triangles packed on the device into `pack` (grown by the caller), so that they cross to the host in one copy per
+// stream (a single pair's lists are copied as they lie).  `parts` names the arrays that are not null.  Errors go to
+// ctx->err (needs ctx->mu), or with err_out to *err_out (no ctx state is touched).  Returns only after every copy it
+// enqueued has finished.
 t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t stream,
                                 t3d_vertex* cv, t3d_vertex* dv, uint32_t* idx, uint32_t* tri_ids, t3d_vertex* nv,
-                                PackBuf& pack, std::string* err_out = nullptr);
+                                const DownloadParts& parts, PackBuf& pack, std::string* err_out = nullptr);
 void pack_release(t3d_ctx* c, PackBuf& pack);
 // Frame memory a job may need (scratch + outputs + tables), before frustum culling.
 uint64_t estimate_job_bytes(t3d_ctx* c, const t3d_render_desc* desc);

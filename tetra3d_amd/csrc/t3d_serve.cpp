@@ -730,16 +730,16 @@ t3d_status job_download(t3d_server* s, uint64_t job, t3d_pair_result* pairs, t3d
     (void)hipSetDevice(s->ctx->device);
     std::lock_guard<std::mutex> dl(s->dl_mu);   // one download at a time on the download stream
     // the server's packing buffer: grown under ctx->mu (memory accounting), used under dl_mu only
-    const uint64_t need = download_pack_bytes(f, p0, p1, cv || dv || idx, nv != nullptr);
-    if (need > s->pack.cap) {
+    DownloadParts parts = download_parts(f, cv || dv || idx, nv != nullptr, tri_ids != nullptr);
+    if (download_pack_bytes(f, p0, p1, parts) > s->pack.cap) {
       std::lock_guard<std::mutex> cl(s->ctx->mu);
-      st = ensure(s->ctx, s->pack.dev, s->pack.cap, need);
+      st = download_pack_grow(s->ctx, f, p0, p1, parts, s->pack);
       s->pack_bytes = s->pack.dev.bytes;
     }
     if (!st) {
       // errors are reported into a local string (the worker may be writing ctx->err under ctx->mu)
       std::string err;
-      st = frame_download_range(s->ctx, f, p0, p1, s->dl_stream, cv, dv, idx, tri_ids, nv, s->pack, &err);
+      st = frame_download_range(s->ctx, f, p0, p1, s->dl_stream, cv, dv, idx, tri_ids, nv, parts, s->pack, &err);
       if (st) {
         std::lock_guard<std::mutex> cl(s->ctx->mu);
         s->ctx->err = err;
