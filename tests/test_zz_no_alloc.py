@@ -164,3 +164,23 @@ def test_noalloc_triangles_leave_other_frames_alone():
             np.testing.assert_array_equal(_triangle_ids(ctx, frames[1]), ref.triangle_ids)
         finally:
             arrays.free()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 12])
+def test_triangles_need_no_device_memory(count):
+    """With the context's budget used up by the frame itself, its triangles still download."""
+    wl = W.mixed_scene(count=count)
+    with Context(0) as ctx:
+        ctx.prepare(wl)
+        ctx.render_inputs(ctx.inputs(wl.camera, wl.scene, wl.lights, wl.models))
+        used = ctx.memory_used
+        want = _triangle_ids(ctx, ctx.frame)
+    for m in wl.meshes:
+        m._handles.pop("gpu", None)
+    with Context(0, used) as ctx:
+        ctx.prepare(wl)
+        ctx.render_inputs(ctx.inputs(wl.camera, wl.scene, wl.lights, wl.models))
+        assert ctx.memory_used == used
+        print("triangles at the budget", count, len(want), flush=True)
+        np.testing.assert_array_equal(_triangle_ids(ctx, ctx.frame), want)

@@ -2796,8 +2796,17 @@ uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, const
 }
 
 t3d_status download_pack_grow(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, DownloadParts& d, PackBuf& pack) {
-  const uint64_t need = download_pack_bytes(f, p0, p1, d);
-  return need > pack.cap ? ensure(c, pack.dev, pack.cap, need) : T3D_OK;
+  uint64_t need = download_pack_bytes(f, p0, p1, d);
+  if (need <= pack.cap) return T3D_OK;
+  const std::string err = c->err;
+  t3d_status st = ensure(c, pack.dev, pack.cap, need);
+  if (st && d.pack_ids) {   // no room for the tables: the triangles need none
+    d.pack_ids = false;
+    need = download_pack_bytes(f, p0, p1, d);
+    st = need ? ensure(c, pack.dev, pack.cap, need) : T3D_OK;
+    if (!st) c->err = err;
+  }
+  return st;
 }
 
 t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, hipStream_t stream,

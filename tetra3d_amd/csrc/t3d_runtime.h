@@ -282,7 +282,8 @@ struct DownloadParts {
 DownloadParts download_parts(const t3d_frame* f, bool lists, bool normals, bool ids);
 // Device bytes frame_download_range needs in `pack` for pairs [p0, p1) (0 where nothing is packed).
 uint64_t download_pack_bytes(const t3d_frame* f, uint32_t p0, uint32_t p1, const DownloadParts& d);
-// Grows `pack` to that (the caller holds ctx->mu).
+// Grows `pack` to that (the caller holds ctx->mu); where the budget has no room for packing triangles, d.pack_ids is
+// cleared: downloading triangles alone needs no device memory.
 t3d_status download_pack_grow(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uint32_t p1, DownloadParts& d, PackBuf& pack);
 // Copy pairs [p0, p1) of a frame, concatenated, to host memory (any output may be null): vertices, indices and
 // triangles packed on the device into `pack` (grown by the caller), so that they cross to the host in one copy per
