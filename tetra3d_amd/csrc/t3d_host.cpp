@@ -2315,7 +2315,12 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
                         carve_size<uint32_t>(sblocks) + 2 * carve_size<uint32_t>(ntiles_total) +
                         carve_size<uint32_t>(f->vchunk_prefix.back()) + carve_size<PartLight>(n_plights) +
                         carve_size<M4>(pose_bones) + carve_size<float4>(any_normals ? sumV : 1);
-  const uint64_t sbytes = rest + record_scratch(sumV, sumT, any_skinned);
+  // with the uniforms in the tables, these four arrays lie there (or are not read at all) instead of in scratch
+  const uint64_t moved = !f->host_uniforms ? 0
+                                           : carve_size<uint32_t>(4ull * P_n) + carve_size<uint32_t>(ntiles_total) +
+                                                 carve_size<uint32_t>(f->vchunk_prefix.back()) +
+                                                 carve_size<PartLight>(n_plights);
+  const uint64_t sbytes = rest - moved + record_scratch(sumV, sumT, any_skinned);
   uint8_t *tables_dev, *tables_host, *scratch_dev;
   t3d_vertex *out_color, *out_depth, *out_normal = nullptr;
   uint32_t* out_idx;
@@ -2497,13 +2502,9 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   a.sblock_prefix = d_spre;
   a.pscan_prefix = d_ppre;
   take_records(sc, a, sumV, sumT, any_skinned);
-  a.stats = sc.take<uint32_t>(4ull * P_n);
   a.hist = sc.take<uint32_t>(sumHist);
   a.bsum = sc.take<uint32_t>(sblocks);
   a.tile_count = sc.take<uint32_t>(ntiles_total);
-  a.tile_part = sc.take<uint32_t>(ntiles_total);
-  a.vchunk_part = sc.take<uint32_t>(f->vchunk_prefix.back());
-  a.plights = sc.take<PartLight>(n_plights);
   if (f->host_stats) {      // k_pair or k_assemble puts the survivor counts where the host reads them
     a.host_stats = place ? place->pinned_stats : f->pinned_stats;
     for (uint32_t i = 0; i < P_n; i++) a.host_stats[4 * i + 2] = 0;
@@ -2513,6 +2514,11 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
     a.stats = reinterpret_cast<uint32_t*>(d_stats);
     a.tile_part = host_tiles ? d_tpart : nullptr;
     a.vchunk_part = host_tiles ? d_vpart : nullptr;
+  } else {
+    a.stats = sc.take<uint32_t>(4ull * P_n);
+    a.tile_part = sc.take<uint32_t>(ntiles_total);
+    a.vchunk_part = sc.take<uint32_t>(f->vchunk_prefix.back());
+    a.plights = sc.take<PartLight>(n_plights);
   }
   a.pose_world = sc.take<M4>(pose_bones);
   a.vnrm = sc.take<float4>(any_normals ? sumV : 1);
