@@ -492,8 +492,9 @@ t3d_status t3d_profile_read(t3d_ctx* ctx, t3d_kernel_time* per_kernel, uint32_t 
  * [vertex_offset, vertex_offset + 3*survivor_count) of the caller's arrays
  * (t3d_frame_pairs), so the arrays must hold 3 x the triangles of every drawn
  * render pair (T3D_ERR_INVALID_ARGUMENT otherwise, naming the count); a frame
- * whose tables and scratch exceed the array is refused with T3D_ERR_BUDGET.
- * The frame argument carries only host bookkeeping here.  Every call on one
+ * whose tables and scratch exceed the array is refused with T3D_ERR_BUDGET
+ * (counted with 52 bytes a vertex and 36 a triangle, whatever the records
+ * take).  The frame argument carries only host bookkeeping here.  Every call on one
  * GPU shares its array, from any context: calls that overlap on one GPU race. */
 t3d_status t3d_render_noalloc(t3d_ctx* ctx, t3d_frame* frame, const t3d_render_desc* desc,
                               t3d_vertex* color_vertices, t3d_vertex* depth_vertices, uint32_t* indices,

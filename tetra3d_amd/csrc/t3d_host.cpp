@@ -186,11 +186,11 @@ void dev_free(t3d_ctx* c, DevBuf& b) {
 }
 
 // Grow `b` to at least `bytes` (discarding contents), with 25% headroom.
+uint64_t grown_size(uint64_t bytes) { return align_up(bytes + bytes / 4 + 4096, 1 << 16); }
 t3d_status ensure(t3d_ctx* c, DevBuf& b, uint64_t& cap, uint64_t bytes) {
   if (bytes <= cap && b.ptr) return T3D_OK;
   dev_free(c, b);
-  uint64_t want = align_up(bytes + bytes / 4 + 4096, 1 << 16);
-  t3d_status st = dev_alloc(c, b, want);
+  t3d_status st = dev_alloc(c, b, grown_size(bytes));
   if (st) {
     cap = 0;
     return st;
@@ -215,26 +215,50 @@ uint64_t carve_size(uint64_t count) {
   return align_up(std::max<uint64_t>(count, 1) * sizeof(T), 256);
 }
 
-// Per-vertex and per-triangle records of a frame: 49 bytes a vertex (65 when the frame has a skinned model) and
-// 22 a triangle.
-uint64_t record_scratch(uint64_t V, uint64_t T, bool skinned) {
-  return carve_size<float4>(2 * V) + carve_size<float4>(V) + carve_size<uint8_t>(V) + carve_size<float4>(skinned ? V : 1) +
+// Per-vertex and per-triangle records of a frame: 49 bytes a vertex, 65 when the frame has a skinned model, and 22 a
+// triangle.  Lean, they are 49 with skinned models too: the skinned positions, which only the cull reads, lie where the
+// colour halves of the records go once the cull is done, and the vertex pass runs once for each.
+uint64_t record_scratch(uint64_t V, uint64_t T, bool skinned, bool lean) {
+  return carve_size<float4>(2 * V) + carve_size<float4>(V) + carve_size<uint8_t>(V) +
+         (skinned && !lean ? carve_size<float4>(V) : 0) +
          carve_size<float>(T) + carve_size<uint16_t>(T) + carve_size<uint4>(T);
 }
-void take_records(Carve& sc, FrameArgs& a, uint64_t V, uint64_t T, bool skinned) {
-  a.touch_records = V > kTouchVertices ? 1u : 0u;
+void take_records(Carve& sc, FrameArgs& a, uint64_t V, uint64_t T, bool skinned, bool lean) {
+  a.lean = lean ? 1u : 0u;
+  a.touch_records = V > kTouchVertices && !lean ? 1u : 0u;
   a.vab = sc.take<float4>(2 * V);
   a.vq = sc.take<float4>(V);
   a.vz = sc.take<uint8_t>(V);
-  a.vpos = sc.take<float4>(skinned ? V : 1);
+  a.vpos = !skinned ? nullptr : lean ? a.vab : sc.take<float4>(V);
   a.key = sc.take<float>(T);
   a.tri_loc = sc.take<uint16_t>(T);
   a.tri_vo = sc.take<uint4>(T);
 }
+// Whether a frame with skinned models has to do with lean records.  Frames were and are admitted with 52 bytes a vertex
+// and 36 a triangle (estimate_job_bytes; a context's budget that held a frame of an earlier layout holds it still):
+// lean ones never take more, the others do where a mesh has more than 1.08 vertices for each triangle.  So a server's
+// batch (`admitted`) is lean where it would take more, but for half of what an estimate adds for everything else; and
+// any frame where ensure() would otherwise refuse its tables, scratch (`full` bytes) or outputs.
+bool needs_lean(const t3d_ctx* c, const t3d_frame* f, uint64_t tables, uint64_t full, uint64_t outputs, uint64_t V,
+                uint64_t T, bool admitted) {
+  if (f->scratch.ptr && full <= f->scratch_cap) return false;
+  if (admitted && 13 * V > 14 * T + kEstimateExtra / 2) return true;
+  if (!c->budget) return false;
+  uint64_t used = c->used;
+  bool fits = true;
+  auto grow = [&](const DevBuf& b, uint64_t cap, uint64_t bytes) {
+    if (bytes <= cap && b.ptr) return;
+    used = used - b.bytes + grown_size(bytes);
+    fits = fits && used <= c->budget;
+  };
+  grow(f->tables, f->tables_cap, tables);
+  grow(f->scratch, f->scratch_cap, full);
+  grow(f->outputs, f->outputs_cap, outputs);
+  return !fits;
+}
 // What t3d_render_noalloc counts against T3D_NOALLOC_SCRATCH_BYTES for them: 52 bytes a vertex and 36 a triangle,
-// whatever the records take, so which frames fit is a rule on their sizes that a change of layout does not move.
-// The static array is a quarter larger than the limit: a frame whose models are all skinned takes up to 65 bytes
-// where 52 are counted.
+// whatever the records take, so which frames fit is a rule on their sizes that a change of layout does not move (a
+// frame that is counted as fitting and does not fit has lean records).
 uint64_t placed_charge(uint64_t V, uint64_t T) {
   return carve_size<float4>(2 * V) + carve_size<float4>(V) + carve_size<uint32_t>(T) + 2 * carve_size<uint4>(T) +
          carve_size<float4>(128) + carve_size<float>(V);
@@ -1143,7 +1167,7 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
   }
   {
     ProfScope ps(c, st, "k_vertex", tr.vertex + tr.uv, prof);
-    HIP_TRY(c, launch_vertex(a, vb0, vb1 - vb0, f->vertex_threads, st));
+    HIP_TRY(c, launch_vertex(a, vb0, vb1 - vb0, f->vertex_threads, a.lean ? VERTEX_FOR_CULL : VERTEX_ALL, st));
   }
   {
     ProfScope ps(c, st, "k_cull", tr.cull, prof);
@@ -1165,6 +1189,10 @@ t3d_status run_chain(t3d_ctx* c, t3d_frame* f, uint32_t p0, uint32_t p1, hipStre
   {
     ProfScope ps(c, st, "k_scatter", 0, prof);
     HIP_TRY(c, launch_scatter(a, tb0, tb1 - tb0, c->tuning.scatter_waves, st));
+  }
+  if (a.lean) {
+    ProfScope ps(c, st, "k_vertex", 0, prof);
+    HIP_TRY(c, launch_vertex(a, vb0, vb1 - vb0, f->vertex_threads, VERTEX_FOR_LISTS, st));
   }
   {
     ProfScope ps(c, st, "k_assemble", 0, prof);
@@ -1386,7 +1414,8 @@ void mesh_worst_case(Mesh& m, uint32_t vchunk, uint32_t tile) {
 // candidate pair being drawn.  Returns T3D_ERR_UNSUPPORTED without touching
 // the frame when that worst case would not fit the chain's 32-bit counts
 // (frame_build then builds it on the host).
-t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* descs, uint32_t ndesc) {
+t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* descs, uint32_t ndesc,
+                             bool admitted) {
   const auto wall0 = std::chrono::steady_clock::now();
   (void)hipSetDevice(c->device);
   const t3d_tuning& tu = c->tuning;
@@ -1500,14 +1529,19 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   const uint64_t rb_stats = rb_pairs + carve_size<PairOut>(maxP);
   const uint64_t rb_bytes = rb_stats + carve_size<uint32_t>(4ull * maxP);
   // scratch: the stage's arrays, the pair records and prefix arrays, then the chain's scratch at worst-case sizes
-  const uint64_t sbytes = rb_bytes + carve_size<PartGPU>(maxP) + 4 * carve_size<uint32_t>(maxP + 1ull) +
+  const uint64_t obytes = 2 * carve_size<t3d_vertex>(3 * wT) + carve_size<uint32_t>(3 * wT) +
+                          (any_normals ? carve_size<t3d_vertex>(3 * wT) : 0);
+  const uint64_t stage_bytes = rb_bytes + carve_size<PartGPU>(maxP) + 4 * carve_size<uint32_t>(maxP + 1ull) +
                           4 * carve_size<uint32_t>(ncand) + carve_size<float>(ncand) + carve_size<int32_t>(ncand) +
                           carve_size<uint4>(2 * ncand) + 2 * carve_size<uint4>(ncand) + 2 * carve_size<uint32_t>(ndesc) +
                           carve_size<uint32_t>(8ull * maxP) +
-                          record_scratch(wV, wT, any_skinned) + carve_size<uint32_t>(whist) + carve_size<uint32_t>(wsb) +
+                          carve_size<uint32_t>(whist) + carve_size<uint32_t>(wsb) +
                           2 * carve_size<uint32_t>(wtiles) + carve_size<uint32_t>(wvch) +
                           carve_size<PartLight>(wpl) + carve_size<M4>(pose_bones) +
                           carve_size<float4>(any_normals ? wV : 1);
+  const bool lean = any_skinned &&
+                    needs_lean(c, f, tbytes, stage_bytes + record_scratch(wV, wT, true, false), obytes, wV, wT, admitted);
+  const uint64_t sbytes = stage_bytes + record_scratch(wV, wT, any_skinned, lean);
   t3d_status st = ensure(c, f->tables, f->tables_cap, tbytes);
   if (st) return st;
   if (tbytes > f->pinned_cap) {
@@ -1518,8 +1552,6 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   }
   st = ensure(c, f->scratch, f->scratch_cap, sbytes);
   if (st) return st;
-  const uint64_t obytes = 2 * carve_size<t3d_vertex>(3 * wT) + carve_size<uint32_t>(3 * wT) +
-                          (any_normals ? carve_size<t3d_vertex>(3 * wT) : 0);
   st = ensure(c, f->outputs, f->outputs_cap, obytes);
   if (st) return st;
   if (rb_bytes > f->pinned_rb_cap) {
@@ -1723,10 +1755,10 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
   ms.vchunk = vchunk;
   ms.tile = tile;
   ms.max_pairs = maxP;
-  take_records(sc, a, wV, wT, any_skinned);
+  take_records(sc, a, wV, wT, any_skinned, lean);
   f->max_triangles = max_tri;
   f->max_vertices = max_vert;
-  f->small_pairs = pairs_fit(f, ncand, wT, any_skinned, any_normals, false);
+  f->small_pairs = !lean && pairs_fit(f, ncand, wT, any_skinned, any_normals, false);
   a.hist = sc.take<uint32_t>(whist);
   a.bsum = sc.take<uint32_t>(wsb);
   a.tile_count = sc.take<uint32_t>(wtiles);
@@ -1779,12 +1811,12 @@ t3d_status frame_build_stage(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* co
 // jobs shares one launch chain; every render pair carries its job's camera
 // index).  Pure host work: nothing is sent to the device yet.
 t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* descs, uint32_t ndesc,
-                       const Placement* place, bool device_stage) {
+                       const Placement* place, bool device_stage, bool admitted) {
   auto wall0 = std::chrono::steady_clock::now();
   if (!c || !f || !descs || ndesc == 0) return fail(c, T3D_ERR_INVALID_ARGUMENT, "render: null argument");
   f->host_uniforms = f->host_stats = false;
   if (device_stage && !place && stage_applies(c, descs, ndesc)) {
-    t3d_status sst = frame_build_stage(c, f, descs, ndesc);
+    t3d_status sst = frame_build_stage(c, f, descs, ndesc, admitted);
     if (sst != T3D_ERR_UNSUPPORTED) return sst;   // else too large for the worst case: sized by what is drawn
   }
   f->device_stage = false;
@@ -2320,7 +2352,13 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
                                            : carve_size<uint32_t>(4ull * P_n) + carve_size<uint32_t>(ntiles_total) +
                                                  carve_size<uint32_t>(f->vchunk_prefix.back()) +
                                                  carve_size<PartLight>(n_plights);
-  const uint64_t sbytes = rest - moved + record_scratch(sumV, sumT, any_skinned);
+  const uint64_t obytes = 2 * carve_size<t3d_vertex>(3 * sumT) + carve_size<uint32_t>(3 * sumT) +
+                          (any_normals ? carve_size<t3d_vertex>(3 * sumT) : 0);
+  const uint64_t full = rest - moved + record_scratch(sumV, sumT, any_skinned, false);
+  const bool lean = any_skinned && (place ? tbytes + full > place->scratch_bytes
+                                          : needs_lean(c, f, tbytes, full, obytes, sumV, sumT, admitted));
+  const uint64_t sbytes = rest - moved + record_scratch(sumV, sumT, any_skinned, lean);
+  if (lean) f->small_pairs = false;
   uint8_t *tables_dev, *tables_host, *scratch_dev;
   t3d_vertex *out_color, *out_depth, *out_normal = nullptr;
   uint32_t* out_idx;
@@ -2330,12 +2368,9 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
                                           "this entry point does not take");
     // no allocation: tables and scratch carved from the placement's scratch, outputs the caller's
     const uint64_t charge = tbytes - host_bytes + rest + placed_charge(sumV, sumT);
-    if (charge > place->scratch_bytes)
+    if (charge > place->scratch_bytes || tbytes + sbytes > place->scratch_bytes)   // the second is never more
       return fail(c, T3D_ERR_BUDGET, "render_noalloc: the frame needs %llu bytes of scratch, the static scratch holds %llu",
                   (unsigned long long)charge, (unsigned long long)place->scratch_bytes);
-    if (tbytes + sbytes > place->scratch_room)
-      return fail(c, T3D_ERR_BUDGET, "render_noalloc: the frame's records need %llu bytes, the static array has %llu",
-                  (unsigned long long)(tbytes + sbytes), (unsigned long long)place->scratch_room);
     if (3 * sumT > place->capacity)
       return fail(c, T3D_ERR_INVALID_ARGUMENT, "render_noalloc: outputs hold %llu vertices, the frame needs %llu",
                   (unsigned long long)place->capacity, (unsigned long long)(3 * sumT));
@@ -2358,8 +2393,6 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
     }
     st = ensure(c, f->scratch, f->scratch_cap, sbytes);
     if (st) return st;
-    const uint64_t obytes = 2 * carve_size<t3d_vertex>(3 * sumT) + carve_size<uint32_t>(3 * sumT) +
-                            (any_normals ? carve_size<t3d_vertex>(3 * sumT) : 0);
     st = ensure(c, f->outputs, f->outputs_cap, obytes);
     if (st) return st;
     if (4ull * P_n > f->pinned_stats_cap) {
@@ -2501,7 +2534,7 @@ t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* d
   a.tile_prefix = d_tpre;
   a.sblock_prefix = d_spre;
   a.pscan_prefix = d_ppre;
-  take_records(sc, a, sumV, sumT, any_skinned);
+  take_records(sc, a, sumV, sumT, any_skinned, lean);
   a.hist = sc.take<uint32_t>(sumHist);
   a.bsum = sc.take<uint32_t>(sblocks);
   a.tile_count = sc.take<uint32_t>(ntiles_total);
@@ -2952,14 +2985,12 @@ void pack_release(t3d_ctx* c, PackBuf& pack) {
 }
 
 uint64_t estimate_job_bytes(t3d_ctx* c, const t3d_render_desc* desc) {
-  // scratch: clip + colour + skinned position + unbillboarded depth (52 B/V; a job whose camera renders normals
-  // adds 16 B/V here and
-  // 144 B/T of normal vertices) and a block->pair entry per vertex block (at least 64
-  // vertices); key + two records (36 B/T); per tile a 512-bin histogram column, a scan block sum share, a survivor
-  // count and a tile->pair entry (~2 KB); outputs: 3 x (48 + 48 + 4) = 300 B/T; tables: ~1 KB per model plus
-  // palettes
+  // scratch: 52 B/V, at least what vertex records take (see needs_lean; a job whose camera renders normals adds 16 B/V
+  // here and 144 B/T of normal vertices), and a block->pair entry per vertex block (at least 64 vertices); 36 B/T, at
+  // least the triangle records; per tile a 512-bin histogram column, a scan block sum share, a survivor count and a
+  // tile->pair entry (~2 KB); outputs: 3 x (48 + 48 + 4) = 300 B/T; tables: ~1 KB per model plus palettes
   const uint64_t tile = std::max<uint32_t>(64, c->tuning.triangle_tile);
-  uint64_t V = 0, T = 0, tiles = 0, extra = 64 * 1024;
+  uint64_t V = 0, T = 0, tiles = 0, extra = kEstimateExtra;
   for (uint32_t mi = 0; mi < desc->model_count; mi++) {
     const t3d_model_desc& md = desc->models[mi];
     auto it = c->meshes.find(md.mesh);

@@ -304,7 +304,7 @@ struct FrameArgs {
   uint32_t xcd_swizzle;         // 1: give each XCD a contiguous range of blocks (see block_index_n)
   uint32_t touch_records;       // 1: more vertex records than the memory-side cache keeps (see k_scatter4; a frame
                                 // built on the device has their count in counts[FC_SUMV] instead)
-  uint32_t pad0;
+  uint32_t lean;                // 1: vpos lies in vab until the cull is done; the vertex pass runs twice
   const LightGPU* lights;
   PartLight* plights;
   const uint32_t* vchunk_prefix;  // [P+1]
@@ -404,7 +404,12 @@ struct RasterPair {
 // form can launch one part's blocks at a time.
 hipError_t launch_palettes(const FrameArgs& a, hipStream_t s);
 hipError_t launch_uniforms(const FrameArgs& a, uint32_t part0, uint32_t nparts, hipStream_t s);
-hipError_t launch_vertex(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, hipStream_t s);
+enum VertexOut : uint32_t {
+  VERTEX_FOR_CULL = 1,          // skinned positions, vq, vz, vnrm and the pair's out-of-range word
+  VERTEX_FOR_LISTS = 2,         // vab
+  VERTEX_ALL = 3
+};
+hipError_t launch_vertex(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, VertexOut out, hipStream_t s);
 hipError_t launch_cull(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, hipStream_t s);
 hipError_t launch_hist(const FrameArgs& a, uint32_t blk0, uint32_t nblk, hipStream_t s);
 hipError_t launch_scan(const FrameArgs& a, uint32_t sblk0, uint32_t nsblk, uint32_t part0, uint32_t nparts,

@@ -460,6 +460,9 @@ __device__ __forceinline__ VertexRecord shade_vertex(const FrameArgs& a, const F
 // scalar registers held the occupancy at six wavefronts a SIMD and cost an
 // LDS read per light and field: 112 us; scalar, but with 65 registers (seven
 // wavefronts), 104 us.
+// kOut: which of its outputs are written (a frame with lean records runs it
+// twice, see record_scratch).
+template <uint32_t kOut>
 __global__ __launch_bounds__(256, 8) void k_vertex(FrameArgs a, uint32_t blk0) {
   const uint32_t lb = frame_block(a, FC_VCHUNKS, 1);
   if (lb == kNoBlock) return;
@@ -486,16 +489,20 @@ __global__ __launch_bounds__(256, 8) void k_vertex(FrameArgs a, uint32_t blk0) {
     const uint32_t o = vbase + i;
     V3 vp;
     const VertexRecord r = shade_vertex(a, fc, P, flags, vmin + i, lds_bones ? s_bone_rows : nullptr, s_umvp, vp);
-    if (normals) {   // model.go:814-818: the rotation applied to the position; colour camera.go:1718-1720
+    if ((kOut & VERTEX_FOR_CULL) && normals) {   // model.go:814-818: the rotation applied to the position; colour camera.go:1718-1720
       const V3 tn = mult_vec(load_uniform(&P.nrot), vp);
       a.vnrm[o] = make_float4(tn.x * 0.5f + 0.5f, tn.y * 0.5f + 0.5f, tn.z * 0.5f + 0.5f, 0.0f);
     }
-    a.vab[2 * (size_t)o + 0] = r.a;
-    a.vab[2 * (size_t)o + 1] = r.b;
-    a.vq[o] = r.q;
-    a.vz[o] = r.zin ? 1 : 0;
-    out_of_range |= !r.zin;
-    if (skinned) a.vpos[o] = make_float4(vp.x, vp.y, vp.z, 0.0f);
+    if (kOut & VERTEX_FOR_LISTS) {
+      a.vab[2 * (size_t)o + 0] = r.a;
+      a.vab[2 * (size_t)o + 1] = r.b;
+    }
+    if (kOut & VERTEX_FOR_CULL) {
+      a.vq[o] = r.q;
+      a.vz[o] = r.zin ? 1 : 0;
+      out_of_range |= !r.zin;
+      if (skinned) a.vpos[o] = make_float4(vp.x, vp.y, vp.z, 0.0f);
+    }
   }
   // a pair with no vertex out of the Z range needs no look at vz in the cull
   if (__ballot(out_of_range) && threadIdx.x % 64 == 0) a.stats[4 * p + 3] = 1u;   // every writer stores the same word
@@ -1169,7 +1176,7 @@ __global__ __launch_bounds__(256) void k_scatter4(FrameArgs a, uint32_t blk0) {
   // less they are still cached and reading them only costs (113 and 110
   // against 35 and 25).
   float touch = 0.0f;
-  if (a.counts ? a.counts[FC_SUMV] > kTouchVertices : a.touch_records != 0) {
+  if (a.counts ? a.counts[FC_SUMV] > kTouchVertices && !a.lean : a.touch_records != 0) {
     constexpr uint32_t kLine = 128 / sizeof(float);
     const uint32_t v0 = (uint32_t)((uint64_t)P.vcount * tl / P.ntiles);
     const uint32_t nv = (uint32_t)((uint64_t)P.vcount * (tl + 1) / P.ntiles) - v0;
@@ -1714,9 +1721,13 @@ hipError_t launch_uniforms(const FrameArgs& a, uint32_t part0, uint32_t nparts, 
   hipLaunchKernelGGL(k_uniforms, dim3(nparts), dim3(kUniformThreads), 0, s, a, part0, nparts);
   return hipGetLastError();
 }
-hipError_t launch_vertex(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, hipStream_t s) {
+hipError_t launch_vertex(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, VertexOut out, hipStream_t s) {
   if (!nblk) return hipSuccess;
-  hipLaunchKernelGGL(k_vertex, dim3(nblk), dim3(threads), 0, s, a, blk0);
+  switch (out) {
+    case VERTEX_FOR_CULL: hipLaunchKernelGGL(k_vertex<VERTEX_FOR_CULL>, dim3(nblk), dim3(threads), 0, s, a, blk0); break;
+    case VERTEX_FOR_LISTS: hipLaunchKernelGGL(k_vertex<VERTEX_FOR_LISTS>, dim3(nblk), dim3(threads), 0, s, a, blk0); break;
+    default: hipLaunchKernelGGL(k_vertex<VERTEX_ALL>, dim3(nblk), dim3(threads), 0, s, a, blk0); break;
+  }
   return hipGetLastError();
 }
 hipError_t launch_cull(const FrameArgs& a, uint32_t blk0, uint32_t nblk, uint32_t threads, hipStream_t s) {

@@ -4,7 +4,8 @@
 // The frame's tables (per-pair uniforms, lights, block prefixes, palettes)
 // and its scratch (vertex records, depth keys, survivor records, histograms,
 // per-pair stats) come from one file-scope device array of
-// kNoallocRoom bytes per GPU, which each GPU holds until the process ends.  The host side reaches it only through the address
+// T3D_NOALLOC_SCRATCH_BYTES per GPU, which each GPU holds until the process
+// ends.  The host side reaches it only through the address
 // hipGetSymbolAddress returns for the current device: the array's name in
 // host code is a host-side stand-in, not a device address.
 //
@@ -20,7 +21,7 @@
 
 namespace t3d {
 
-static __device__ __align__(256) uint8_t scratch[kNoallocRoom];
+static __device__ __align__(256) uint8_t scratch[T3D_NOALLOC_SCRATCH_BYTES];
 
 namespace {
 
@@ -69,7 +70,6 @@ extern "C" t3d_status t3d_render_noalloc(t3d_ctx* c, t3d_frame* f, const t3d_ren
   Placement pl;
   pl.scratch = reinterpret_cast<uint8_t*>(c->noalloc_scratch);
   pl.scratch_bytes = T3D_NOALLOC_SCRATCH_BYTES;
-  pl.scratch_room = kNoallocRoom;
   pl.pinned_tables = c->pinned;
   pl.pinned_stats = reinterpret_cast<uint32_t*>(c->pinned + kPinnedTables);
   pl.color = color_vertices;

@@ -222,8 +222,6 @@ hipError_t noalloc_scratch_address(int device, void** out);
 constexpr uint32_t kHostUniforms = 192, kHostLights = 2048;
 constexpr uint32_t kHostModels = 640;   // frames of at most so many models have their pairs built on the host
 constexpr uint64_t kPinnedTables = 64 << 10;
-// Its size: a quarter over the limit that frames are counted against.
-constexpr uint64_t kNoallocRoom = T3D_NOALLOC_SCRATCH_BYTES + T3D_NOALLOC_SCRATCH_BYTES / 4;
 t3d_status dev_alloc(t3d_ctx* c, DevBuf& b, uint64_t bytes);
 // Grow `b` to at least `bytes` (contents discarded); the caller holds ctx->mu.
 t3d_status ensure(t3d_ctx* c, DevBuf& b, uint64_t& cap, uint64_t bytes);
@@ -243,8 +241,7 @@ t3d_status validate_desc(t3d_ctx* c, const t3d_render_desc* desc);
 // tables and scratch are carved from `scratch`, its outputs are the caller's.
 struct Placement {
   uint8_t* scratch = nullptr;
-  uint64_t scratch_bytes = 0;    // what a frame may count (T3D_NOALLOC_SCRATCH_BYTES)
-  uint64_t scratch_room = 0;     // bytes at `scratch`
+  uint64_t scratch_bytes = 0;
   uint8_t* pinned_tables = nullptr;   // the context's pinned staging, kPinnedTables bytes ...
   uint32_t* pinned_stats = nullptr;   // ... and 16 bytes for each of kHostUniforms pairs
   t3d_vertex* color = nullptr;
@@ -260,8 +257,9 @@ struct Placement {
 // memory.
 // With device_stage, a frame that allows it (and whose tuning asks for it) has its model-level stage run on the
 // device: frustum tests, render pairs and their slices are then known only after the frame (frame_collect).
+// admitted: the frame may take no more than estimate_job_bytes of its jobs.
 t3d_status frame_build(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* const* descs, uint32_t ndesc,
-                       const Placement* place = nullptr, bool device_stage = false);
+                       const Placement* place = nullptr, bool device_stage = false, bool admitted = false);
 // Runs a frame built with a placement on `stream` and waits for it: table
 // upload, the chain (per pair for the plain form, one
 // chain for the batched form; never a graph), stats readback.  Calls no
@@ -295,6 +293,7 @@ t3d_status frame_download_range(t3d_ctx* c, const t3d_frame* f, uint32_t p0, uin
                                 const DownloadParts& parts, PackBuf& pack, std::string* err_out = nullptr);
 void pack_release(t3d_ctx* c, PackBuf& pack);
 // Frame memory a job may need (scratch + outputs + tables), before frustum culling.
+constexpr uint64_t kEstimateExtra = 64 << 10;   // of each job's, for small tables and rounding
 uint64_t estimate_job_bytes(t3d_ctx* c, const t3d_render_desc* desc);
 
 }  // namespace t3d
