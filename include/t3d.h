@@ -520,9 +520,8 @@ typedef struct {
   uint32_t model_stage;              /* 1: the batched form runs the model-level stage (frustum test, render
                                         pairs and their order, per-pair slices) on the device when the
                                         frame allows it: no dynamic batch, RenderDepth on, every model at a
-                                        finite distance from its camera; 0: always on the host.  Until a
-                                        shape is set or autotuned, 1 leaves frames of up to 640 models
-                                        to the host */
+                                        finite distance from its camera; 0: always on the host; 2 (as a
+                                        context starts): as 1, but frames of up to 640 models on the host */
 } t3d_tuning;
 t3d_status t3d_get_tuning(const t3d_ctx* ctx, t3d_tuning* out);
 t3d_status t3d_set_tuning(t3d_ctx* ctx, const t3d_tuning* tuning);

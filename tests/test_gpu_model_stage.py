@@ -8,6 +8,7 @@ import pytest
 
 from tetra3d_amd import _abi as A
 from tetra3d_amd import workloads as W
+from tetra3d_amd.runtime import Context
 from tetra3d_amd.scene import Material, Model, Scene, World, DirectionalLight, Camera
 from tests.feature_scenes import feature_scene, pair_order_scene
 from tests.parity import compare_frames
@@ -45,14 +46,42 @@ def test_stage_runs_where_it_applies(gpu_ctx, oracle):
 
 
 @pytest.mark.gpu
-def test_feature_scenes_host_build(gpu_ctx, oracle):
-    """The feature scenes the stage would take, built on the host instead
-    (the default takes them on the device in test_gpu_features)."""
-    saved = _with_stage(gpu_ctx, 0)
+def test_tuning_round_trip():
+    """A small frame is built on the host as a context starts; setting the tuning that the context has, or another field
+    of it, changes nothing about that; model_stage 1 takes the frame to the device, and what was saved takes it back."""
+    wl = pair_order_scene(1)
+    with Context(0) as ctx:
+        def staged():
+            ctx.profile(True)
+            ctx.profile_read(reset=True)
+            ctx.render_workload(wl)
+            ctx.profile(False)
+            return "k_models" in ctx.profile_read(reset=True)
+
+        saved = ctx.tuning()
+        print("tuning round trip", saved.model_stage, flush=True)
+        assert not staged()
+        ctx.set_tuning()
+        assert not staged()
+        ctx.set_tuning(store_mode=18)
+        assert not staged()
+        ctx.set_tuning(model_stage=1)
+        assert staged()
+        ctx._check(ctx.L.t3d_set_tuning(ctx.ctx, saved))
+        assert not staged()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("on", [0, 1], ids=["host", "device"])
+def test_feature_scenes_host_build(gpu_ctx, oracle, on):
+    """The feature scenes built on the host whatever their size, and by the
+    stage where it applies (as a context starts, scenes so small are left to
+    the host)."""
+    saved = _with_stage(gpu_ctx, on)
     try:
         for seed in range(40):
             wl = feature_scene(seed)
-            print("feature scene", seed, "host build", flush=True)
+            print("feature scene", seed, "stage", on, flush=True)
             compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
     finally:
         gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
@@ -95,18 +124,22 @@ def _transparent_field(seed, n, spots=6):
 def test_transparent_order_on_device(gpu_ctx, oracle, n):
     """Hundreds of transparents at shared distances with several render
     orders, in one and in more than one 1024-candidate chunk of k_plist."""
-    for seed in range(2):
-        wl = _transparent_field(seed, n)
-        print("transparent field", seed, n, flush=True)
-        s = compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
-        assert s["pairs"] > 0
+    saved = _with_stage(gpu_ctx, 1)
+    try:
+        for seed in range(2):
+            wl = _transparent_field(seed, n)
+            print("transparent field", seed, n, flush=True)
+            s = compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
+            assert s["pairs"] > 0
+    finally:
+        gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
 
 
 @pytest.mark.gpu
 def test_cubes_camera_turning(gpu_ctx, oracle):
     """4,096 cubes under a turning camera: the visible set changes every
-    frame while the launch shape (sized for every cube drawn) and its graph
-    stay the same."""
+    frame while the launch shape (sized for every cube drawn) stays the
+    same."""
     wl = W.cubes_scene()
     counts = []
     for k, yaw in enumerate([0.0, 0.4, 1.3, 3.0]):

@@ -1,6 +1,6 @@
 """Frames of small render pairs, which one workgroup each draws whole: pairs at and one past the sizes where the
-workgroup changes or the chain of passes takes over, static and skinned, in the three sort modes, against the oracle
-bit for bit."""
+workgroup changes or the chain of passes takes over, static and skinned, in the three sort modes, built on the host and
+on the device, against the oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -28,10 +28,15 @@ def _mesh(v, t, seed):
     return Mesh("m%d" % seed, pos, nrm, idx, colors=np.c_[r.random((v, 3)), np.ones(v)], uvs=r.random((v, 2)))
 
 
+def _one_workgroup_each(v, t, count):
+    return (v <= 1024 and t <= 2048) or (v <= 2816 and t <= 5632 and count >= 64)
+
+
 @pytest.mark.gpu
+@pytest.mark.parametrize("stage", [2, 1], ids=["host", "device"])
 @pytest.mark.parametrize("visible", [True, False], ids=["culled", "all"])
 @pytest.mark.parametrize("size", SIZES, ids=["v%d_t%d_x%d" % s for s in SIZES])
-def test_pair_sizes(gpu_ctx, oracle, size, visible):
+def test_pair_sizes(gpu_ctx, oracle, size, visible, stage):
     v, t, count = size
     r = np.random.default_rng(7)
     meshes = [_mesh(v, t, k) for k in range(min(count, 3))]
@@ -53,6 +58,21 @@ def test_pair_sizes(gpu_ctx, oracle, size, visible):
     cam = Camera("camera", 800, 450)
     cam.process_only_visible = visible
     wl = W.Workload("pairs", cam, Scene("pairs", W._world(0.2)), W.icosphere_scene().lights, models)
-    print("pairs", size, visible, flush=True)
-    s = compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
-    assert s["survivors"] == count * t if not visible else s["survivors"] >= 0
+    print("pairs", size, visible, stage, flush=True)
+    saved = gpu_ctx.tuning()
+    gpu_ctx.set_tuning(model_stage=stage)
+    try:
+        gpu_ctx.profile(True)
+        gpu_ctx.profile_read(reset=True)
+        got = gpu_ctx.render_workload(wl)
+        ran = gpu_ctx.profile_read(reset=True)
+    finally:
+        gpu_ctx.profile(False)
+        gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
+    assert ("k_pair" in ran) == _one_workgroup_each(*size) != ("k_cull" in ran)
+    assert ("k_models" in ran) == (stage == 1 and visible)     # without culling the host builds every frame
+    s = compare_frames(got, oracle.render_workload(wl))
+    if not visible:
+        assert s["survivors"] == count * t
+    elif t > 2:                               # some of each mesh's triangles lie behind the camera or face away
+        assert 0 < s["survivors"] < count * t

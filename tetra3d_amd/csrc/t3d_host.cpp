@@ -1335,11 +1335,11 @@ bool few_models(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t 
 // the tuning asks for it, no model is dynamically batched, every camera has
 // RenderDepth on (its solids then keep model order), and no drawable model is
 // at a NaN distance from its camera (the transparents' comparator is then a
-// strict weak order, so a stable sort by it is Go's SliceStable's order).  Until a shape is
-// set or autotuned, a frame of few models is left to the host.
+// strict weak order, so a stable sort by it is Go's SliceStable's order).  With model_stage 2 a frame
+// of few models is left to the host.
 bool stage_applies(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
   if (!c->tuning.model_stage) return false;
-  if (c->stage_auto && few_models(c, descs, ndesc)) return false;
+  if (c->tuning.model_stage == 2 && few_models(c, descs, ndesc)) return false;
   for (uint32_t j = 0; j < ndesc; j++) {
     const t3d_render_desc* d = descs[j];
     if (!d || !d->camera || !d->camera->render_depth || d->process_all_triangles) return false;
@@ -3275,9 +3275,8 @@ t3d_status t3d_set_tuning(t3d_ctx* c, const t3d_tuning* t) {
   if (t->vertex_split > 1) return fail(c, T3D_ERR_INVALID_ARGUMENT, "tuning: vertex_split is 0 or 1");
   if (t->cull_block != 256 && t->cull_block != 512 && t->cull_block != 1024)
     return fail(c, T3D_ERR_INVALID_ARGUMENT, "tuning: cull_block is 256, 512 or 1024");
-  if (t->model_stage > 1) return fail(c, T3D_ERR_INVALID_ARGUMENT, "tuning: model_stage is 0 or 1");
+  if (t->model_stage > 2) return fail(c, T3D_ERR_INVALID_ARGUMENT, "tuning: model_stage is 0, 1 or 2");
   c->tuning = *t;
-  c->stage_auto = false;
   return T3D_OK;
 }
 
@@ -3288,8 +3287,6 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
   if (!c || !f || !desc) return T3D_ERR_INVALID_ARGUMENT;
   reps = std::max<uint32_t>(reps, 1);
   const t3d_tuning base = c->tuning;
-  const bool base_auto = c->stage_auto;
-  c->stage_auto = false;   // a candidate's model_stage is what it says
   t3d_render_desc d = *desc;
   d.exec_mode = T3D_EXEC_BATCHED;
   auto valid = [](const t3d_tuning& t) {
@@ -3398,7 +3395,6 @@ t3d_status t3d_autotune(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, u
   if (f2) (void)t3d_frame_destroy(c, f2);
   if (st) {
     c->tuning = base;
-    c->stage_auto = base_auto;
     return st;
   }
   c->tuning = best;

@@ -190,9 +190,7 @@ struct t3d_ctx {
   std::string err;
   // Launch shape.  No graph: replaying one puts about 13 us before a frame's first kernel (512 mixed models 549 us a
   // frame with it, 535 without; 4,096 cubes 219 and 207), and the chain's launches are enqueued faster than they run.
-  t3d_tuning tuning{256, 1, 2048, 4, 0, 2, 8, 1, 0, 256, 1};
-  // until a launch shape is set by hand or autotuned: frames of few models don't use the model stage
-  bool stage_auto = true;
+  t3d_tuning tuning{256, 1, 2048, 4, 0, 2, 8, 1, 0, 256, 2};
   // Guards resources, the budget and err between callers and the serving
   // thread; frame builds hold it, device work runs outside it.
   std::mutex mu;
