@@ -267,3 +267,56 @@ def test_failed_batch_build_retries_jobs_alone(pool):
                   "failed", st.failed, flush=True)
             # every job completed alone, and at least one batch of several failed to build and was split
             assert st.completed == len(order) and st.failed == 0 and st.batches > st.completed
+
+
+def test_release_while_the_device_is_waited_for():
+    """Jobs are submitted and released while another thread makes the context wait for the device (a light volume that is
+    freed, a frame that grows): the slots' completions still come through."""
+    import ctypes as C
+    import threading
+    import time
+    from tetra3d_amd.runtime import Context
+    from tetra3d_amd.scene import LightVolume
+    from tetra3d_amd.serving import Server
+    wls = [W.mixed_scene(seed=3 + k, count=2 + 2 * k) for k in range(3)]
+    with Context(0) as ctx:
+        for wl in wls:
+            ctx.prepare(wl)
+        inputs = [ctx.inputs(w.camera, w.scene, w.lights, w.models) for w in wls]
+        stop, done, errors = time.perf_counter() + 2, [], []
+
+        def waits():
+            while time.perf_counter() < stop:
+                v = LightVolume("v", (0, 0, 0), (8, 8, 8), (1, 1, 1))
+                ctx.upload_volume(v)
+                ctx._check(ctx.L.t3d_volume_free(ctx.ctx, v.handle))
+                f = C.c_void_p()
+                ctx._check(ctx.L.t3d_frame_create(ctx.ctx, C.byref(f)))
+                for k in (0, 2):
+                    ctx._check(ctx.L.t3d_render(ctx.ctx, f, C.byref(inputs[k].render)))
+                ctx._check(ctx.L.t3d_frame_destroy(ctx.ctx, f))
+
+        def serves():
+            with Server(ctx, slots=4, max_batch_jobs=2) as srv:
+                while time.perf_counter() < stop:
+                    jobs = [srv.submit_inputs(inputs[k % 3]) for k in range(12)]
+                    for j in jobs:
+                        srv.wait(j, 20000)
+                        srv.release(j)
+                        done.append(j)
+
+        def run(work):
+            try:
+                work()
+            except Exception as e:      # reported by the test's own thread
+                errors.append(e)
+
+        print("release while the device is waited for", flush=True)
+        threads = [threading.Thread(target=run, args=(w,), daemon=True) for w in (waits, serves)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(40)
+        assert not any(t.is_alive() for t in threads), "locked up after %d jobs" % len(done)
+        assert not errors, errors
+        assert len(done) > 20

@@ -98,7 +98,6 @@ struct t3d_server {
   t3d_ctx* ctx = nullptr;
   t3d_server_config cfg{};
   std::mutex mu;
-  std::condition_variable cv_work;   // wakes the worker (submit, release, stop)
   std::condition_variable cv_done;   // wakes waiters
   std::deque<uint64_t> queue;
   std::unordered_map<uint64_t, std::unique_ptr<Job>> jobs;
@@ -111,7 +110,13 @@ struct t3d_server {
   // readable under mu (counted with the frames the server holds)
   t3d::PackBuf pack;
   std::atomic<uint64_t> pack_bytes{0};
-  uint64_t wakeups = 0;                  // slot completions signalled from the slot streams
+  // Wakes the worker (submit, release, stop, a slot's completion): counted under a lock of its own, which nobody holds
+  // while waiting for anything.  The slot streams' callbacks take only this one: whoever waits for the device holds
+  // ctx->mu (a frame that grows, a resource that is freed), a thread that holds mu may wait for ctx->mu (drop_job), and a
+  // callback that wanted mu would then keep the device from finishing.
+  std::mutex wake_mu;
+  std::condition_variable cv_work;
+  uint64_t wakeups = 0;
   std::thread worker;
   bool stop = false;
   uint64_t next_id = 1, next_batch = 1;
@@ -126,6 +131,14 @@ struct t3d_server {
 };
 
 namespace {
+
+void wake_worker(t3d_server* s) {
+  {
+    std::lock_guard<std::mutex> lk(s->wake_mu);
+    s->wakeups++;
+  }
+  s->cv_work.notify_one();
+}
 
 // Called with ctx->mu held: copies a descriptor and everything it points to.
 t3d_status copy_desc(t3d_ctx* c, const t3d_render_desc* in, Job& j) {
@@ -346,15 +359,10 @@ void requeue_solo(t3d_server* s, Batch* b) {
 }
 
 // Slot stream callback after a batch's chain: wakes the worker, which then
-// finds the slot's completion event done.  Runs on a runtime thread; takes
-// the server lock and calls no HIP function.
+// finds the slot's completion event done.  Runs on a runtime thread and calls
+// no HIP function.
 void slot_done(void* arg) {
-  t3d_server* s = static_cast<t3d_server*>(arg);
-  {
-    std::lock_guard<std::mutex> lk(s->mu);
-    s->wakeups++;
-  }
-  s->cv_work.notify_one();
+  wake_worker(static_cast<t3d_server*>(arg));
 }
 
 // Called with s->mu held: the batch never ran (or its launch failed).
@@ -381,6 +389,11 @@ void worker_main(t3d_server* s) {
   (void)hipSetDevice(s->ctx->device);
   std::unique_lock<std::mutex> lk(s->mu);
   for (;;) {
+    uint64_t seen;
+    {
+      std::lock_guard<std::mutex> wl(s->wake_mu);
+      seen = s->wakeups;
+    }
     bool progressed = false;
     bool running = false;
     for (int i = 0; i < (int)s->slots.size(); i++) {
@@ -508,8 +521,14 @@ void worker_main(t3d_server* s) {
     }
     if (!progressed) {
       // woken by submit, release, stop, or a slot stream's completion callback; the timeout is only a safety net
-      if (running) s->cv_work.wait_for(lk, std::chrono::milliseconds(2));
-      else s->cv_work.wait(lk);
+      lk.unlock();
+      {
+        std::unique_lock<std::mutex> wl(s->wake_mu);
+        const auto woken = [&] { return s->wakeups != seen; };
+        if (running) s->cv_work.wait_for(wl, std::chrono::milliseconds(2), woken);
+        else s->cv_work.wait(wl, woken);
+      }
+      lk.lock();
     }
   }
 }
@@ -567,7 +586,7 @@ t3d_status t3d_server_destroy(t3d_server* s) {
     s->queue.clear();
     s->stop = true;
   }
-  s->cv_work.notify_all();
+  wake_worker(s);
   s->worker.join();
   std::vector<t3d_frame*> frames;
   {
@@ -632,7 +651,7 @@ t3d_status t3d_job_submit(t3d_server* s, const t3d_render_desc* desc, uint64_t* 
   *out_job = j->id;
   s->queue.push_back(j->id);
   s->jobs[j->id] = std::move(j);
-  s->cv_work.notify_one();
+  wake_worker(s);
   return T3D_OK;
 }
 
@@ -776,7 +795,7 @@ t3d_status t3d_job_release(t3d_server* s, uint64_t job) {
   if (j.pins) return T3D_ERR_BUSY;
   release_job(s, j);
   s->jobs.erase(it);
-  s->cv_work.notify_one();
+  wake_worker(s);
   return T3D_OK;
 }
 
