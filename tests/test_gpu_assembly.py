@@ -53,10 +53,22 @@ def test_chunk_edges(gpu_ctx, oracle, tile, split, normals, mode):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("counts", [[5], [12, 12, 12], [300, 40], [1, 2000]])
-def test_small_pairs(gpu_ctx, oracle, counts):
-    """Frames whose largest pair is smaller than a tile launch fewer blocks per tile."""
-    wl = _scene(counts, False)
-    print("assembly small", counts, flush=True)
-    s = compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
+@pytest.mark.parametrize("normals", [False, True], ids=["lists", "normals"])
+@pytest.mark.parametrize("counts", [[5], [12, 12, 12], [300, 40], [256, 257], [1, 2000]])
+def test_small_pairs(gpu_ctx, oracle, counts, normals):
+    """Frames whose largest pair is smaller than a tile: with normal lists the chain draws them, with fewer blocks per
+    tile in its assembly (1, 1, 2, 2 and the full 8); without, one workgroup draws each pair (but for the last frame's,
+    which are too large for that)."""
+    wl = _scene(counts, normals)
+    print("assembly small", counts, normals, flush=True)
+    gpu_ctx.profile(True)
+    try:
+        gpu_ctx.profile_read(reset=True)
+        got = gpu_ctx.render_workload(wl)
+        ran = gpu_ctx.profile_read(reset=True)
+    finally:
+        gpu_ctx.profile(False)
+    chain = normals or 3 * max(counts) > 2816
+    assert ("k_assemble" in ran) == chain == ("k_pair" not in ran)
+    s = compare_frames(got, oracle.render_workload(wl))
     assert s["survivors"] == sum(counts)

@@ -15,26 +15,48 @@ SCENES = {
 }
 
 
+STORE_MODES = [0, 1, 2, 3, 4, 6, 8, 10, 12, 14, 16, 18, 20, 22, 34, 38, 50, 54, 80, 82, 114]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("store_mode", [0, 1, 2, 3, 4, 6, 8, 10, 12, 14, 16, 18, 20, 22, 34, 38, 50, 54, 80, 82, 114],
-                         ids=["staged", "direct", "staged_nt", "direct_nt", "half", "half_nt", "pipe", "pipe_nt",
-                              "pipe_half", "pipe_half_nt", "w4", "w4_nt", "w4_half", "w4_half_nt", "one_nt",
-                              "one_half_nt", "w4_one_nt", "w4_one_half_nt", "w4_noswz", "w4_nt_noswz",
-                              "w4_one_nt_noswz"])
+@pytest.mark.parametrize("store_mode", [0, 2, 80, 82], ids=["plain", "nt", "noswz", "nt_noswz"])
 @pytest.mark.parametrize("mode", [A.EXEC_BATCHED, A.EXEC_PLAIN], ids=["batched", "plain"])
 @pytest.mark.parametrize("scene", list(SCENES))
 def test_scene_parity(gpu_ctx, oracle, scene, mode, store_mode):
+    """The four kinds of assembly that the store modes choose among: streaming stores or not, block order."""
     wl = SCENES[scene]()
     print("parity", scene, "mode", mode, "store_mode", store_mode, "tris", wl.triangle_count, flush=True)
+    saved = gpu_ctx.tuning()
     gpu_ctx.set_tuning(store_mode=store_mode)
     try:
         g = gpu_ctx.render_workload(wl, exec_mode=mode)
     finally:
-        gpu_ctx.set_tuning(store_mode=2)
+        gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
     o = oracle.render_workload(wl)
     s = compare_frames(g, o)
     print(s, flush=True)
     assert s["survivors"] > 0
+
+
+@pytest.mark.gpu
+def test_store_modes_accepted(gpu_ctx, oracle):
+    """Every store mode that a saved tuning may hold is accepted and gives the same frame; others are refused."""
+    from tetra3d_amd.runtime import T3DError
+    wl = SCENES["mixed_48"]()
+    want = oracle.render_workload(wl)
+    saved = gpu_ctx.tuning()
+    try:
+        for store_mode in range(128):
+            if store_mode not in STORE_MODES:
+                with pytest.raises(T3DError) as e:
+                    gpu_ctx.set_tuning(store_mode=store_mode)
+                assert e.value.status == A.T3D_ERR_INVALID_ARGUMENT
+                continue
+            print("store mode", store_mode, flush=True)
+            gpu_ctx.set_tuning(store_mode=store_mode)
+            compare_frames(gpu_ctx.render_workload(wl), want)
+    finally:
+        gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
 
 
 SHAPES = [  # (triangle_tile, scatter_waves, assemble_split, xcd_swizzle, vertex_split, cull_block)
@@ -47,8 +69,8 @@ SHAPES = [  # (triangle_tile, scatter_waves, assemble_split, xcd_swizzle, vertex
 @pytest.mark.parametrize("shape", SHAPES, ids=["t%d_w%d_s%d_x%d_v%d_c%d" % s for s in SHAPES])
 @pytest.mark.parametrize("scene", ["heightfield_128", "mixed_48"])
 def test_launch_shapes_parity(gpu_ctx, oracle, scene, shape):
-    """Every tile size, scatter width, assembly split, block order and vertex
-    record layout gives the same frame."""
+    """Every tile size, scatter width, assembly split and block order gives
+    the same frame, and so does vertex_split, which changes nothing."""
     wl = SCENES[scene]()
     tile, waves, split, swz, vsplit, cblock = shape
     print("shape parity", scene, shape, flush=True)
