@@ -226,8 +226,7 @@ def add_cell_lights(rng, vol, lo, hi, n_lights=None, frac=0.3):
 def cell_lights_scene(seed, many=False):
     """Models inside a LightVolume whose cells name lights, in every shading
     mode, rigid and skinned, the volume in the scene lights and in a
-    LightGroup; `many` gives the volume 80 cell lights, so a pair's light list
-    passes what the vertex pass stages in LDS."""
+    LightGroup; `many` gives the volume 80 cell lights."""
     rng = np.random.default_rng(seed)
     lo, hi = np.array([-6, -4, -14], dtype=f32), np.array([6, 4, -3], dtype=f32)
     cam = Camera("cam", 640, 360)

@@ -34,9 +34,21 @@ def test_armature_past_level_walk(gpu_ctx, oracle, mode):
     assert s["survivors"] > 100
 
 
-def test_pose_changes_between_frames(gpu_ctx, oracle):
-    """Same launch shape every frame, so the batched form replays its graph;
-    only the poses and the armature parent move."""
+@pytest.fixture(params=["direct", "graph"])
+def launched(request, gpu_ctx):
+    """The context launching the batched form directly, or replaying it from
+    a HIP graph (frames built on the device, whose launch shape stays)."""
+    saved = gpu_ctx.tuning()
+    if request.param == "graph":
+        gpu_ctx.set_tuning(use_graph=1, model_stage=1)
+    yield gpu_ctx
+    gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
+
+
+def test_pose_changes_between_frames(launched, oracle):
+    """Same launch shape every frame, which a graph replays; only the poses
+    and the armature parent move."""
+    gpu_ctx = launched
     wl = posed_scene(2)
     rng = np.random.default_rng(5)
     for frame in range(4):
@@ -96,9 +108,10 @@ def animated_scene(seed):
 
 
 @pytest.mark.parametrize("mode", [A.EXEC_BATCHED, A.EXEC_PLAIN], ids=["batched", "plain"])
-def test_animated_matches_oracle(gpu_ctx, oracle, mode):
+def test_animated_matches_oracle(launched, oracle, mode):
     """Playheads before, inside, on and after the keyframes, frame after
-    frame (the batched form replays its graph with new playheads)."""
+    frame (which a graph replays with new playheads)."""
+    gpu_ctx = launched
     wl = animated_scene(10)
     for frame, t in enumerate([-0.5, 0.0, 0.125, 0.37, 0.5, 0.99, 1.0, 2.0]):
         for i, m in enumerate(wl.models):

@@ -138,8 +138,7 @@ def test_cell_lights(gpu_ctx, oracle, mode, many):
     cell's lights lights the vertex before the volume's colour, unskipped and
     whatever its visibility, with beginModel for the model at hand; rigid and
     skinned models in every shading mode, the volume in the scene lights and
-    in LightGroups; with 80 cell lights a pair's list passes the 64 lights
-    the vertex pass stages in LDS."""
+    in LightGroups; with a few cell lights and with 80."""
     for seed in range(4):
         wl = cell_lights_scene(seed, many)
         print("cell-lights scene", seed, "many", many, "mode", mode, flush=True)

@@ -42,10 +42,10 @@ def test_model_counts(fresh_ctx, oracle, count, large):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("count", [799, 801])
-def test_large_frames_in_flight(fresh_ctx, oracle, count):
+@pytest.mark.parametrize("count,graph", [(799, 0), (801, 0), (801, 1)])
+def test_large_frames_in_flight(fresh_ctx, oracle, count, graph):
     """Two frames of just under and just over 2.4 million vertices in flight, which overlap on the device or run in
-    turn: each equals the oracle's."""
+    turn, launched directly or from a graph: each equals the oracle's."""
     mesh = _mesh(3000, 5000, 3)
     r = np.random.default_rng(count)
     models = []
@@ -63,10 +63,15 @@ def test_large_frames_in_flight(fresh_ctx, oracle, count):
         wls.append(W.Workload("large", cam, Scene("large", W._world(0.2)), lights, models))
     fresh_ctx.prepare(wls[0])
     inputs = [fresh_ctx.inputs(w.camera, w.scene, w.lights, w.models) for w in wls]
-    print("large frames in flight", count, flush=True)
-    for _ in range(2):
-        for f, inp in zip(frames, inputs):
-            fresh_ctx.render_async(inp, f)
+    print("large frames in flight", count, graph, flush=True)
+    saved = fresh_ctx.tuning()
+    fresh_ctx.set_tuning(use_graph=graph)
+    try:
+        for _ in range(2):
+            for f, inp in zip(frames, inputs):
+                fresh_ctx.render_async(inp, f)
+    finally:
+        fresh_ctx.L.t3d_set_tuning(fresh_ctx.ctx, saved)
     for f, w in zip(frames, wls):
         fresh_ctx.wait(f)
         compare_frames(fresh_ctx.download(frame=f), oracle.render_workload(w))

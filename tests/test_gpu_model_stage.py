@@ -136,15 +136,21 @@ def test_transparent_order_on_device(gpu_ctx, oracle, n):
 
 
 @pytest.mark.gpu
-def test_cubes_camera_turning(gpu_ctx, oracle):
+@pytest.mark.parametrize("graph", [0, 1], ids=["direct", "graph"])
+def test_cubes_camera_turning(gpu_ctx, oracle, graph):
     """4,096 cubes under a turning camera: the visible set changes every
-    frame while the launch shape (sized for every cube drawn) stays the
-    same."""
+    frame while the launch shape (sized for every cube drawn), and with it a
+    graph of the launches, stays the same."""
     wl = W.cubes_scene()
     counts = []
-    for k, yaw in enumerate([0.0, 0.4, 1.3, 3.0]):
-        wl.camera.set_local_rotation(W.axis_angle_matrix((0, 1, 0), yaw))
-        print("cubes frame", k, "yaw", yaw, flush=True)
-        s = compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
-        counts.append(s["pairs"])
+    saved = gpu_ctx.tuning()
+    gpu_ctx.set_tuning(use_graph=graph)
+    try:
+        for k, yaw in enumerate([0.0, 0.4, 1.3, 3.0]):
+            wl.camera.set_local_rotation(W.axis_angle_matrix((0, 1, 0), yaw))
+            print("cubes frame", k, "yaw", yaw, "graph", graph, flush=True)
+            s = compare_frames(gpu_ctx.render_workload(wl), oracle.render_workload(wl))
+            counts.append(s["pairs"])
+    finally:
+        gpu_ctx.L.t3d_set_tuning(gpu_ctx.ctx, saved)
     assert len(set(counts)) > 1

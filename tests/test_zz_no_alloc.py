@@ -89,9 +89,8 @@ def test_noalloc_matches_render_twice_shrinking(mode):
 
 @pytest.mark.gpu
 def test_noalloc_cell_lights():
-    """A LightVolume whose cells name 80 lights (past the 64 the vertex pass
-    stages in LDS), skinned and rigid models: the no-alloc render matches
-    t3d_render bit for bit."""
+    """A LightVolume whose cells name 80 lights, skinned and rigid models: the
+    no-alloc render matches t3d_render bit for bit."""
     from tests.feature_scenes import cell_lights_scene
     wl = cell_lights_scene(2, many=True)
     hip = _hip()

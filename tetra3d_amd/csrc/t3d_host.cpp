@@ -5,8 +5,7 @@
 // computes on the CPU (camera.go:1269-1601, model.go:142-182, 600-695,
 // light.go beginRender/beginModel), decides the render-pair order exactly as
 // the reference does, and drives the kernel chain of t3d_kernels.hip in the
-// plain (one chain per render pair) or batched (one chain per frame, replayed
-// from a HIP graph) form.
+// plain (one chain per render pair) or batched (one chain per frame) form.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -266,9 +265,15 @@ uint64_t placed_charge(uint64_t V, uint64_t T) {
 
 // Whether a frame of `pairs` render pairs (or candidates) and T triangles in all is drawn by one workgroup per render
 // pair (k_pair) instead of the chain of passes over all pairs: where no pair is over kPairVertices and kPairTriangles; and
-// up to the larger limits where there are only a few, none skinned (one sphere of 2,562 vertices: 45 us a frame, 53 with
-// the chain; five uneven models 43 and 60; two skinned spheres 86 and 80), or many whose mean is at least half of the
-// largest, so that no workgroup is waited for long (64 skinned spheres 150 and 155, 256 of them 295 and 335).
+// up to the larger limits where there are only a few, none skinned, or many whose mean is at least half of the largest,
+// so that no workgroup is waited for long.  Synchronous frames, us with the chain and with k_pair:
+//   2,562 vertices, static    1: 57, 54   16: 68, 65   24: 70, 65   48: 79, 70   160: 120, 95
+//   2,562 vertices, skinned   1: 60, 62   16: 70, 74   32: 76, 77   48: 84, 81   64: 92, 84   160: 135, 117
+//   60 to 2,700 vertices      4: 49, 39   16: 56, 45   64: 65, 52   160: 86, 70
+// so both counts lie on the safe side: skinned pairs break even between 32 and 48, static ones gain at any number, and
+// uneven ones did so up to 2,700 vertices (200 models of up to 4,000: 141 with the chain, 151 with a k_pair that took
+// them).  The larger limits hold the 2,562-vertex sphere with 114 KB of LDS and are not where the gain ends either: with
+// room for 3,584 vertices and 7,168 triangles (143 KB), 16 grids of 3,249 vertices took 49 us instead of 56.
 bool pairs_fit(const t3d_frame* f, uint64_t pairs, uint64_t T, bool skinned, bool normals, bool groups) {
   if (normals || groups) return false;
   const uint64_t v = f->max_vertices, t = f->max_triangles;
@@ -1314,9 +1319,11 @@ t3d_status validate_desc(t3d_ctx* c, const t3d_render_desc* desc) {
 namespace {
 
 // A frame of at most kHostModels models and MeshParts: its pairs are built on the host, at about 0.1 us each, where the
-// stage's two kernels take 15 us and more on the device, and the readback of what they built another ten: 500 cubes
-// 80 us a frame and 96, 300 uneven models 345 and 358, 512 of them 535 and 554.  Past that the host's part is longer
-// than what it saves (4,096 cubes: 0.25 ms against 0.21).
+// stage's two kernels take 15 us and more on the device, and the readback of what they built another ten.  Us a frame
+// built on the host and on the device, synchronous / two in flight:
+//   cubes          300: 58, 65 / 31, 50   640: 66, 87 / 57, 56   1,000: 83, 96 / 69, 63   2,000: 133, 131 / 118, 106
+//   uneven models  300: 335, 348 / 311, 315   640: 705, 721 / 617, 620   1,000: 1,265, 1,265 / 1,119, 1,126
+// The line lies where cubes in flight break even; synchronous ones would gain up to about 1,800.
 bool few_models(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
   uint64_t pairs = 0;
   for (uint32_t j = 0; j < ndesc; j++) {

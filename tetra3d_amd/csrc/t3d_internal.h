@@ -117,7 +117,8 @@ struct alignas(16) LightGPU {
 };
 
 // Per (render pair, light) values from beginModel and the per-model skip,
-// written by k_uniforms (frame scratch, never uploaded).
+// written by k_uniforms into the frame's scratch, or by the host into its
+// tables (frames of few pairs).
 struct alignas(16) PartLight {
   float v[3];           // point: workingPosition; volume per-object mode: cell colour
   uint32_t light;       // index into the frame's LightGPU array

@@ -455,11 +455,11 @@ __device__ __forceinline__ VertexRecord shade_vertex(const FrameArgs& a, const F
   return r;
 }
 
-// Its vertices move about 105 bytes each (3.9 M of them: 410 MB in 94 us, 4.4
-// TB/s, where a copy reaches 4.7).  Light constants staged in LDS instead of
+// Its vertices move about 105 bytes each (3.9 M of them: 410 MB in 87 us, 4.7
+// TB/s, where a copy reaches 5.1).  Light constants staged in LDS instead of
 // scalar registers held the occupancy at six wavefronts a SIMD and cost an
-// LDS read per light and field: 112 us; scalar, but with 65 registers (seven
-// wavefronts), 104 us.
+// LDS read per light and field: 112 us, in a run that had 94 without; scalar,
+// but with 65 registers (seven wavefronts), 104 us.
 // kOut: which of its outputs are written (a frame with lean records runs it
 // twice, see record_scratch).
 template <uint32_t kOut>
@@ -1298,8 +1298,8 @@ __device__ __forceinline__ void store1(uint32_t* p, uint32_t v) {
 // follows the survivors more finely than the sort's tiles.
 //
 // What bounds it: the stores.  1.02 GB of lists (3.4 M triangles of 465 pairs)
-// take 212 us, 4.8 TB/s; a kernel that only stores the same lists takes 190
-// (242 with its runs 48 bytes off the lines).  Three float4 computed per
+// take 211 us, 4.8 TB/s; a kernel that only stores the same lists takes 190
+// (242 with its runs 48 bytes off the lines), a fill of as many bytes 150.  Three float4 computed per
 // corner and staged in LDS, nine rows a triangle, took 265 us.
 constexpr uint32_t kAsmThreads = 256;
 template <bool kNT, bool kNormals>
@@ -1389,14 +1389,15 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble(FrameArgs a, uint32_t 
 // CU); tri_vo is written for t3d_frame_download_triangles.
 //
 // kThreads, kV and kT: threads, and the most vertices and triangles a pair may
-// have (launch_pairs chooses).  LDS per block: 17 B a vertex, 8 B a triangle
+// have (launch_pairs chooses by the frame's largest, and refuses what no
+// variant holds, so the check below never finds a larger one).  LDS per block: 17 B a vertex, 8 B a triangle
 // and 1 KB a wavefront; 112 KB at the largest.
 //
 // What bounds it: instructions and latency while a workgroup shades (10 us a
 // round of 1,024 skinned vertices under six lights; 7 us before the first, of
-// cold loads), then the stores of the lists.  642 vertices alone: 19 us, where
-// the chain's six launches take 44; 4,096 cubes 16 us against 52; 256 skinned
-// characters of 2,562 vertices 83 us against 125.  Where one pair is much
+// cold loads), then the stores of the lists.  642 vertices alone: 16 us, where
+// the chain's six launches take 44; 4,096 cubes 12 us against 52; 256 skinned
+// characters of 2,562 vertices 82 us against 125.  Where one pair is much
 // larger than the others its workgroup is what the frame waits for (200
 // uneven models of up to 4,000 vertices: 151 us a frame against 141 with the
 // chain), so larger pairs come here only in even company (pairs_fit).

@@ -216,7 +216,10 @@ t3d_status fail(t3d_ctx* c, t3d_status st, const char* fmt, ...);
 // Device address of `device`'s copy of the no-allocation scratch array (t3d_noalloc.hip); the device must be
 // current.  Looked up once per device.
 hipError_t noalloc_scratch_address(int device, void** out);
-// Frames of at most this many render pairs (and per-light values) have their uniforms built on the host too.
+// Frames of at most this many render pairs (and per-light values) have their uniforms built on the host too.  Cubes, us
+// a frame with that and with k_uniforms, two in flight / synchronous: 50: 20, 37 / 39, 40; 100: 24, 39 / 46, 44; 192:
+// 31, 45 / 59, 49; 300: 43, 51 / 73, 57; 400: 55, 57 / 85, 66.  A compromise between the two: frames in flight gain up to
+// about 400 pairs, where the host's part runs beside the frame before, synchronous ones only up to about 60.
 constexpr uint32_t kHostUniforms = 192, kHostLights = 2048;
 constexpr uint32_t kHostModels = 640;   // frames of at most so many models have their pairs built on the host
 constexpr uint64_t kPinnedTables = 64 << 10;
