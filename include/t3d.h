@@ -651,6 +651,9 @@ t3d_status t3d_server_stats_reset(t3d_server* s);
  * instead of keeping an earlier render's value (tests pass a NaN pattern).
  * 0 turns it off.  No counterpart in the reference: a debugging aid. */
 t3d_status t3d_debug_poison_outputs(t3d_ctx* ctx, uint32_t word);
+/* Whether the frame's last t3d_render_async was a large one, which runs after
+ * the kernels of the large one before it (1), or overlaps with others (0). */
+t3d_status t3d_debug_frame_in_turn(const t3d_frame* frame, int32_t* out);
 
 /* Bounding spheres of n models as the frustum test computes them
  * (Model.onTransformUpdate, model.go:142-182): out_batched from the

@@ -1,6 +1,8 @@
 """Frames at and one past the model counts where the pairs stop being built on the host, the uniforms stop coming from
 it and the tile tables start, on a context whose tuning nobody has set, against the oracle bit for bit; and their
 lists downloaded with and without the triangle ids."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -75,3 +77,39 @@ def test_large_frames_in_flight(fresh_ctx, oracle, count, graph):
     for f, w in zip(frames, wls):
         fresh_ctx.wait(f)
         compare_frames(fresh_ctx.download(frame=f), oracle.render_workload(w))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("stage", [0, 1], ids=["host", "device"])
+@pytest.mark.parametrize("shown,turns", [(40, 0), (799, 0), (801, 1)])
+def test_what_is_drawn_decides_who_takes_turns(fresh_ctx, shown, turns, stage):
+    """820 models listed, 2.46 million vertices in all: their frames take turns only when over 2.4 million are drawn, by
+    the drawn pairs of a host-built frame or of a device-built one's last render; a frame that is waited for never does."""
+    mesh = _mesh(3000, 5000, 3)
+    models = []
+    for i in range(820):
+        m = Model("m%d" % i, mesh)
+        m.set_local_position(0.01 * (i % 100), 0, -6 if i < shown else 300)
+        models.append(m)
+    wl = W.Workload("listed", Camera("camera", 800, 450), Scene("listed", W._world(0.2)), W.icosphere_scene().lights, models)
+    fresh_ctx.prepare(wl)
+    inp = fresh_ctx.inputs(wl.camera, wl.scene, wl.lights, wl.models)
+    frame, out = fresh_ctx.new_frame(), C.c_int32()
+
+    def in_turn():
+        assert fresh_ctx.L.t3d_debug_frame_in_turn(frame, C.byref(out)) == 0
+        return out.value
+
+    print("drawn of the listed", shown, stage, flush=True)
+    saved = fresh_ctx.tuning()
+    fresh_ctx.set_tuning(model_stage=stage)
+    try:
+        for k in range(2):
+            fresh_ctx.render_async(inp, frame)
+            assert in_turn() == (turns if k or not stage else 0)
+            fresh_ctx.wait(frame)
+            assert len(fresh_ctx.pairs(frame)) == shown
+        fresh_ctx._check(fresh_ctx.L.t3d_render(fresh_ctx.ctx, frame, C.byref(inp.render)))
+        assert in_turn() == 0
+    finally:
+        fresh_ctx.L.t3d_set_tuning(fresh_ctx.ctx, saved)

@@ -3186,6 +3186,12 @@ t3d_status t3d_frame_download_triangles(t3d_ctx* c, const t3d_frame* f, uint32_t
   return frame_download_range(c, f, 0, np, c->stream, nullptr, nullptr, nullptr, ids, nullptr, parts, fm->pack);
 }
 
+t3d_status t3d_debug_frame_in_turn(const t3d_frame* f, int32_t* out) {
+  if (!f || !out) return T3D_ERR_INVALID_ARGUMENT;
+  *out = f->in_turn ? 1 : 0;
+  return T3D_OK;
+}
+
 t3d_status t3d_debug_model_spheres(const t3d_mat4* transforms, const float* dims, const uint8_t* skinned, uint32_t n,
                                    float* out_batched, float* out_scalar) {
   if (!transforms || !dims || !skinned || !out_batched || !out_scalar) return T3D_ERR_INVALID_ARGUMENT;

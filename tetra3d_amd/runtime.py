@@ -65,6 +65,7 @@ def lib():
     L.t3d_render_async.argtypes = [vp, vp, P(A.RenderDesc)]
     L.t3d_render_noalloc.argtypes = [vp, vp, P(A.RenderDesc), vp, vp, vp, C.c_uint64]
     L.t3d_debug_poison_outputs.argtypes = [vp, C.c_uint32]
+    L.t3d_debug_frame_in_turn.argtypes = [vp, P(C.c_int32)]
     L.t3d_frame_wait.argtypes = [vp, vp]
     L.t3d_frame_pairs.argtypes = [vp, P(C.c_uint32), P(P(A.PairResult))]
     L.t3d_frame_device_outputs.argtypes = [vp, P(vp), P(vp), P(vp)]
@@ -92,7 +93,7 @@ def lib():
                  "t3d_volume_free", "t3d_volume_set_cell_lights", "t3d_frame_create", "t3d_frame_destroy", "t3d_render", "t3d_frame_pairs",
                  "t3d_frame_device_outputs", "t3d_frame_download", "t3d_frame_download_triangles",
                  "t3d_profile_enable", "t3d_profile_read", "t3d_get_tuning", "t3d_set_tuning", "t3d_autotune",
-                 "t3d_selftest_fp", "t3d_selftest_copy", "t3d_debug_model_spheres", "t3d_animation_upload",
+                 "t3d_selftest_fp", "t3d_selftest_copy", "t3d_debug_model_spheres", "t3d_debug_frame_in_turn", "t3d_animation_upload",
                  "t3d_animation_free", "t3d_render_noalloc", "t3d_frame_device_normals",
                  "t3d_frame_download_normals", "t3d_texture_upload", "t3d_texture_free", "t3d_frame_rasterize",
                  "t3d_frame_device_images", "t3d_frame_download_images"):
