@@ -183,3 +183,6 @@ def test_triangles_need_no_device_memory(count):
         assert ctx.memory_used == used
         print("triangles at the budget", count, len(want), flush=True)
         np.testing.assert_array_equal(_triangle_ids(ctx, ctx.frame), want)
+        normals = np.zeros((3 * len(want), 12), dtype=np.float32)       # a list that the frame does not have
+        assert ctx.L.t3d_frame_download_normals(ctx.ctx, ctx.frame,
+                                                normals.ctypes.data_as(C.POINTER(A.Vertex))) == A.T3D_ERR_NOT_FOUND

@@ -2825,7 +2825,7 @@ static uint64_t pack_layout_bytes(uint64_t np, uint64_t verts, const DownloadPar
 DownloadParts download_parts(const t3d_frame* f, bool lists, bool normals, bool ids) {
   DownloadParts d;
   d.lists = lists;
-  d.normals = normals;
+  d.normals = normals && f->args.out_normal;   // (a frame without them refuses, and needs no room for that)
   d.pack_ids = ids && !f->placed;   // a placed frame's keys lie in an array that other frames use after it
   return d;
 }
