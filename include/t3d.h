@@ -521,7 +521,8 @@ typedef struct {
                                         pairs and their order, per-pair slices) on the device when the
                                         frame allows it: no dynamic batch, RenderDepth on, every model at a
                                         finite distance from its camera; 0: always on the host; 2 (as a
-                                        context starts): as 1, but frames of up to 640 models on the host */
+                                        context starts): as 1, but frames of up to 640 models on the host
+                                        unless use_graph is 1 */
 } t3d_tuning;
 t3d_status t3d_get_tuning(const t3d_ctx* ctx, t3d_tuning* out);
 t3d_status t3d_set_tuning(t3d_ctx* ctx, const t3d_tuning* tuning);

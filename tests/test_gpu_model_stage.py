@@ -65,6 +65,10 @@ def test_tuning_round_trip():
         assert not staged()
         ctx.set_tuning(store_mode=18)
         assert not staged()
+        ctx.set_tuning(use_graph=1)           # a graph wants launches that stay the same: the device's
+        assert staged()
+        ctx.set_tuning(use_graph=0)
+        assert not staged()
         ctx.set_tuning(model_stage=1)
         assert staged()
         ctx._check(ctx.L.t3d_set_tuning(ctx.ctx, saved))

@@ -1343,10 +1343,11 @@ bool few_models(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t 
 // RenderDepth on (its solids then keep model order), and no drawable model is
 // at a NaN distance from its camera (the transparents' comparator is then a
 // strict weak order, so a stable sort by it is Go's SliceStable's order).  With model_stage 2 a frame
-// of few models is left to the host.
+// of few models is left to the host; but not where its launches are replayed from a graph, which a host-built frame
+// needs anew whenever other models are in view.
 bool stage_applies(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
   if (!c->tuning.model_stage) return false;
-  if (c->tuning.model_stage == 2 && few_models(c, descs, ndesc)) return false;
+  if (c->tuning.model_stage == 2 && !c->tuning.use_graph && few_models(c, descs, ndesc)) return false;
   for (uint32_t j = 0; j < ndesc; j++) {
     const t3d_render_desc* d = descs[j];
     if (!d || !d->camera || !d->camera->render_depth || d->process_all_triangles) return false;
