@@ -397,7 +397,7 @@ t3d_status t3d_frame_destroy(t3d_ctx* ctx, t3d_frame* frame);
 t3d_status t3d_render(t3d_ctx* ctx, t3d_frame* frame, const t3d_render_desc* desc);
 
 /* The same render without the wait: builds the frame's tables, enqueues the
- * table upload (on the context's copy stream) and the kernel chain, and
+ * table upload (on the frame's own stream) and the kernel chain, and
  * returns.  A caller that alternates two frames overlaps the host work of
  * one Camera.Render with the device work of the previous one.  Rendering
  * into a frame that is still in flight waits for it first; its earlier

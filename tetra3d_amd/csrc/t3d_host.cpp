@@ -734,21 +734,14 @@ t3d_status t3d_ctx_create(int32_t device, uint64_t hbm_budget_bytes, t3d_ctx** o
     delete c;
     return T3D_ERR_DEVICE;
   }
-  if (hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking) != hipSuccess) {
-    (void)hipStreamDestroy(c->stream);
-    delete c;
-    return T3D_ERR_DEVICE;
-  }
   if (hipHostMalloc((void**)&c->pinned, kPinnedTables + 16ull * kHostUniforms, hipHostMallocDefault) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
-    (void)hipStreamDestroy(c->copy_stream);
     delete c;
     return T3D_ERR_DEVICE;
   }
   // this device's copy of the scratch array of t3d_render_noalloc, looked up with the device current
   if (noalloc_scratch_address(device, &c->noalloc_scratch) != hipSuccess) {
     (void)hipStreamDestroy(c->stream);
-    (void)hipStreamDestroy(c->copy_stream);
     (void)hipHostFree(c->pinned);
     delete c;
     return T3D_ERR_DEVICE;
@@ -761,14 +754,12 @@ t3d_status t3d_ctx_destroy(t3d_ctx* c) {
   if (!c) return T3D_ERR_INVALID_ARGUMENT;
   (void)hipSetDevice(c->device);
   (void)hipStreamSynchronize(c->stream);
-  (void)hipStreamSynchronize(c->copy_stream);
   for (auto& kv : c->meshes) dev_free(c, kv.second->buf);
   for (auto& kv : c->volumes) {
     dev_free(c, kv.second->buf);
     dev_free(c, kv.second->lists);
   }
   (void)hipStreamDestroy(c->stream);
-  (void)hipStreamDestroy(c->copy_stream);
   (void)hipHostFree(c->pinned);
   delete c;
   return T3D_OK;
@@ -3083,15 +3074,16 @@ t3d_status render_submit(t3d_ctx* c, t3d_frame* f, const t3d_render_desc* desc, 
   // uneven models, two frames in flight: 471 us a frame one after the other, 497 side by side).  What counts is what the
   // camera sees.  For a frame built on the device that is not known here: its handle's last render stands in, and a
   // wrong guess costs time only.
-  // Frames built on the host take the context's stream then, not one more: a process has four hardware queues, and with
-  // five streams (this one, the copies' and two frames' besides) two frames shared a queue and ran in turn whatever
-  // their size (20 uneven models 79 us a frame with five, 54 with four; a 1024 x 1024 grid 131 and 93).  One built on
-  // the device keeps its own, where its model stage, palettes and uniforms run beside the frame before, and waits for
+  // Frames built on the host take the context's stream then, not one more: a process has four hardware queues, for the
+  // null stream, the context's and two frames'.  With one or two more (one for the large frames, one for the tables'
+  // copies, which now go on the frame's own) two frames could share a queue, by the order in which the streams were
+  // made, and ran in turn whatever their size (20 uneven models 79 us a frame instead of 54; a 1024 x 1024 grid 131
+  // instead of 93; a 357 x 357 grid 72 instead of 45).  One built on the device keeps its own, where its model stage, palettes and uniforms run beside the frame before, and waits for
   // that frame's kernels ahead of its vertices (700 uneven models 704 us a frame, 738 all in turn; 1,000 of them 1,128
   // and 1,160; but on the host, with less to overlap, 512 of them 474 and 470).
   f->in_turn = !alone && f->drawn_vertices > kTouchVertices;
   hipStream_t stream = f->stream && (f->device_stage || !f->in_turn) ? f->stream : c->stream;
-  st = frame_launch(c, f, stream, c->copy_stream, desc->exec_mode, true, true, alone);
+  st = frame_launch(c, f, stream, f->stream ? f->stream : stream, desc->exec_mode, true, true, alone);
   if (st) return st;
   f->submitted = wall0;
   f->inflight = true;

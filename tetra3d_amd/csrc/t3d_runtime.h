@@ -177,7 +177,6 @@ struct t3d_frame {
 struct t3d_ctx {
   int device = 0;
   hipStream_t stream = nullptr;        // kernel chains of t3d_render / t3d_render_async
-  hipStream_t copy_stream = nullptr;   // table uploads, so they overlap the previous frame's kernels
   // the last large frame that t3d_render_async launched (render_submit): recorded after its kernels, and its stream
   hipEvent_t large_done = nullptr;
   hipStream_t large_on = nullptr;
