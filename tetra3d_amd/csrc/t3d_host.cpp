@@ -1312,9 +1312,10 @@ namespace {
 // A frame of at most kHostModels models and MeshParts: its pairs are built on the host, at about 0.1 us each, where the
 // stage's two kernels take 15 us and more on the device, and the readback of what they built another ten.  Us a frame
 // built on the host and on the device, synchronous / two in flight:
-//   cubes          300: 58, 65 / 31, 50   640: 66, 87 / 57, 56   1,000: 83, 96 / 69, 63   2,000: 133, 131 / 118, 106
-//   uneven models  300: 335, 348 / 311, 315   640: 705, 721 / 617, 620   1,000: 1,265, 1,265 / 1,119, 1,126
-// The line lies where cubes in flight break even; synchronous ones would gain up to about 1,800.
+//   cubes          300: 57, 65 / 30, 38   640: 66, 87 / 37, 56   1,000: 84, 97 / 52, 60   1,400: 104, 110 / 69, 67
+//                  2,000: 132, 132 / 95, 80   4,096: 247, 200 / 196, 110
+//   uneven models  150: 208, 217 / 142, 144   640: 708, 722 / 618, 618   1,000: 1,265, 1,263 / 1,119, 1,122
+// The line is on the safe side: cubes in flight break even near 1,400, synchronous ones near 2,000.
 bool few_models(const t3d_ctx* c, const t3d_render_desc* const* descs, uint32_t ndesc) {
   uint64_t pairs = 0;
   for (uint32_t j = 0; j < ndesc; j++) {
